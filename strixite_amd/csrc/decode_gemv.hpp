@@ -49,106 +49,16 @@ struct DecodeArgs {
     uint32_t q_bytes, s_bytes, x_bytes, y_bytes;
 };
 
-// A unit's per-lane load offsets and its output rows.
-struct DecUnit {
-    uint32_t qoff;           // code bytes of this lane's row (first tile) + its 16-byte lane group
-    uint32_t soff;           // scale bytes of the dword holding this lane's row's group 0 (element e rounded down)
-    uint32_t par;            // e & 1: the row's groups start in the dword's high half
-    int32_t tile, col0;      // tile index; first output column
-    bool nan;                // the tile's bucket is not an expert (invalid ids): NaN outputs
-};
-
-// RPU: weight rows a unit starts apart (its first row is RPU c + lane's row)
-template <int RPU>
-__device__ __forceinline__ DecUnit dec_unit(const DecodeArgs &a, int64_t u, int64_t units_per_tile, int64_t rec0,
-                                            bool valid) {
-    const int lane = threadIdx.x % kWave, g = lane / 16, j = lane % 16;
-    DecUnit d;
-    const int32_t t = valid ? (int32_t)(u / units_per_tile) : 0, c = valid ? (int32_t)(u % units_per_tile) : 0;
-    const int32_t bucket = __builtin_amdgcn_readfirstlane(a.ws[rec0 + route::kRec16 * t]);
-    d.nan = bucket < 0 || bucket >= a.E;
-    const uint32_t expert = d.nan ? 0u : (uint32_t)bucket;
-    d.tile = t;
-    d.col0 = RPU * c;
-    const uint32_t row = expert * (uint32_t)a.N + (uint32_t)(RPU * c) + (uint32_t)j;
-    const uint32_t e = row * (uint32_t)(a.K / 128);
-    d.par = e & 1u;
-    d.qoff = valid ? row * (uint32_t)(a.K / 2) + 16u * g : a.q_bytes;
-    d.soff = valid ? (e - d.par) * 2 : a.s_bytes;
-    return d;
-}
-
-// step s reads element e + s: dword (e + s) >> 1 = (e - par) / 2 + (s >> 1) + (par & s), the high half when e + s
-// is odd; the perm selector moves the wanted bf16 to the high half
-__device__ __forceinline__ uint32_t dec_sel(const DecUnit &d, int s) {
-    return (d.par ^ (uint32_t)(s & 1)) ? 0x03020C0Cu : 0x01000C0Cu;
-}
-
 template <int NT> struct DecRing {
     uint4 q[NT];
-    uint32_t s[NT], m[NT];
 };
-
-// Loads of K step s of unit d (NT tiles: the second tile_q / tile_s bytes on); an invalid unit loads past the end.
-template <int NT>
-__device__ __forceinline__ void dec_fetch(const __amdgpu_buffer_rsrc_t &rq, const __amdgpu_buffer_rsrc_t &rs,
-                                          const __amdgpu_buffer_rsrc_t &rm, const DecUnit &d, int s,
-                                          uint32_t tile_q, uint32_t tile_s, DecRing<NT> &r) {
-    const uint32_t so = d.soff + 4 * (d.par & (uint32_t)s), sd = (uint32_t)(s >> 1) * 4;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        r.q[t] = bld16(rq, d.qoff, (uint32_t)s * 64 + t * tile_q);
-        r.s[t] = bld4(rs, so, sd + t * tile_s);
-        r.m[t] = bld4(rm, so, sd + t * tile_s);
-    }
-}
 
 // Code loads only (the scales come from elsewhere): K step s of the row at qoff (NT tiles, tile_q bytes apart)
 template <int NT>
-__device__ __forceinline__ void dec_fetch(const __amdgpu_buffer_rsrc_t &rq, const __amdgpu_buffer_rsrc_t &,
-                                          const __amdgpu_buffer_rsrc_t &, uint32_t qoff, int s, uint32_t tile_q,
+__device__ __forceinline__ void dec_fetch(const __amdgpu_buffer_rsrc_t &rq, uint32_t qoff, int s, uint32_t tile_q,
                                           DecRing<NT> &r) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) r.q[t] = bld16(rq, qoff, (uint32_t)s * 64 + t * tile_q);
-}
-
-// One K step with the scale and min given: acc[t] += s * D + (m - 128 s) * xs
-template <int NT>
-__device__ __forceinline__ void dec_step_f(const DecRing<NT> &r, const Frag (&af)[4], const float (&xs)[4],
-                                           const float (&sc)[NT], const float (&mn)[NT], float4v (&acc)[NT]) {
-    float4v dd[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) dd[t] = float4v{0, 0, 0, 0};
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) dd[t] = mfma_bf16(af[u], b_frag<4>(r.q[t], u), dd[t]);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const float m = fmaf(-128.0f, sc[t], mn[t]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(sc[t], dd[t][i], fmaf(m, xs[i], acc[t][i]));
-    }
-}
-
-// One K step: acc[t] += s * D + (m - 128 s) * xs, D = the step's four MFMAs over the fragments af
-template <int NT>
-__device__ __forceinline__ void dec_step(const DecRing<NT> &r, const Frag (&af)[4], const float (&xs)[4],
-                                         uint32_t sel, float4v (&acc)[NT]) {
-    float4v dd[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) dd[t] = float4v{0, 0, 0, 0};
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) dd[t] = mfma_bf16(af[u], b_frag<4>(r.q[t], u), dd[t]);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const float sc = __uint_as_float(__builtin_amdgcn_perm(0u, r.s[t], sel));
-        const float mn = fmaf(-128.0f, sc, __uint_as_float(__builtin_amdgcn_perm(0u, r.m[t], sel)));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(sc, dd[t][i], fmaf(mn, xs[i], acc[t][i]));
-    }
 }
 
 // The wave's unit range [u0, u1) of nu units over nw waves dealt as the header describes; false: this wave is idle.
@@ -294,7 +204,7 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
         advance();
         sreg[r] = scale_load(ud[r]);
 #pragma unroll
-        for (int t = 0; t < SPW; ++t) dec_fetch<NT>(rq, rs, rm, ud[r].qoff, sb + t, tile_q, ring[r * SPW + t]);
+        for (int t = 0; t < SPW; ++t) dec_fetch<NT>(rq, ud[r].qoff, sb + t, tile_q, ring[r * SPW + t]);
     }
     for (int64_t t = tid; t < n_tiles; t += WAVES * kWave) tb[t] = a.ws[rec0 + route::kRec16 * t];
     scale_store(sreg[0], 0);
@@ -350,7 +260,7 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
 #pragma unroll
                     for (int i = 0; i < 4; ++i) acc[tt][i] = fmaf(sv, dd[tt][i], acc[tt][i]);
                 }
-                dec_fetch<NT>(rq, rs, rm, nu.qoff, sb + t, tile_q, ring[r * SPW + t]);
+                dec_fetch<NT>(rq, nu.qoff, sb + t, tile_q, ring[r * SPW + t]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             // the K parts meet: wave w's partials to red[par][w]; the next unit's scales to its buffer; then wave w
@@ -627,110 +537,35 @@ __global__ void __launch_bounds__((W + 1) * kWave) decode_gate_up_lds_kernel(Dec
     wait_vmcnt<0>();  // no load still landing in LDS when the wave ends
 }
 
-// ---- down -------------------------------------------------------------------------------------------------------------
-// A unit: 32 rows (two 16-row tiles) of one expert over K = 512 (four steps). A operand: the tile's h rows (lane (g, i):
-// slot i's 8 values at k = 128 step + 32 g + 8 u), reloaded when the unit's tile changes; their per-group sums come from
-// one more MFMA against an all-ones B. Output: FP32 partials by slot.
-constexpr int kDecDownSteps = 4;
-template <int SH>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-    decode_down_kernel(DecodeArgs a, SharedJob sh) {
-    constexpr int NT = 2, KS = kDecDownSteps, D = KS;  // the ring: one unit ahead
-    int bid = (int)blockIdx.x, nblk = (int)gridDim.x;
-    if constexpr (SH == 2) {
-        if (bid < sh.blocks) {  // the shared expert's down, split-K parts
-            const int64_t w = (int64_t)bid * (blockDim.x / kWave) + threadIdx.x / kWave;
-            if (w < sh.units) dense_part_unit<8>(sh.a, sh.spp, sh.parts, sh.pout, w);
-            return;
-        }
-        bid -= sh.blocks, nblk -= sh.blocks;
-    }
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int g = lane / 16, j = lane % 16;
-    const int64_t n_tiles = a.ws[0] < a.tiles_bound ? a.ws[0] : a.tiles_bound;
-    const int64_t upt = a.N / 32;
-    int64_t u0, u1;
-    if (!dec_range(n_tiles * upt, (int64_t)wave * nblk + bid, (int64_t)nblk * kWaves, u0, u1)) return;
-    const __amdgpu_buffer_rsrc_t rq = rsrc(a.q, a.q_bytes), rs = rsrc(a.scale, a.s_bytes),
-                                 rm = rsrc(a.minv, a.s_bytes), rx = rsrc(a.x, a.x_bytes), ry = rsrc(a.y, a.y_bytes);
-    const uint32_t tile_q = 16u * (uint32_t)(a.K / 2), tile_s = 16u * (uint32_t)(a.K / 128) * 2;  // +16 rows
-    const int64_t rec0 = route::t16_rec_at(a.S, a.E);
-    const Frag ones{{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}};
-
-    DecUnit cur = dec_unit<32>(a, u0, upt, rec0, true);
-    DecUnit nxt = dec_unit<32>(a, u0 + 1, upt, rec0, u0 + 1 < u1);
-    DecRing<NT> ring[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) dec_fetch<NT>(rq, rs, rm, cur, k, tile_q, tile_s, ring[k]);
-    // segments of units on one tile: the tile's h rows (and their per-group sums) are loaded at a segment's start
-    for (int64_t u = u0; u < u1;) {
-        const int32_t slot_l = a.ws[rec0 + route::kRec16 * cur.tile + 4 + j];  // a slot past the tile's rows: -1
-        const uint32_t xo = slot_l >= 0 ? ((uint32_t)slot_l * (uint32_t)a.K + 32u * g) * 2 : a.x_bytes;
-        Frag hf[KS][4];
-        float hs[KS][4];  // per-group sums of the tile rows this lane's outputs belong to
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint4 t = bld16(rx, xo, (uint32_t)(s * dec::kSpan + 8 * v) * 2);
-                hf[s][v] = Frag{{t.x, t.y, t.z, t.w}};
-            }
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            float4v d = {0, 0, 0, 0};
-#pragma unroll
-            for (int v = 0; v < 4; ++v) d = mfma_bf16(hf[s][v], ones, d);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) hs[s][i] = d[i];
-        }
-        const int64_t seg_end = std::min<int64_t>(u1, (int64_t)(cur.tile + 1) * upt);
-        for (; u < seg_end; ++u) {
-            float4v acc[NT] = {float4v{0, 0, 0, 0}, float4v{0, 0, 0, 0}};
-#pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                dec_step<NT>(ring[s], hf[s], hs[s], dec_sel(cur, s), acc);
-                dec_fetch<NT>(rq, rs, rm, nxt, s, tile_q, tile_s, ring[s]);  // step s of the next unit
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // partial[slot][col]: tile row 4 g + i is slot lane (4 g + i)'s record entry
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int32_t sl = __shfl(slot_l, 4 * g + i, kWave);
-                if (sl >= 0)
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        __builtin_amdgcn_raw_buffer_store_b32(
-                            __float_as_uint(cur.nan ? qnan() : acc[t][i]), ry,
-                            ((uint32_t)sl * (uint32_t)a.N + cur.col0 + 16 * t + j) * 4, 0, 0);
-            }
-            cur = nxt;
-            nxt = dec_unit<32>(a, u + 2, upt, rec0, u + 2 < u1);
-        }
-    }
-}
-
 // ---- down through per-wave LDS rings ---------------------------------------------------------------------------------
-// K = 512 (Q4 g128: 256 bytes a row, four groups). A unit is 16 consecutive weight rows of one expert (4 KB,
+// K = 128 KS (Q4 g128: 64 KS bytes a row, KS groups). A unit is 16 consecutive weight rows of one expert (KS KB,
 // contiguous) against one 16-slot tile; the tile's h rows are the MFMA's A operand for all of its units, held in
 // registers. Waves are dealt to tiles, not to a flat unit range: every tile gets floor or ceil(waves / tiles) waves,
 // each a contiguous range of the tile's N / 16 row blocks, so a wave loads its tile's h rows once, before its loop,
-// and streams one contiguous region of the expert's rows. A unit's codes reach LDS by four direct loads of 4 rows x
-// 256 bytes (1 KB contiguous each), with its rows' scale and min dwords, into the wave's own ring of kDnStages
-// positions; no barrier, no K split. The FP32 partials are stored as each unit ends: the waits count loads only (a
+// and streams one contiguous region of the expert's rows. A unit's codes reach LDS by KS direct loads of 1 KB
+// (contiguous), with its rows' scale and min dwords, into the wave's own ring of kDnStages positions; no barrier, no K split. The FP32 partials are stored as each unit ends: the waits count loads only (a
 // store may complete before older loads, so counting it could release a wait early; not counting it only makes a wait
 // stricter).
-// LDS layout of a position (uint4): codes [4 loads][lane], lane l holding row 4 load + l / 16's 16-byte chunk
-// (l % 16) ^ row at position l % 16 (the MFMA-layout reads of one chunk of the 16 rows hit 16 bank groups); then
-// 32 dwords of scales (row r: dword 2 r + group / 2) and 32 of mins.
+// LDS layout of a position (uint4): the rows' 4 KS 16-byte chunks in row order, chunk c of row r at place c ^ swz(r) of
+// its row; then 8 KS dwords of scales (row r's group s: bf16 KS r + s) and as many of mins. swz spreads the 16 rows'
+// reads of one chunk over the 64 LDS banks: rows 16 KS dwords apart share their banks every 4 (KS odd), 8 (KS = 2 mod
+// 4) or 16 / 16 (KS = 4) rows apart, and the aliasing rows take different places of a 4-, 8- or 16-chunk block.
 namespace gdn {
-constexpr int kDnStages = 3, kDnWaves = 4;  // per-wave ring; waves a block (three blocks a CU)
-constexpr int kPosU4 = 4 * kWave + 16;      // codes + 64 dwords of scales and mins
+constexpr int kDnStages = 3;                                    // per-wave ring
+template <int KS> constexpr int pos_u4() { return 4 * KS * 17; }  // codes + 16 KS dwords of scales and mins
+// waves a block: 4 (three blocks, 12 waves a CU) at KS = 4; 2 (five blocks, 10 waves) at KS = 5, whose positions are
+// 5,440 bytes (4 waves a block would leave room for two blocks, 8 waves)
+template <int KS> constexpr int waves() { return KS <= 4 ? 4 : 2; }
+template <int KS> constexpr int blocks_per_cu() { return 163840 / (waves<KS>() * kDnStages * pos_u4<KS>() * 16); }
+template <int KS> __device__ __forceinline__ int swz(int r) {
+    return KS % 2 ? (r >> 2) & 3 : KS % 4 ? (r >> 1) & 7 : r;
+}
 }  // namespace gdn
 
-template <int SH, int WB = gdn::kDnWaves, int NS = gdn::kDnStages>
+template <int SH, int KS, int WB = gdn::waves<KS>(), int NS = gdn::kDnStages>
 __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs a, SharedJob sh) {
     static_assert(NS >= 3 && NS <= 8, "ring positions: separate LDS arrays, at most 8");
-    constexpr int KS = kDecDownSteps;  // KS: groups a row (K = 512)
+    static_assert(KS >= 2 && KS <= 8, "K = 128 KS");
     int bid = (int)blockIdx.x, nblk = (int)gridDim.x;
     if constexpr (SH == 2) {
         if (bid < sh.blocks) {  // the shared expert's down, split-K parts
@@ -741,7 +576,7 @@ __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs 
         bid -= sh.blocks, nblk -= sh.blocks;
     }
     // one array a ring position (the compiler tracks the direct-to-LDS loads' aliasing per array); unused ones 1 x 1
-    constexpr int P = gdn::kPosU4;
+    constexpr int P = gdn::pos_u4<KS>();
     __shared__ __attribute__((aligned(16))) uint4 rp0[WB][P], rp1[WB][P], rp2[WB][P], rp3[NS > 3 ? WB : 1][NS > 3 ? P : 1],
         rp4[NS > 4 ? WB : 1][NS > 4 ? P : 1], rp5[NS > 5 ? WB : 1][NS > 5 ? P : 1], rp6[NS > 6 ? WB : 1][NS > 6 ? P : 1],
         rp7[NS > 7 ? WB : 1][NS > 7 ? P : 1];
@@ -788,30 +623,30 @@ __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs 
 #pragma unroll
             for (int v = 0; v < 4; ++v) hr[s][v] = bld16(rx, xo, (uint32_t)(s * dec::kSpan + 8 * v) * 2);
     }
-    // this lane's code load pieces: load i covers rows 4 i .. 4 i + 3: lane l row 4 i + l / 16, chunk (l % 16) ^ row
-    uint32_t loff[4];
+    // this lane's code load pieces: load i fills places 64 i .. 64 i + 63 of the unit (place p of row rr: chunk p ^ swz)
+    uint32_t loff[KS];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int rr = 4 * i + lane / 16;
-        loff[i] = (uint32_t)rr * 256u + (uint32_t)(((lane % 16) ^ rr) * 16);
+    for (int i = 0; i < KS; ++i) {
+        const int p = i * kWave + lane, rr = p / (4 * KS);
+        loff[i] = (uint32_t)rr * (64u * KS) + (uint32_t)(((p % (4 * KS)) ^ gdn::swz<KS>(rr)) * 16);
     }
     const uint32_t row_e = expert * (uint32_t)a.N;  // the expert's first row
-    // unit q (row block r + q k) into position P: four code loads and (lanes 0..31) the 16 rows' scale and min dwords;
-    // past the expert's rows:
-    // offsets past the ends
+    // unit q (row block r + q k) into position P: KS code loads and (lanes below 8 KS) the 16 rows' scale and min
+    // dwords; past the expert's rows: offsets past the ends
     auto issue = [&](int32_t q, auto P) __attribute__((always_inline)) {
         uint4 *R = ring(P);
         const int32_t rb = r + q * k;
         const bool valid = rb < rbs;
         const uint32_t row0 = row_e + 16u * (uint32_t)rb;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) lds_load16_nt(rq, R + i * kWave, valid ? row0 * 256u + loff[i] : a.q_bytes, 0);
-        if (lane < 32) {  // dword l of the rows' scales (16 rows x 4 bf16 = 32 dwords), then of the mins
+        for (int i = 0; i < KS; ++i)
+            lds_load16_nt(rq, R + i * kWave, valid ? row0 * (64u * KS) + loff[i] : a.q_bytes, 0);
+        if (lane < 8 * KS) {  // dword l of the rows' scales (16 rows x KS bf16), then of the mins
             const uint32_t so = valid ? row0 * (uint32_t)(KS * 2) + 4u * (uint32_t)lane : a.s_bytes;
-            uint32_t *dst = reinterpret_cast<uint32_t *>(R + 4 * kWave);
+            uint32_t *dst = reinterpret_cast<uint32_t *>(R + KS * kWave);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 4, so, 0, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, (__attribute__((address_space(3))) void *)(dst + 32), 4, so, 0,
-                                                     0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, (__attribute__((address_space(3))) void *)(dst + 8 * KS), 4, so,
+                                                     0, 0, 0);
         }
     };
     const int32_t nq_pad = (nq + NS - 1) / NS * NS;
@@ -842,20 +677,23 @@ __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs 
     }
     auto step = [&](int32_t q, auto P) __attribute__((always_inline)) {
         constexpr int p = decltype(P)::value;
-        wait_vmcnt<6 * (NS - 2)>();  // loads issued after unit q's: units q + 1 .. q + NS - 2, six each
+        wait_vmcnt<(KS + 2) * (NS - 2)>();  // loads issued after unit q's: units q + 1 .. q + NS - 2, KS + 2 each
         __builtin_amdgcn_sched_barrier(0);
         issue(q + NS - 1, std::integral_constant<int, (p + NS - 1) % NS>{});
         const uint4 *R = ring(P);
-        const uint32_t *scl = reinterpret_cast<const uint32_t *>(R + 4 * kWave);
+        const uint32_t *scl = reinterpret_cast<const uint32_t *>(R + KS * kWave);
         float4v acc = {0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const int c = 4 * s + g;  // lane group g's 16-byte chunk of group s
             // a native vector load (a uint4 struct copy would become a memcpy that loses the LDS alias scopes)
-            const u32x4v v = *reinterpret_cast<const u32x4v *>(R + (j / 4) * kWave + 16 * (j % 4) + (c ^ j));
-            const uint32_t sw = scl[2 * j + s / 2], mw = scl[32 + 2 * j + s / 2];
-            const float sc = __uint_as_float(s % 2 == 0 ? sw << 16 : sw & 0xFFFF0000u);
-            const float mn = fmaf(-128.0f, sc, __uint_as_float(s % 2 == 0 ? mw << 16 : mw & 0xFFFF0000u));
+            const u32x4v v = *reinterpret_cast<const u32x4v *>(R + 4 * KS * j + (c ^ gdn::swz<KS>(j)));
+            // bf16 e of the rows' scales and mins (KS even: its half of the dword is the group's parity)
+            const int e = KS * j + s;
+            const bool odd = KS % 2 ? e & 1 : s & 1;
+            const uint32_t sw = scl[e / 2], mw = scl[8 * KS + e / 2];
+            const float sc = __uint_as_float(odd ? sw & 0xFFFF0000u : sw << 16);
+            const float mn = fmaf(-128.0f, sc, __uint_as_float(odd ? mw & 0xFFFF0000u : mw << 16));
             float4v d = {0, 0, 0, 0};
             const uint32_t qw[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -881,14 +719,30 @@ __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs 
 constexpr int kDecGuWaves = 8, kDecGuAhead = 2;  // waves a block; units of loads in flight ahead of the math
 constexpr int kDecMaxTiles = 1024;               // M <= 16 tokens x A <= 64 slots
 
-// Q4 g128 experts, at most 16 tokens; gate_up: K = 128 * kDecGuWaves * SPW, SPW in 2..4; down: K = 512
+inline bool gate_up_lds_fits(const GemmArgs &ga);
+// the LDS-ring down kernel's shapes: Q4 g128, K = 512 or 640 (the benchmark's and the served model's I); it deals its
+// waves to tiles, so every tile needs a wave. Measured on MI355X at H 2560, I 640, 513 experts, 11 slots a token, against
+// the register-fed stream kernels (this and the gate_up at W = 10 together): a layer of 11 tokens 116 -> 86 us, of 1
+// token 40.0 -> 33.5, of 333 tokens 526 -> 366
+inline bool down_lds_fits(const GemmArgs &ga) {
+    const int64_t tiles = std::min(ga.S, ga.S / 16 + ga.E + 2);
+    auto waves = [](auto ks) { return gdn::blocks_per_cu<decltype(ks)::value>() * gdn::waves<decltype(ks)::value>(); };
+    if (ga.G != dec::kSpan || ga.N % 16 != 0) return false;
+    if (ga.K == 4 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 4>{}) * device_cus();
+    if (ga.K == 5 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 5>{}) * device_cus();
+    return false;
+}
+
+// Q4 g128 experts, at most 16 tokens; gate_up: the LDS-ring kernel's shapes or K = 128 * kDecGuWaves * SPW, SPW in 2..4;
+// down: the LDS-ring kernel's shapes
 inline bool decode_fits(const GemmArgs &ga, int64_t M, bool swiglu) {
     if (ga.G != dec::kSpan || M > dec::kMaxTokens || ga.K % dec::kSpan != 0 || ga.S > kDecMaxTiles) return false;
     if (swiglu) {
         const int64_t steps = ga.K / dec::kSpan;
-        return steps % kDecGuWaves == 0 && steps / kDecGuWaves >= 2 && steps / kDecGuWaves <= 4 && (ga.N / 2) % 16 == 0;
+        return gate_up_lds_fits(ga) ||
+               (steps % kDecGuWaves == 0 && steps / kDecGuWaves >= 2 && steps / kDecGuWaves <= 4 && (ga.N / 2) % 16 == 0);
     }
-    return ga.K == dec::kSpan * kDecDownSteps && ga.N % 32 == 0;
+    return down_lds_fits(ga);
 }
 
 inline DecodeArgs decode_args(const GemmArgs &ga, int64_t M, bool swiglu) {
@@ -916,12 +770,12 @@ void launch_decode_gate_up_lds(const DecodeArgs &d, SharedJob s, hipStream_t str
     else decode_gate_up_lds_kernel<W, 0><<<blocks, (W + 1) * kWave, 0, stream>>>(d, s);
 }
 
-// the LDS-ring gate_up's shapes: K = 256 W (W 8 or 12), Q4 g128; a block's unit range (at most ceil(units / CUs)
+// the LDS-ring gate_up's shapes: K = 256 W (W 8, 10 or 12: H 2048, 2560, 3072), Q4 g128; a block's unit range (at most ceil(units / CUs)
 // units) must touch at most kGuMaxBlockTiles tiles, and the tile count fit the block's table
 inline bool gate_up_lds_fits(const GemmArgs &ga) {
     const int64_t tiles_bound = std::min(ga.S, ga.S / 16 + ga.E + 2);
     const int64_t upt = ga.N / 32, most_units = (tiles_bound * upt + device_cus() - 1) / device_cus();
-    return ga.G == dec::kSpan && ga.K % 256 == 0 && (ga.K / 256 == 8 || ga.K / 256 == 12) && (ga.N / 2) % 16 == 0 &&
+    return ga.G == dec::kSpan && ga.K % 256 == 0 && (ga.K / 256 == 8 || ga.K / 256 == 10 || ga.K / 256 == 12) && (ga.N / 2) % 16 == 0 &&
            (most_units + upt - 1) / upt + 1 <= gul::kGuMaxBlockTiles && tiles_bound <= kDecMaxTilesL;
 }
 
@@ -934,6 +788,7 @@ inline void launch_gate_up_stream(const GemmArgs &ga, int64_t M, hipStream_t str
     const DecodeArgs d = decode_args(ga, M, true);
     switch (ga.K / 256) {
         case 8: return launch_decode_gate_up_lds<8>(d, SharedJob{}, stream, true);
+        case 10: return launch_decode_gate_up_lds<10>(d, SharedJob{}, stream, true);
         default: return launch_decode_gate_up_lds<12>(d, SharedJob{}, stream, true);
     }
 }
@@ -966,6 +821,7 @@ inline void launch_decode_gate_up(const GemmArgs &ga, int64_t M, const SharedJob
         t.units = sh ? s.units : 0;
         switch (ga.K / 256) {
             case 8: return launch_decode_gate_up_lds<8>(d, t, stream);
+            case 10: return launch_decode_gate_up_lds<10>(d, t, stream);
             case 12: return launch_decode_gate_up_lds<12>(d, t, stream);
             default: break;
         }
@@ -977,40 +833,27 @@ inline void launch_decode_gate_up(const GemmArgs &ga, int64_t M, const SharedJob
     }
 }
 
-// The LDS-ring down kernel at any token count (it reads h by slot and writes partials by slot; every tile needs one of
-// its waves): Q4 g128, K = 512
+// The LDS-ring down kernel at any token count (it reads h by slot and writes partials by slot)
 inline bool down_stream_fits(const GemmArgs &ga) {
-    constexpr int kDnBlocksPerCu = 163840 / (gdn::kDnWaves * gdn::kDnStages * gdn::kPosU4 * 16);
-    return ga.G == dec::kSpan && ga.K == dec::kSpan * kDecDownSteps && ga.N % 32 == 0 &&
-           std::min(ga.S, ga.S / 16 + ga.E + 2) <= (int64_t)kDnBlocksPerCu * device_cus() * gdn::kDnWaves &&
-           ga.S * ga.K * 2 < (1ll << 31) && ga.S * ga.N * 4 < (1ll << 31) && ga.N * ga.E * ga.K / 2 < (1ll << 31) &&
-           ga.N * ga.E * (ga.K / ga.G) * 2 < (1ll << 31);
+    return down_lds_fits(ga) && ga.S * ga.K * 2 < (1ll << 31) && ga.S * ga.N * 4 < (1ll << 31) &&
+           ga.N * ga.E * ga.K / 2 < (1ll << 31) && ga.N * ga.E * (ga.K / ga.G) * 2 < (1ll << 31);
 }
 
 // down into FP32 partials; sh (optional): the shared expert's down parts riding along in leading blocks
 inline void launch_decode_down(const GemmArgs &ga, int64_t M, const SharedJob *sh, hipStream_t stream) {
     const DecodeArgs d = decode_args(ga, M, false);
-    const SharedJob s = sh ? *sh : SharedJob{};
-    const int blocks = 2 * device_cus() + s.blocks;  // two waves a SIMD
-    // the LDS-ring kernel deals its waves to tiles: every tile needs a wave
-    constexpr int kDnBlocksPerCu = 163840 / (gdn::kDnWaves * gdn::kDnStages * gdn::kPosU4 * 16);
-    if (ga.K == dec::kSpan * kDecDownSteps && ga.N % 16 == 0 &&
-        d.tiles_bound <= (int64_t)kDnBlocksPerCu * device_cus() * gdn::kDnWaves) {
-        // 4 waves x 3 ring positions a block, three blocks a CU (12 waves): measured on MI355X at 16 tokens, H 3072,
-        // I 512, 512 experts top-10 (layer us): 4 x 4 two blocks 104.2, 4 x 3 102.7, 3 x 4 104.1, 3 x 6 109.9,
-        // 2 x 8 109.3, 1 x 8 110.4 - more waves beat more units in flight (the LDS reads and the dequantisation
-        // of a unit are hidden by other waves, not by a wave's own ring)
-        auto go = [&](auto wbc, auto nsc) {
-            constexpr int WB = decltype(wbc)::value, NS = decltype(nsc)::value;
-            constexpr int lds = WB * NS * gdn::kPosU4 * 16;
-            const int bpc = 163840 / lds;  // blocks a CU by LDS
-            const int nb = bpc * device_cus() + s.blocks;
-            if (sh) decode_down_lds_kernel<2, WB, NS><<<(unsigned)nb, WB * kWave, 0, stream>>>(d, s);
-            else decode_down_lds_kernel<0, WB, NS><<<(unsigned)nb, WB * kWave, 0, stream>>>(d, s);
-        };
-        go(std::integral_constant<int, gdn::kDnWaves>{}, std::integral_constant<int, gdn::kDnStages>{});
-        return;
-    }
-    if (sh) decode_down_kernel<2><<<(unsigned)blocks, kThreads, 0, stream>>>(d, s);
-    else decode_down_kernel<0><<<(unsigned)blocks, kThreads, 0, stream>>>(d, s);
+    SharedJob s = sh ? *sh : SharedJob{};
+    // 4 waves x 3 ring positions a block, three blocks a CU (12 waves): measured on MI355X at 16 tokens, H 3072,
+    // I 512, 512 experts top-10 (layer us): 4 x 4 two blocks 104.2, 4 x 3 102.7, 3 x 4 104.1, 3 x 6 109.9,
+    // 2 x 8 109.3, 1 x 8 110.4 - more waves beat more units in flight (the LDS reads and the dequantisation
+    // of a unit are hidden by other waves, not by a wave's own ring)
+    auto go = [&](auto ksc) {
+        constexpr int KS = decltype(ksc)::value, WB = gdn::waves<KS>();
+        s.blocks = sh ? (int)((s.units + WB - 1) / WB) : 0;
+        const unsigned nb = (unsigned)(gdn::blocks_per_cu<KS>() * device_cus() + s.blocks);
+        if (sh) decode_down_lds_kernel<2, KS><<<nb, WB * kWave, 0, stream>>>(d, s);
+        else decode_down_lds_kernel<0, KS><<<nb, WB * kWave, 0, stream>>>(d, s);
+    };
+    if (ga.K == 4 * dec::kSpan) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 5>{});
 }
