@@ -1,0 +1,450 @@
+// Exact-weight projections on 16-row tiles: y = x . dequant(W)^T with x in FP32 or BF16 and W in Q4, Q5 or Q8, FP32
+// accumulation (strixite kernels/linear_q4.hpp:23-58, moe_grouped.hpp:3-16, :93-104, linear_q8.hpp:13-14). It serves the
+// FP32 activation mode and the Q5 experts everywhere, and the dense BF16 projections at small batches.
+//
+// A tile is the 16 A rows of v_mfma_f32_16x16x32_bf16 against RT tiles of 16 weight rows, the B columns. BF16: a row each
+// of 16 slots of one expert (or tokens). FP32: x = hi + mid + lo, the top 16 bits of x, of the rest and of the rest of
+// that (24 significant bits, exact), and the pieces of one row are three A rows, so a tile holds five rows and the
+// matrix cores do one product where three passes over the weights' fragments would (at decode sizes a bucket rarely has
+// more than five slots; 40 tokens: 276 experts, 1.4 slots each); an output is the sum of its three rows. A non-finite x
+// makes its row NaN.
+// Weights enter as integer codes exact in bf16 (Q4: 16 + n, Q5: 32 + n, Q8: c - 128) and each quantization group's
+// product D is rescaled on the FP32 accumulator: w . x = s D' + m' sum(x), with D' and m' for the codes about the middle
+// of their range (D' = D - EXTRA sum(x), m' = m + MID s), where neither term is larger than the result. sum(x) comes
+// from one more MFMA, against ones.
+//
+// What bounds it: grouped, the weight stream beside ~80 vector instructions a wave per 32 k x 64 weight rows (the split
+// and the codes' conversion); dense, latency, so K is split over the block's waves (8 from 32 steps, 4 from 8) and their
+// parts meet in LDS in wave order. The split depends on K and the format only, so a per-slot call gives the grouped
+// call's bits.
+// Measured on MI355X: 40 tokens, H 3072, I 512, 512 experts top-10, Q4 g128, FP32 activations, one wave an output element
+// before: gate_up 651 -> 179 us, down 897 -> 91 us (with the pieces as three MFMAs on one A tile: 201, 123; two weight tiles a
+// wave instead of four: 222, 117).
+#include "common.hpp"
+#include "exact_tile.hpp"
+#include "route_small.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace strix::kernels::xt {
+namespace {
+
+using namespace strix::dev;
+constexpr int kWave = 64;
+constexpr int kMaxWaves = 8;  // waves a block
+
+// A K step covers SP codes of a row (one quantization group at most): 4 lane groups x CPL codes
+template <int FMT, int SP> struct Fmt {
+    static constexpr int W = FMT == 8 ? 8 : 4;       // bits a code in the first plane
+    static constexpr int CPL = SP / 4, LB = CPL * W / 8, NT = CPL / 8;
+    // a code enters as EXTRA + (n - MID), MID the middle of its range
+    static constexpr float MID = FMT == 4 ? 8.f : FMT == 5 ? 16.f : 128.f, EXTRA = FMT == 4 ? 24.f : FMT == 5 ? 48.f : 0.f;
+    static_assert(LB == 16 || LB == 8 || LB == 4, "bytes a lane loads a step");
+};
+
+struct Codes {
+    uint32_t w[4], hi;
+};
+
+// row: byte offset of the lane's row from the tile's first (a uniform buffer resource: no 64-bit lane addresses)
+template <int FMT, int SP>
+__device__ __forceinline__ void load_codes(__amdgpu_buffer_rsrc_t rq, uint32_t row, uint32_t K, uint32_t k, Codes &c) {
+    using F = Fmt<FMT, SP>;
+    const uint32_t p = row + k * F::W / 8;
+    if constexpr (F::LB == 16) {
+        typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+        const u32x4v u = __builtin_amdgcn_raw_buffer_load_b128(rq, p, 0, 0);
+        c.w[0] = u.x, c.w[1] = u.y, c.w[2] = u.z, c.w[3] = u.w;
+    } else if constexpr (F::LB == 8) {
+        typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+        const u32x2v u = __builtin_amdgcn_raw_buffer_load_b64(rq, p, 0, 0);
+        c.w[0] = u.x, c.w[1] = u.y;
+    } else {
+        c.w[0] = __builtin_amdgcn_raw_buffer_load_b32(rq, p, 0, 0);
+    }
+    if constexpr (FMT == 5) {  // bit 4 of the codes: code k at bit k % 8 of byte k / 8 of the row's second plane
+        const uint32_t h = row + K / 2 + k / 8;
+        if constexpr (F::CPL == 32) c.hi = __builtin_amdgcn_raw_buffer_load_b32(rq, h, 0, 0);
+        else if constexpr (F::CPL == 16) c.hi = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rq, h, 0, 0);
+        else c.hi = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rq, h, 0, 0);
+    }
+}
+
+// bits 0, 2, 4, 6 of e to bit 6 of the bytes 0 .. 3
+__device__ __forceinline__ uint32_t spread_bits(uint32_t e) {
+    e &= 0x55u;
+    return ((e << 6) | (e << 12) | (e << 18) | (e << 24)) & 0x40404040u;
+}
+
+// codes 8 u .. 8 u + 7 of the lane as bf16 (OFF + code) in the paired k order k0 k2 k4 k6 k1 k3 k5 k7
+template <int FMT> __device__ __forceinline__ Frag code_frag(const Codes &c, int u) {
+    if constexpr (FMT == 8) {
+        const uint32_t a = c.w[2 * u] ^ 0x80808080u, b = c.w[2 * u + 1] ^ 0x80808080u;  // c - 128, signed
+        auto sb = [](uint32_t w, int i) { return (float)(int8_t)(uint8_t)(w >> (8 * i)); };
+        return Frag{{hi16_pair(sb(a, 0), sb(a, 2)), hi16_pair(sb(b, 0), sb(b, 2)), hi16_pair(sb(a, 1), sb(a, 3)),
+                     hi16_pair(sb(b, 1), sb(b, 3))}};
+    } else {
+        const uint32_t w = c.w[u];
+        uint32_t t, v, top;
+        if constexpr (FMT == 4) {  // 0x4180 | n << 3 = 16 + n
+            t = ((w << 3) & 0x78787878u) | 0x80808080u, v = ((w >> 1) & 0x78787878u) | 0x80808080u, top = 0x41414141u;
+        } else {  // 0x4200 | n << 2 = 32 + n
+            const uint32_t h = c.hi >> (8 * u);
+            t = ((w << 2) & 0x3C3C3C3Cu) | spread_bits(h), v = ((w >> 2) & 0x3C3C3C3Cu) | spread_bits(h >> 1);
+            top = 0x42424242u;
+        }
+        return Frag{{__builtin_amdgcn_perm(top, t, 0x04010400u), __builtin_amdgcn_perm(top, t, 0x04030402u),
+                     __builtin_amdgcn_perm(top, v, 0x04010400u), __builtin_amdgcn_perm(top, v, 0x04030402u)}};
+    }
+}
+
+// Activation rows of the MFMA: BF16 rows are themselves (16 a tile). An FP32 row is three MFMA rows, one per bf16 piece,
+// so a tile holds five: MFMA row r is piece r / 5 of the tile's row r % 5 (row 15 unused), and an output is the sum of
+// its three rows'.
+template <typename TX> constexpr int tile_rows_of() { return std::is_same_v<TX, float> ? 5 : 16; }
+
+// 8 activations of MFMA row j as bf16 in the paired order
+template <typename TX> struct Act8;
+template <> struct Act8<float> {
+    float4 a, b;
+    __device__ __forceinline__ void load(const float *p) {
+        a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
+    }
+    // piece j / 5: the top 16 bits of x, of the rest, of the rest of that (exact: 24 significant bits)
+    __device__ __forceinline__ Frag frag(int j) const {
+        const uint32_t m1 = j >= 5 ? 0xFFFF0000u : 0u, m2 = j >= 10 ? 0xFFFF0000u : 0u;
+        float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] -= __uint_as_float(__float_as_uint(v[i]) & m1);
+            v[i] -= __uint_as_float(__float_as_uint(v[i]) & m2);
+        }
+        return Frag{{hi16_pair(v[0], v[2]), hi16_pair(v[4], v[6]), hi16_pair(v[1], v[3]), hi16_pair(v[5], v[7])}};
+    }
+};
+template <> struct Act8<uint16_t> {
+    uint4 a;
+    __device__ __forceinline__ void load(const uint16_t *p) { a = *reinterpret_cast<const uint4 *>(p); }
+    __device__ __forceinline__ Frag frag(int) const {
+        return Frag{{__builtin_amdgcn_perm(a.y, a.x, 0x05040100u), __builtin_amdgcn_perm(a.w, a.z, 0x05040100u),
+                     __builtin_amdgcn_perm(a.y, a.x, 0x07060302u), __builtin_amdgcn_perm(a.w, a.z, 0x07060302u)}};
+    }
+};
+
+// The RT weight tiles' rows: a uniform first row each, and the lane's row in it (clamped at the last one for SwiGLU's
+// ragged ends)
+template <int RT> struct Rows {
+    __amdgpu_buffer_rsrc_t q[RT], s[RT], m[RT];
+    uint32_t j[RT];
+};
+
+// columns c0 + 16 t of an expert: SwiGLU takes gate tiles 0 .. RT / 2 - 1 and the matching up tiles; a tile past the
+// columns reads the first one's rows (never stored)
+template <int FMT, bool SWI, int RT>
+__device__ __forceinline__ Rows<RT> tile_rows(const Args &a, int64_t expert, int64_t c0) {
+    const int j = threadIdx.x % 16;
+    const int64_t row_bytes = FMT == 8 ? a.K : FMT == 4 ? a.K / 2 : a.K / 2 + a.K / 8, groups = a.K / a.G;
+    Rows<RT> r;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        int64_t c = c0 + 16 * (SWI ? t % (RT / 2) : t);
+        if (c >= a.ncol) c = 0;
+        const int64_t last = a.ncol - 1 - c;
+        r.j[t] = j < last ? j : (uint32_t)last;
+        const int64_t row = expert * a.N + c + (SWI && t >= RT / 2 ? a.ncol : 0);
+        auto res = [](const void *p, int64_t bytes) {
+            return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+        };
+        const int64_t n = last < 15 ? last + 1 : 16;  // the tile's rows
+        r.q[t] = res(a.q + row * row_bytes, n * row_bytes);
+        r.s[t] = res(a.scale + row * groups, n * groups * 2);
+        r.m[t] = res(a.minv + row * groups, n * groups * 2);
+    }
+    return r;
+}
+
+// acc[t] = the tile's sums over K steps [s0, s1): lane (g, j) holds rows 4 g .. 4 g + 3 against weight row j of tile t.
+// xp: the activation row of MFMA row lane % 16 (any row for an unused one: rows do not mix, and nobody reads its sums).
+template <int FMT, int SP, typename TX, int RT>
+__device__ __forceinline__ void tile_dot(const Args &a, const Rows<RT> &rw, const TX *xp, int s0, int s1,
+                                         float4v (&acc)[RT]) {
+    using F = Fmt<FMT, SP>;
+    const int g = threadIdx.x % kWave / 16;
+    const uint32_t row_bytes = (uint32_t)(FMT == 8 ? a.K : FMT == 4 ? a.K / 2 : a.K / 2 + a.K / 8);
+    const uint32_t groups = (uint32_t)(a.K / a.G), G = (uint32_t)a.G;
+    struct Buf {
+        Codes c[RT];
+        uint16_t s[RT], m[RT];
+        Act8<TX> x[F::NT];
+    };
+    auto fetch = [&](int s, Buf &b) {
+        const uint32_t k = (uint32_t)s * SP + g * F::CPL, gi = (uint32_t)s * SP / G;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            load_codes<FMT, SP>(rw.q[t], rw.j[t] * row_bytes, (uint32_t)a.K, k, b.c[t]);
+            b.s[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.s[t], (rw.j[t] * groups + gi) * 2, 0, 0);
+            b.m[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.m[t], (rw.j[t] * groups + gi) * 2, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < F::NT; ++u) {
+            b.x[u].load(xp + k + 8 * u);
+        }
+    };
+    auto step = [&](Buf &b, int next) {
+        const Frag ones{{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}};
+        float4v d[RT], dx = {0, 0, 0, 0};  // dx: the activations' own sums
+#pragma unroll
+        for (int t = 0; t < RT; ++t) d[t] = float4v{0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < F::NT; ++u) {
+            const Frag xf = b.x[u].frag(threadIdx.x % 16);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) d[t] = mfma_bf16(xf, code_frag<FMT>(b.c[t], u), d[t]);
+            dx = mfma_bf16(xf, ones, dx);
+            __builtin_amdgcn_sched_barrier(0);  // a group of codes is decoded just before its MFMAs (registers)
+        }
+        float sc[RT], mp[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            sc[t] = bf16_to_f32(b.s[t]);
+            mp[t] = fmaf(F::MID, sc[t], bf16_to_f32(b.m[t]));
+        }
+        if (next < s1) fetch(next, b);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const float n = F::EXTRA != 0.f ? fmaf(-F::EXTRA, dx[i], d[t][i]) : d[t][i];
+                acc[t][i] = fmaf(sc[t], n, fmaf(mp[t], dx[i], acc[t][i]));
+            }
+    };
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t] = float4v{0, 0, 0, 0};
+    Buf b0, b1;
+    if (s0 < s1) fetch(s0, b0);
+    if (s0 + 1 < s1) fetch(s0 + 1, b1);
+    for (int s = s0; s < s1; s += 2) {
+        step(b0, s + 2);
+        if (s + 1 < s1) step(b1, s + 3);
+    }
+}
+
+__device__ __forceinline__ void store(const Args &a, bool f32, int64_t row, int64_t col, float v) {
+    if (f32) static_cast<float *>(a.y)[row * a.ldy + col] = v;
+    else static_cast<uint16_t *>(a.y)[row * a.ldy + col] = f32_to_bf16(v);
+}
+
+__device__ __forceinline__ void report(uint32_t *err, int32_t id, int64_t slot) {
+    if (atomicCAS(&err[0], 0u, 1u) == 0u) err[1] = (uint32_t)id, err[2] = (uint32_t)slot;
+}
+
+// MFMA row r's sum over the parts of ks waves (wave order), column j of tile t
+template <int RT>
+__device__ __forceinline__ float row_sum(const float4v (*red)[RT][kWave], int w0, int ks, int t, int r, int j) {
+    auto at = [&](int w) { return reinterpret_cast<const float *>(&red[w][t][r / 4 * 16 + j])[r % 4]; };
+    float v = at(w0);
+    for (int w = 1; w < ks; ++w) v += at(w0 + w);
+    return v;
+}
+// tile row r: the sum of its MFMA rows
+template <typename TX, int RT>
+__device__ __forceinline__ float tile_sum(const float4v (*red)[RT][kWave], int w0, int ks, int t, int r, int j) {
+    const float v = row_sum<RT>(red, w0, ks, t, r, j);
+    if constexpr (std::is_same_v<TX, float>)
+        return v + (row_sum<RT>(red, w0, ks, t, r + 5, j) + row_sum<RT>(red, w0, ks, t, r + 10, j));
+    return v;
+}
+
+// Block (tile, column block): ks waves split K (ks = 1: each of the block's waves takes a column block of its own). A
+// grouped tile record holds up to 16 slots: FP32 takes them five at a time (the weights again from L1 / L2).
+template <int FMT, int SP, bool SWI, typename TX, int RT>
+__global__ void __launch_bounds__(kMaxWaves *kWave)
+    exact_tile_kernel(Args a, int mode, bool y_f32, int tiles_bound, int cbs, int bpt, int ks) {
+    static_assert(!SWI || RT % 2 == 0, "SwiGLU: gate and up tiles");
+    constexpr int TC = SWI ? RT / 2 : RT, TR = tile_rows_of<TX>();  // column tiles; rows a tile
+    __shared__ float4v red[kMaxWaves][RT][kWave];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int g = lane / 16, j = lane % 16, nw = (int)(blockDim.x / kWave);
+    const int tile = (int)(blockIdx.x / (uint32_t)bpt), cb = (int)(blockIdx.x % (uint32_t)bpt) * (nw / ks) + (ks > 1 ? 0 : wave);
+    int64_t expert = 0;
+    int rows, rec = 0;  // the record's rows; lane j: its row j as an output row
+    bool nan = false;
+    if (mode == GROUPED) {
+        if (tile >= a.ws[0] || tile >= tiles_bound) return;  // whole block, before any barrier
+        const int32_t *p = a.ws + route::Layout{a.S, a.E, 0, 0, 0}.t16_rec() + route::kRec16 * (int64_t)tile;
+        const int32_t b = __builtin_amdgcn_readfirstlane(p[0]);
+        nan = b < 0 || b >= a.E;
+        expert = nan ? 0 : b;
+        rows = __builtin_amdgcn_readfirstlane(p[2]);
+        rec = p[4 + j];
+    } else if (mode == PERSLOT) {
+        const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[tile]);
+        nan = id < 0 || id >= a.E;
+        expert = nan ? 0 : id;
+        rows = 1, rec = tile;
+        if (nan && blockIdx.x % (uint32_t)bpt == 0 && threadIdx.x == 0) report(a.err, id, tile);
+    } else {
+        rows = (int)(a.S - (int64_t)tile * TR < TR ? a.S - (int64_t)tile * TR : TR);
+        rec = tile * TR + j;
+    }
+    const int64_t c0 = (int64_t)cb * 16 * TC;
+    if (cb >= cbs) return;  // ks = 1 only (its waves meet no barrier)
+    const int spans = (int)(a.K / SP), part = ks > 1 ? wave : 0;
+    const Rows<RT> rw = tile_rows<FMT, SWI, RT>(a, expert, c0);
+    for (int r0 = 0; r0 < rows; r0 += TR) {
+        const int n = rows - r0 < TR ? rows - r0 : TR;
+        const int xi = std::is_same_v<TX, float> ? (j < 15 ? j % 5 : 15) : j;  // the tile row of MFMA row j
+        const int my = __shfl(rec, r0 + (xi < n ? xi : 0), kWave);
+        const TX *xp = static_cast<const TX *>(a.x) + (int64_t)((uint32_t)my / (uint32_t)a.A) * a.K;
+        float4v acc[RT];
+        tile_dot<FMT, SP, TX, RT>(a, rw, xp, spans * part / ks, spans * (part + 1) / ks, acc);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) red[wave][t][lane] = acc[t];
+        if (ks > 1) __syncthreads();
+        else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        // ks > 1: wave t finishes column tile t; else each wave its own. Lane (g, j): rows g, g + 4, ... of column j
+        for (int r = 0; r < n; r += 4) {
+            const int row = __shfl(rec, r0 + (r + g < n ? r + g : 0), kWave);
+#pragma unroll
+            for (int t = 0; t < TC; ++t) {
+                const int64_t col = c0 + 16 * t + j;
+                if ((ks > 1 && t != wave) || r + g >= n || col >= a.ncol) continue;
+                const int w0 = ks > 1 ? 0 : wave;
+                float v = tile_sum<TX, RT>(red, w0, ks, t, r + g, j);
+                if constexpr (SWI) v = silu(v) * tile_sum<TX, RT>(red, w0, ks, RT / 2 + t, r + g, j);
+                store(a, y_f32, row, col, nan ? qnan() : v);
+            }
+        }
+        if (ks > 1 && r0 + TR < rows) __syncthreads();  // red is read before the next rows' parts
+    }
+}
+
+// Block (token, column block), the token's slots one after another as exact_tile_kernel's one-row tiles (MFMA rows 0, 5
+// and 10 of an FP32 slot, row 0 of a BF16 one), their dots summed with the coefficients.
+template <int FMT, int SP, typename TX, int RT>
+__global__ void __launch_bounds__(kMaxWaves *kWave)
+    exact_perslot_combine_kernel(Args a, const float *coef, bool y_f32, int cbs, int bpt, int ks) {
+    __shared__ float4v red[2][kMaxWaves][RT][kWave];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int g = lane / 16, j = lane % 16, nw = (int)(blockDim.x / kWave);
+    const int64_t m = blockIdx.x / (uint32_t)bpt;
+    const int cb = (int)(blockIdx.x % (uint32_t)bpt) * (nw / ks) + (ks > 1 ? 0 : wave);
+    const int64_t c0 = (int64_t)cb * 16 * RT;
+    if (cb >= cbs) return;  // ks = 1 only (its waves meet no barrier)
+    const int spans = (int)(a.K / SP), part = ks > 1 ? wave : 0;
+    float out[RT] = {};
+    bool bad = false;
+    for (int64_t s = 0; s < a.A; ++s) {
+        const int64_t slot = m * a.A + s;
+        const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[slot]);
+        const bool nan = id < 0 || id >= a.E;
+        if (nan && blockIdx.x % (uint32_t)bpt == 0 && threadIdx.x == 0) report(a.err, id, slot);
+        bad = bad || nan;
+        const float cf = coef[slot];
+        float4v acc[RT];
+        tile_dot<FMT, SP, TX, RT>(a, tile_rows<FMT, false, RT>(a, nan ? 0 : id, c0),
+                                  static_cast<const TX *>(a.x) + slot * a.K, spans * part / ks, spans * (part + 1) / ks, acc);
+        float4v(&rb)[kMaxWaves][RT][kWave] = red[s & 1];  // two buffers: one barrier a slot
+#pragma unroll
+        for (int t = 0; t < RT; ++t) rb[wave][t][lane] = acc[t];
+        if (ks > 1) __syncthreads();
+        else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) out[t] = fmaf(cf, tile_sum<TX, RT>(rb, ks > 1 ? 0 : wave, ks, t, 0, j), out[t]);
+    }
+    if (g != 0 || (ks > 1 && wave != 0)) return;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+        if (c0 + 16 * t + j < a.ncol) store(a, y_f32, m, c0 + 16 * t + j, bad ? qnan() : out[t]);
+}
+
+int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n = 256;
+        return n > 0 ? n : 256;
+    }();
+    return cus;
+}
+
+// waves that split K: by the K steps alone (the bits of a dot follow from it)
+int split_of(int64_t spans) { return spans >= 32 ? 8 : spans >= 8 ? 4 : 1; }
+
+// the K step of a format and group size: the 16-byte load's span unless the group is smaller
+template <typename F> void by_format(int fmt, int64_t G, F &&f) {
+    using std::integral_constant;
+    if (fmt == 4) {
+        if (G == 128) f(integral_constant<int, 4>{}, integral_constant<int, 128>{});
+        else if (G == 64) f(integral_constant<int, 4>{}, integral_constant<int, 64>{});
+        else f(integral_constant<int, 4>{}, integral_constant<int, 32>{});
+    } else if (fmt == 5) {
+        if (G == 128) f(integral_constant<int, 5>{}, integral_constant<int, 128>{});
+        else if (G == 64) f(integral_constant<int, 5>{}, integral_constant<int, 64>{});
+        else f(integral_constant<int, 5>{}, integral_constant<int, 32>{});
+    } else {
+        if (G >= 64) f(integral_constant<int, 8>{}, integral_constant<int, 64>{});
+        else f(integral_constant<int, 8>{}, integral_constant<int, 32>{});
+    }
+}
+
+}  // namespace
+
+void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &a, hipStream_t stream) {
+    const int64_t tr = x_act == Act::F32 ? tile_rows_of<float>() : tile_rows_of<uint16_t>();
+    const int64_t tiles = mode == GROUPED ? std::min(a.S, a.S / 16 + a.E + 2) : mode == DENSE ? (a.S + tr - 1) / tr : a.S;
+    by_format(fmt, a.G, [&](auto fc, auto sc) {
+        constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value;
+        const int ks = split_of(a.K / SP), nw = ks > 1 ? ks : 4;
+        auto go = [&](auto swc, auto tx, auto rtc) {
+            constexpr bool SWI = decltype(swc)::value;
+            constexpr int RT = decltype(rtc)::value, TC = SWI ? RT / 2 : RT;
+            const int64_t cbs = (a.ncol + 16 * TC - 1) / (16 * TC), bpt = ks > 1 ? cbs : (cbs + nw - 1) / nw;
+            STRIX_CHECK(tiles * bpt < (1ll << 31) && a.S < (1ll << 31), "exact projection: ", a.S, " x ", a.ncol,
+                        " outputs, too many");
+            exact_tile_kernel<FMT, SP, SWI, decltype(tx), RT>
+                <<<(unsigned)(tiles * bpt), nw * kWave, 0, stream>>>(a, (int)mode, y_act == Act::F32, (int)tiles, (int)cbs,
+                                                                     (int)bpt, ks);
+        };
+        auto by_rt = [&](auto swc, auto tx) {
+            // four weight tiles a wave share the activations' pieces; two where four would leave most CUs without a block
+            const int64_t tc4 = decltype(swc)::value ? 2 : 4;
+            if (tiles * ((a.ncol + 16 * tc4 - 1) / (16 * tc4)) / (ks > 1 ? 1 : 4) < 2 * device_cus())
+                go(swc, tx, std::integral_constant<int, 2>{});
+            else go(swc, tx, std::integral_constant<int, 4>{});
+        };
+        auto by_x = [&](auto swc) {
+            if (x_act == Act::F32) by_rt(swc, float{});
+            else by_rt(swc, uint16_t{});
+        };
+        if (swiglu) by_x(std::true_type{});
+        else by_x(std::false_type{});
+    });
+}
+
+void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStream_t stream) {
+    by_format(fmt, a.G, [&](auto fc, auto sc) {
+        constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value, RT = 2;
+        const int ks = split_of(a.K / SP), nw = ks > 1 ? ks : 4;
+        const int64_t cbs = (a.ncol + 16 * RT - 1) / (16 * RT), bpt = ks > 1 ? cbs : (cbs + nw - 1) / nw;
+        STRIX_CHECK(a.S * bpt < (1ll << 31), "exact per-slot combine: ", a.S, " x ", a.ncol, " outputs, too many");
+        const unsigned blocks = (unsigned)(a.S * bpt);
+        if (act == Act::F32)
+            exact_perslot_combine_kernel<FMT, SP, float, RT>
+                <<<blocks, nw * kWave, 0, stream>>>(a, coef, true, (int)cbs, (int)bpt, ks);
+        else
+            exact_perslot_combine_kernel<FMT, SP, uint16_t, RT>
+                <<<blocks, nw * kWave, 0, stream>>>(a, coef, false, (int)cbs, (int)bpt, ks);
+    });
+}
+
+}  // namespace strix::kernels::xt

@@ -13,6 +13,7 @@
 // A span (Q4: 128 codes, Q8: 64) never crosses a group: Q4 needs G = 128, Q8 G = 64 or 128 (the reference's
 // served layout: q4g128, q8g64).
 #include "common.hpp"
+#include "exact_tile.hpp"
 #include "route_small.hpp"
 #include "router_small.hpp"
 
@@ -1049,6 +1050,27 @@ __global__ void __launch_bounds__(kThreads) add_bias_kernel(float *logits, int64
     }
 }
 
+// y[m, n] = sum_a coef[m, a] partial[m A + a, n] in slot order (fmaf), FP32; an invalid id of the token: NaN
+__global__ void __launch_bounds__(kThreads) f32_combine_kernel(const float *partial, const int32_t *ids, const float *coef,
+                                                               int64_t M, int64_t A, int64_t E, int64_t N, float *y) {
+    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i >= M * N) return;
+    const int64_t m = i / N, n = i % N;
+    float acc = 0.f;
+    bool bad = false;
+    for (int64_t s = 0; s < A; ++s) {
+        const int32_t id = ids[m * A + s];
+        bad = bad || id < 0 || id >= E;
+        acc = fmaf(coef[m * A + s], partial[(m * A + s) * N + n], acc);
+    }
+    y[i] = bad ? qnan() : acc;
+}
+void f32_combine(const float *partial, const int32_t *ids, const float *coef, int64_t M, int64_t A, int64_t E, int64_t N,
+                 float *y, hipStream_t stream) {
+    const unsigned blocks = (unsigned)((M * N + kThreads - 1) / kThreads);
+    f32_combine_kernel<<<blocks, kThreads, 0, stream>>>(partial, ids, coef, M, A, E, N, y);
+}
+
 // ---- host side --------------------------------------------------------------------------------------------------
 struct QV {
     const uint8_t *q;
@@ -1096,11 +1118,10 @@ int swiglu_ks(int64_t spans, int D) {
 }
 
 #include "decode_gemv.hpp"
-#include "f32act.hpp"
 
-// ---- FP32 activations (f32act.hpp) -----------------------------------------------------------------------------------
-f32a::Args f32_args(const QV &w, int64_t E, const void *x, void *y, int64_t ncol) {
-    f32a::Args a{};
+// ---- FP32 activations and Q5 experts (exact_tile.hip) -----------------------------------------------------------------
+xt::Args tile_args(const QV &w, int64_t E, const void *x, void *y, int64_t ncol) {
+    xt::Args a{};
     a.x = x, a.q = w.q, a.scale = w.scale, a.minv = w.minv;
     a.N = w.N / E, a.K = w.K, a.G = w.G, a.E = E, a.y = y, a.ldy = ncol, a.ncol = ncol;
     return a;
@@ -1126,27 +1147,17 @@ void f32_gather(const char *fn, const void *x, const QV &w, int64_t E, const voi
     STRIX_CHECK(act == Act::F32 || act == Act::BF16, fn, ": unsupported activation dtype ", (int)act);
     const int64_t ncol = swi ? w.N / E / 2 : w.N / E;
     check_f32(fn, x, w, E, M, A, y, M * A * ncol, M, act == Act::F32 ? 4 : 2);
-    f32a::Args a = f32_args(w, E, x, y, ncol);
+    xt::Args a = tile_args(w, E, x, y, ncol);
     a.A = A, a.S = M * A;
-    auto go = [&](auto mode, auto ty) {
-        constexpr int MD = decltype(mode)::value;
-        using T = decltype(ty);
-        if (swi) f32a::launch_bits<MD, true, T, T>(w.bits, a, stream);
-        else f32a::launch_bits<MD, false, T, T>(w.bits, a, stream);
-    };
-    auto by_act = [&](auto mode) {
-        if (act == Act::F32) go(mode, float{});
-        else go(mode, uint16_t{});
-    };
     if (ws != nullptr) {
         STRIX_CHECK(ws_bytes >= moe_route_workspace_bytes(M, A, E), fn, ": workspace of ", ws_bytes, " bytes, needs ",
                     moe_route_workspace_bytes(M, A, E));
         a.ws = static_cast<const int32_t *>(ws);
-        by_act(std::integral_constant<int, f32a::GROUPED_POS>{});
+        xt::project(w.bits, xt::GROUPED, swi, act, act, a, stream);
     } else {
         STRIX_CHECK(ids != nullptr && err != nullptr, fn, ": null ids or err");
         a.ids = ids, a.err = err;
-        by_act(std::integral_constant<int, f32a::PERSLOT_IDS>{});
+        xt::project(w.bits, xt::PERSLOT, swi, act, act, a, stream);
     }
     STRIX_HIP_CHECK_LAUNCH(fn, " ", act_str(act), " M=", M, " A=", A, " E=", E, " Q", w.bits);
 }
@@ -1473,11 +1484,10 @@ void combine_grouped(const char *fn, const void *h, const V &wv, int64_t E, cons
         check_f32(fn, h, w, E, M, A, partial, M * A * N, M * A);
         STRIX_CHECK(ws_bytes >= moe_route_workspace_bytes(M, A, E), fn, ": workspace of ", ws_bytes, " bytes, needs ",
                     moe_route_workspace_bytes(M, A, E));
-        f32a::Args a = f32_args(w, E, h, partial, N);
+        xt::Args a = tile_args(w, E, h, partial, N);
         a.A = 1, a.S = M * A, a.ws = static_cast<const int32_t *>(ws);  // h and partial rows are slots
-        f32a::launch_bits<f32a::GROUPED_POS, false, float>(w.bits, a, stream);
-        const unsigned blocks = (unsigned)((M * N + 255) / 256);
-        f32a::f32_combine_kernel<<<blocks, 256, 0, stream>>>(partial, ids, coef, M, A, E, N, static_cast<float *>(y));
+        xt::project(w.bits, xt::GROUPED, false, Act::F32, Act::F32, a, stream);
+        f32_combine(partial, ids, coef, M, A, E, N, static_cast<float *>(y), stream);
         STRIX_HIP_CHECK_LAUNCH(fn, " F32 combine M=", M, " N=", N);
         if (shared != nullptr)
             moe_shared_add(y, shared->s, shared->gate_logit, shared->gate_ld, M, N, shared->gate_index, Act::F32,
@@ -1621,11 +1631,9 @@ void linear_q4_experts_combine(const void *h, const Q4DeviceView &w, int64_t E, 
         const int64_t N = v.N / E;
         check_f32(fn, h, v, E, M, A, y, M * N, M * A);
         STRIX_CHECK(ids != nullptr && err != nullptr && coef != nullptr, fn, ": null ids, err or coef");
-        f32a::Args a = f32_args(v, E, h, y, N);
+        xt::Args a = tile_args(v, E, h, y, N);
         a.A = A, a.S = M, a.ids = ids, a.err = err;
-        const int64_t blocks = (M * N + 3) / 4;
-        STRIX_CHECK(blocks < (1ll << 31), fn, ": M * N too large");
-        f32a::f32_perslot_combine_kernel<4, float, float><<<(unsigned)blocks, 256, 0, stream>>>(a, coef, M);
+        xt::perslot_combine(4, Act::F32, a, coef, stream);
         STRIX_HIP_CHECK_LAUNCH(fn, " F32 M=", M, " A=", A, " E=", E);
         return;
     }
@@ -1686,18 +1694,17 @@ void linear_q5_experts_combine_grouped(const void *h, const Q5DeviceView &w, int
                         shared->gate_ld >= 1 && reinterpret_cast<uintptr_t>(shared->s) % 16 == 0,
                     fn, ": shared add with a null pointer, gate_ld < 1 or a misaligned s");
     // FP32 per-slot partials (h and partial rows are slots), then the ordered sum in the activation dtype
-    f32a::Args a = f32_args(v, E, h, partial, N);
+    xt::Args a = tile_args(v, E, h, partial, N);
     a.A = 1, a.S = M * A, a.ws = static_cast<const int32_t *>(ws);
     if (act == Act::F32) {
-        f32a::launch_bits<f32a::GROUPED_POS, false, float, float>(5, a, stream);
-        f32a::f32_combine_kernel<<<(unsigned)((M * N + 255) / 256), 256, 0, stream>>>(partial, ids, coef, M, A, E, N,
-                                                                                      static_cast<float *>(y));
+        xt::project(5, xt::GROUPED, false, Act::F32, Act::F32, a, stream);
+        f32_combine(partial, ids, coef, M, A, E, N, static_cast<float *>(y), stream);
         STRIX_HIP_CHECK_LAUNCH(fn, " F32 M=", M, " N=", N);
         if (shared != nullptr)
             moe_shared_add(y, shared->s, shared->gate_logit, shared->gate_ld, M, N, shared->gate_index, Act::F32,
                            shared->err, stream);
     } else {
-        f32a::launch_bits<f32a::GROUPED_POS, false, float, uint16_t>(5, a, stream);
+        xt::project(5, xt::GROUPED, false, Act::BF16, Act::F32, a, stream);
         combine_reduce(partial, ids, coef, M, A, E, N, static_cast<uint16_t *>(y), shared, nullptr, nullptr, stream);
         STRIX_HIP_CHECK_LAUNCH(fn, " BF16 M=", M, " N=", N);
     }
@@ -1722,12 +1729,9 @@ void linear_q5_experts_combine(const void *h, const Q5DeviceView &w, int64_t E, 
     const int64_t N = v.N / E;
     check_f32(fn, h, v, E, M, A, y, M * N, M * A, act == Act::F32 ? 4 : 2);
     STRIX_CHECK(ids != nullptr && err != nullptr && coef != nullptr, fn, ": null ids, err or coef");
-    f32a::Args a = f32_args(v, E, h, y, N);
+    xt::Args a = tile_args(v, E, h, y, N);
     a.A = A, a.S = M, a.ids = ids, a.err = err;
-    const int64_t blocks = (M * N + 3) / 4;
-    STRIX_CHECK(blocks < (1ll << 31), fn, ": M * N too large");
-    if (act == Act::F32) f32a::f32_perslot_combine_kernel<5, float, float><<<(unsigned)blocks, 256, 0, stream>>>(a, coef, M);
-    else f32a::f32_perslot_combine_kernel<5, uint16_t, uint16_t><<<(unsigned)blocks, 256, 0, stream>>>(a, coef, M);
+    xt::perslot_combine(5, act, a, coef, stream);
     STRIX_HIP_CHECK_LAUNCH(fn, " ", act_str(act), " M=", M, " A=", A, " E=", E);
 }
 
@@ -1769,14 +1773,13 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
     STRIX_CHECK(act == Act::BF16 || act == Act::F32, fn, ": unsupported activation dtype ", (int)act);
     STRIX_CHECK(out_act == Act::BF16 || out_act == Act::F32, fn, ": output dtype ", (int)out_act);
     check_view(fn, v, 1);
-    if (act == Act::F32) {  // FP32 activations: f32act.hpp
+    if (act == Act::F32) {  // FP32 activations: exact_tile.hip
         STRIX_CHECK(M >= 1 && v.K % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, fn, ": M = ", M, ", K = ", v.K,
                     " (a multiple of 32) and x 16-byte aligned with FP32 activations");
         STRIX_CHECK(disjoint(y, M * v.N * (out_act == Act::F32 ? 4 : 2), x, M * v.K * 4), fn, ": y overlaps x");
-        f32a::Args a = f32_args(v, 1, x, y, v.N);
+        xt::Args a = tile_args(v, 1, x, y, v.N);
         a.A = 1, a.S = M;
-        if (out_act == Act::F32) f32a::launch_bits<f32a::DENSE_ROWS, false, float>(v.bits, a, stream);
-        else f32a::launch_bits<f32a::DENSE_ROWS, false, uint16_t>(v.bits, a, stream);
+        xt::project(v.bits, xt::DENSE, false, Act::F32, out_act, a, stream);
         STRIX_HIP_CHECK_LAUNCH(fn, " F32 M=", M, " N=", v.N, " K=", v.K);
         return;
     }

@@ -55,3 +55,52 @@ def test_streamed_experts_at_the_served_widths(M, A, E, H, I):
     b, q, s, m, G = qspec(dn)
     pref = orc.experts_down(hz, orc.qview(b, q, s, m, dn.N, I, G), E, ok_ids)
     assert rel_err(p[good], pref[good]) < 1e-4  # FP32 sums of 640 products in another order
+
+
+def _w64(w: moe.QWeight) -> np.ndarray:
+    from oracle import hc
+
+    return hc.weights64(w.bits, to_np(w.q), to_np(w.scale), to_np(w.minv), w.N, w.K, w.G)
+
+
+def _rel64(got: torch.Tensor, ref: np.ndarray) -> float:
+    return float(np.abs(got.double().cpu().numpy() - ref).max() / np.abs(ref).max())
+
+
+# exact-weight 16-row tiles with FP32 activations: one step of K, K split over 4 and 8 waves, a ragged column end
+# (I = 24: half a tile of columns), rows past the tiles, each K step length
+@pytest.mark.parametrize("bits,G,K,I", [(4, 128, 128, 24), (4, 128, 4096, 16), (4, 64, 576, 40), (4, 32, 1024, 24),
+                                        (8, 64, 448, 24), (8, 128, 2048, 32), (8, 32, 96, 8)])
+def test_fp32_activation_tiles(bits, G, K, I):
+    say("fp32 tiles", bits, G, K, I)
+    M, A, E = 19, 2, 3
+    gu = _weight(bits, E * 2 * I, K, G, 41)
+    g64 = _w64(gu)
+    x = torch.from_numpy(np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)).to(DEV)
+    X = x.double().cpu().numpy()
+    ids = np.stack([np.random.default_rng(m).permutation(E)[:A] for m in range(M)]).astype(np.int32)
+    tid = torch.from_numpy(ids).to(DEV)
+    ws, _ = moe.moe_group_routes(tid, E)
+    ref = np.stack([X[s // A] @ g64[e * 2 * I:(e + 1) * 2 * I].T for s, e in enumerate(ids.ravel())])
+    href = ref[:, :I] / (1 + np.exp(-ref[:, :I])) * ref[:, I:]
+    h = moe.experts_gather_grouped_swiglu(x, gu, E, ws, M, A)
+    # every product is exact, so the error is that of FP32 sums of up to 4096 terms whose partial sums reach a few
+    # times the result (code offsets): ~sqrt(4096) 2^-24 x 4
+    assert _rel64(h, href) < 2e-5
+    if bits == 4:
+        assert _rel64(moe.experts_gather_grouped(x, gu, E, ws, M, A), ref) < 2e-5
+        assert torch.equal(moe.experts_gather(x, gu, E, tid, moe.zero_err(), swiglu=True), h)
+    lin = moe.linear_q4 if bits == 4 else moe.linear_q8
+    d64 = X @ g64.T
+    assert _rel64(lin(x, gu, out_dtype=torch.float32), d64) < 2e-5
+
+
+def test_fp32_router_rows_match_bf16_bits():
+    say("fp32 router")
+    # FP32 x holding BF16 values: the canonical order's bits, with token counts around the four-token groups, chunk
+    # counts that leave lanes without a last chunk, and rows that are not 16-byte aligned
+    for M, N, K in [(1, 33, 2560), (2, 5, 520), (5, 17, 1000), (9, 4, 1003)]:
+        rng = np.random.default_rng(M)
+        x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+        w = torch.from_numpy(rng.standard_normal((N, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+        assert torch.equal(moe.linear_bf16w(x.float(), w), moe.linear_bf16w(x, w)), (M, N, K)
