@@ -332,7 +332,7 @@ __global__ void __launch_bounds__((W + 1) * kWave) decode_gate_up_lds_kernel(Dec
     __shared__ __attribute__((aligned(16))) uint4 rg0[W][PU4], rg1[W][2 * kWave], rg2[W][PU4], rg3[W][2 * kWave];
     __shared__ float4v red[2][W][2][kWave];
     __shared__ int32_t tb[kDecMaxTilesL];
-    __shared__ int32_t tslot[gul::kGuMaxBlockTiles][16];
+    __shared__ __attribute__((aligned(16))) int32_t tslot[gul::kGuMaxBlockTiles][16];
     int bid = (int)blockIdx.x, nblk = (int)gridDim.x;
     if constexpr (SH == 1) {
         if (bid < sh.blocks) {  // the shared expert's gate_up finish: h = bf16(silu(sum g) * sum u), a thread each
@@ -398,13 +398,30 @@ __global__ void __launch_bounds__((W + 1) * kWave) decode_gate_up_lds_kernel(Dec
             const int32_t t = u / upt, c = u % upt;
             const int32_t bucket = tb[t];
             const bool nan = bucket < 0 || bucket >= a.E;
+            if constexpr (GA) {
+                // lane (g, j): tile rows 4 g .. 4 g + 3 of column j, the layout the K parts were written in: one 16-byte
+                // read a part for all 16 rows. (A pass a 4 rows, as below, costs a buckets' rows / 4 round trips of LDS a
+                // unit, and the streaming waves wait for the finisher once it is slower than a unit's stream.)
+                float4v gv = {0, 0, 0, 0}, uv = {0, 0, 0, 0};
+#pragma unroll
+                for (int w = 0; w < W; ++w) gv += red[par][w][0][lane], uv += red[par][w][1][lane];
+                const int4 sl = *reinterpret_cast<const int4 *>(&tslot[t - T0][4 * g]);
+                const int32_t slot[4] = {sl.x, sl.y, sl.z, sl.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = nan ? qnan() : silu(gv[i]) * uv[i];
+                    __builtin_amdgcn_raw_buffer_store_b16(
+                        f32_to_bf16(v), ry,
+                        slot[i] >= 0 ? ((uint32_t)slot[i] * ldh + 16u * (uint32_t)c + j) * 2 : a.y_bytes, 0, 0);
+                }
+                continue;
+            }
             // lane (rs, j): tile rows 4 pass + rs, column j (a row with slot -1, past the record's rows, is skipped)
             for (int k0 = 0; k0 < 16; k0 += 4) {
                 const int32_t sl = tslot[t - T0][k0 + g];
                 if (__builtin_amdgcn_readfirstlane(tslot[t - T0][k0]) < 0) break;
                 if (sl < 0) continue;
-                // the MFMA row of the slot: its token (decode) or its place in the tile (GA)
-                const uint32_t tok = GA ? (uint32_t)(k0 + g) : (uint32_t)sl / A32, i = tok % 4;
+                const uint32_t tok = (uint32_t)sl / A32, i = tok % 4;  // the MFMA row of the slot: its token
                 const int src = (int)(tok / 4) * 16 + j;
                 float gv = 0.f, uv = 0.f;
 #pragma unroll
