@@ -1765,8 +1765,15 @@ void swiglu(const void *gu, void *h, int64_t rows, int64_t I, Act act, hipStream
 }
 
 namespace {
-// y [M, N] = x [M, K] . dequant(W)^T for one Q4 or Q8 weight: 16-token tiles, each wave streaming 32 weight rows
-// over all of K (the DENSE mode of the stream kernel); FP32 accumulation, y stored in out_act
+// Dense projections of fewer than 64 tokens, or of M N up to this, take the exact 16-row tiles (K split over a block's
+// waves), larger ones the LDS-tiled GEMM of 64-token tiles. The GEMM's blocks walk K alone, a time in proportion to K
+// until they fill the chip; the tiles convert the weights' codes once for 16 tokens, a time in proportion to M N K.
+// Measured on MI355X (gate_up + SwiGLU + down of one FFN, tiles / GEMM): H 3072, I 512, Q8 g64 at 100 tokens 26 us (the
+// stream kernel that walked K alone: 56), at 130 34 / 62, 200 41 / 62, 300 55 / 62, 500 72 / 62 (tiles for the down only:
+// 73); H 3072, I 2048, Q4 at 100 73 / 79, at 130 97 / 78.
+constexpr int64_t kDenseTileOutputs = 400000;
+
+// y [M, N] = x [M, K] . dequant(W)^T for one Q4 or Q8 weight, FP32 accumulation, y stored in out_act
 void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64_t M, Act act, Act out_act,
                       hipStream_t stream) {
     STRIX_CHECK(x != nullptr && y != nullptr, fn, ": null pointer (x=", x, ", y=", y, ")");
@@ -1790,8 +1797,7 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
     STRIX_CHECK(disjoint(y, M * v.N * oes, x, M * v.K * 2), fn, ": y overlaps x");
     GemmArgs a = make_args(v, 1, x, y, v.N);
     a.M = M;
-    // prefill-size batches on the matrix-core GEMM (exact weights, 64-token tiles), decode sizes on the stream kernel
-    if (M >= 128 && v.K % gemm::BK == 0 && v.G % gemm::BK == 0 && v.K / v.G <= gemm::kMaxGroups) {
+    if (M >= 64 && M * v.N > kDenseTileOutputs && v.K % gemm::BK == 0 && v.G % gemm::BK == 0 && v.K / v.G <= gemm::kMaxGroups) {
         auto go = [&](auto bits) {
             constexpr int B = decltype(bits)::value;
             if (out_act == Act::F32) launch_expert_gemm<B, DENSE, EPI_F32, false, false>(a, stream);
@@ -1799,10 +1805,10 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
         };
         if (v.bits == 4) go(std::integral_constant<int, 4>{});
         else go(std::integral_constant<int, 8>{});
-    } else if (out_act == Act::F32) {
-        launch_bits<DENSE, EPI_F32, false, false, false>(v.bits, a, (M + 15) / 16, stream);
     } else {
-        launch_bits<DENSE, EPI_BF16, false, false, false>(v.bits, a, (M + 15) / 16, stream);
+        xt::Args t = tile_args(v, 1, x, y, v.N);
+        t.A = 1, t.S = M;
+        xt::project(v.bits, xt::DENSE, false, Act::BF16, out_act, t, stream);
     }
     STRIX_HIP_CHECK_LAUNCH(fn, " M=", M, " N=", v.N, " K=", v.K, " G=", v.G);
 }
@@ -2037,8 +2043,10 @@ void moe_layer_forward(const MoeLayerWeights &w, const void *x, int64_t M, const
             launch_expert_gemm<8, DENSE, EPI_SWIGLU, false, false>(a, sh_stream);
             launch_expert_gemm<8, DENSE, EPI_BF16, false, false>(b, sh_stream);
         } else {
-            launch_gemm<8, DENSE, EPI_SWIGLU, false, false, false>(a, (M + 15) / 16, sh_stream);
-            launch_gemm<8, DENSE, EPI_BF16, false, false, false>(b, (M + 15) / 16, sh_stream);
+            xt::Args tg = tile_args(gv, 1, x, sh_h, I), td = tile_args(dv, 1, sh_h, sh_s, H);
+            tg.A = td.A = 1, tg.S = td.S = M;
+            xt::project(8, xt::DENSE, true, Act::BF16, Act::BF16, tg, sh_stream);
+            xt::project(8, xt::DENSE, false, Act::BF16, Act::BF16, td, sh_stream);
         }
         STRIX_HIP_CHECK_LAUNCH(fn, " shared expert M=", M);
         if (ctx != nullptr) STRIX_HIP_CHECK(hipEventRecord(ctx->join, ctx->s), fn, ": join");

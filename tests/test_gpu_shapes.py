@@ -104,3 +104,16 @@ def test_fp32_router_rows_match_bf16_bits():
         x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
         w = torch.from_numpy(rng.standard_normal((N, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
         assert torch.equal(moe.linear_bf16w(x.float(), w), moe.linear_bf16w(x, w)), (M, N, K)
+
+
+# dense BF16 on either side of the tiles' and the GEMM's sizes, with a remainder of the 16-token tiles
+@pytest.mark.parametrize("bits,G,M,N,K", [(8, 64, 17, 1040, 3072), (4, 128, 111, 96, 512), (8, 64, 113, 4096, 2048),
+                                          (4, 64, 300, 1024, 2048), (8, 32, 1, 16, 96)])
+def test_dense_tiles_and_gemm(bits, G, M, N, K):
+    say("dense", bits, G, M, N, K)
+    w = _weight(bits, N, K, G, 51)
+    x = _bf16(orc.gen_bf16_normal(orc.tensor_key(9, "x"), 1.0, (M, K)))
+    ref = x.double().cpu().numpy() @ _w64(w).T
+    lin = moe.linear_q4 if bits == 4 else moe.linear_q8
+    assert _rel64(lin(x, w, out_dtype=torch.float32), ref) < 1e-4  # FP32 sums; the GEMM's Q4 codes carry an offset of 128
+    assert _rel64(lin(x, w), ref) < 2.0 ** -8  # one BF16 rounding
