@@ -12,9 +12,9 @@
 //     j])), W_up [4 d, r] chunk-major (32-code chunk c of row n at q[(c N + n) * 16] (Q4) or [(c N + n) * 32] (Q8),
 //     group g's scale / min at [g N + n]; strixite formats/q4.hpp:43-55).
 //
-// Two kernel designs, chosen by the token count:
+// The kernels, chosen by the token count (kDownDotTokens):
 //
-// * Matrix-core tiles (the up mix from 1 token; the down mix from 256 tokens and d % 128 == 0). Weights enter the
+// * Matrix-core tiles (the up mix from 1 token; the down mix of large batches with d % 128 == 0). Weights enter the
 //   bf16 MFMA (v_mfma_f32_16x16x32_bf16) as their exact integer codes and each quantization group's partial product D is
 //   rescaled on the FP32 accumulator: w . x = s D + m' sum(x) (Q4 codes enter as 128 + n with m' = m - 128 s, Q8
 //   codes as c - 128 with m' = m + 128 s). The min terms of a whole K stage are one FP32 MFMA
@@ -35,11 +35,9 @@
 //     the epilogue happens in registers. h is converted to bf16 [hi, mid, lo] into LDS once per block (with its group
 //     sums); the chunk-major codes of a chunk's 16 rows are 256 (Q4) or 512 (Q8) contiguous bytes, read by the
 //     wave's lanes directly, four chunks ahead.
-// * Vector rows (down mix below 256 tokens, or d % 128 != 0): a block of 4 waves computes the group's inverse RMS into
-//   LDS, then each wave takes one weight row (T = 1: a row's chunks split over the 4 waves): lane l dots the row's
-//   32-code chunks l, l + 64, ... with the chunk of every token of the group (the codes converted to floats once for
-//   the group) and adds each dot scaled by its stream's inverse RMS into one accumulator a token; a butterfly ends it.
+// * Split-K tiles and lane dots (down mix, smaller batches): described at mix_down_split_kernel and mix_down_dot_kernel.
 #include "common.hpp"
+#include "exact_frag.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -53,33 +51,30 @@ namespace {
 using namespace strix::dev;
 constexpr int kWave = 64, kStreams = 4, kChunk = 32;
 constexpr int64_t kMaxR = 1024, kMaxTokens = 65535, kMaxD = 1 << 20;
-// the down mix's matrix-core tiles from this many tokens: a 32-token tile block streams the whole weight, so with fewer
-// tiles than CUs the vector-row kernel, which spreads the rows over the CUs, is faster (measured at d 2560, r 320: tiles
-// ~100 us flat up to a few hundred tokens; rows 8 us at 1 token, ~60 at 64)
-constexpr int64_t kDownTileMinTokens = 256;
+// The down mix's kernels (us on MI355X at d 2560, r 320, Q4 g64):
+// - lane dots up to this many BF16 tokens: 4.3 at 1 token, 6.1 at 4, 10.2 at 16, 19 at 40, 27 at 64, in proportion;
+// - split-K tiles above, as long as their blocks are at most the CUs (16 tokens x 16 rows a block 18 us flat, 16 x 32 24,
+//   32 x 32 36, 32 x 64 50): a block's time is its K walk, whatever the grid;
+// - then the staged tiles, flat in T until their blocks pass the CUs.
+// FP32 streams (three MFMA rows or products a value): lane dots (20 at 40 tokens, 99 at 255) up to the staged tiles' 168.
+// Before: vector rows 5.6 / 12 / 24 / 35 / 45, 146 at 255 tokens (FP32 43 at 16, 426 at 255), staged tiles 104 from 256.
+constexpr int64_t kDownDotTokens = 32, kDownTileF32Tokens = 440;
+constexpr size_t kDownSplitLds = 160 * 1024 - 1024;
+
+int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n = 256;
+        return n > 0 ? n : 256;
+    }();
+    return cus;
+}
 
 __device__ __forceinline__ float ld_act(const float *p, int64_t i) { return p[i]; }
 __device__ __forceinline__ float ld_act(const uint16_t *p, int64_t i) { return bf16_to_f32(p[i]); }
 __device__ __forceinline__ void st_act(float *p, int64_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void st_act(uint16_t *p, int64_t i, float v) { p[i] = f32_to_bf16(v); }
-
-// 8 consecutive activations at element offset i (16-byte aligned for BF16, 32 for F32)
-__device__ __forceinline__ void ld8(const uint16_t *p, int64_t i, float (&v)[8]) {
-    const uint4 u = *reinterpret_cast<const uint4 *>(p + i);
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[2 * k] = __uint_as_float(w[k] << 16), v[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
-}
-__device__ __forceinline__ void ld8(const float *p, int64_t i, float (&v)[8]) {
-    const float4 a = *reinterpret_cast<const float4 *>(p + i), b = *reinterpret_cast<const float4 *>(p + i + 4);
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
-}
 
 // 8 Q4 codes (a dword, code i at bits 4 i) -> bf16 128 + code in the paired k order k0 k2 k4 k6 k1 k3 k5 k7
 __device__ __forceinline__ Frag q4_paired(uint32_t w) {
@@ -430,114 +425,343 @@ __global__ void __launch_bounds__(dn::kThreads)
 
 template <int BITS, bool F32> constexpr size_t down_tile_lds() { return (size_t)2 * dn::Stage<BITS, F32>::SIZE * 4; }
 
-// ================================================================================================ down: vector rows
-// KS waves share a row (its chunks split over them, their totals meeting in LDS) or, KS = 1, a wave takes one row; MT
-// tokens a block. The streams' inverse RMS is known before the dot products (the block's first phase), so each
-// chunk's dot goes straight into one accumulator a token, scaled by its stream's inverse RMS:
-// a = sum over chunks of inv[stream(chunk)] (s dot + m sum(x)).
-template <typename T, int BITS, int MT, int KS>
-__global__ void __launch_bounds__(256)
-    mix_down_rows_kernel(const T *x, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, int64_t R,
-                         int64_t d, int64_t G, int64_t r, float eps, int64_t Tn, float *h, float *w_in, float *inv) {
-    constexpr int kWaves = 4;
-    __shared__ float invs[MT][kStreams];
-    __shared__ float red[KS > 1 ? kWaves : 1][MT];  // KS > 1: wave w's totals (its row w / KS, part w % KS)
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int64_t K = kStreams * d, t0 = (int64_t)blockIdx.y * MT;
-    const int nt = (int)(Tn - t0 < MT ? Tn - t0 : MT);
-    // wave s: the inverse RMS of stream s of each token of the group (the tokens' loads of a step issued together)
-    {
-        float sq[MT];
+// ================================================================================================ down: split-K tiles
+// A block takes TT 16-token tiles against RT tiles of 16 weight rows (BF16 streams), and its NW waves split K: NW / 4 to
+// a stream. A wave also squares its tokens with the matrix cores (x against itself: the diagonal of one more MFMA), so
+// the streams' inverse RMS costs no other pass. The waves' parts meet in LDS once, in wave order: a = sum_s inv_s (P of
+// the stream's waves). The codes enter about the middle of their range, so no sum is larger than the result; single-tile
+// blocks, where lane dots would be the alternative, also keep their running sums in two levels: the error against 64
+// bits stays at the lane dots' (1.3e-7).
+// What bounds it: the address path (16 rows a load) and the latency of the wave's K walk. The wave's scales and mins go
+// through LDS: as 2-byte loads a step and row they took a third of the time (16 x 32 blocks: 38 -> 24 us).
+// codes 8 u .. 8 u + 7 of the lane about the middle of their range, exact in bf16, in the paired order: 16 (n - 8) (Q4: the
+// nibble in a byte's upper half is the signed byte), c - 128 (Q8)
+template <int BITS> __device__ __forceinline__ Frag signed_frag(const xt::Codes &c, int u) {
+    auto sb = [](uint32_t v, int i) { return (float)(int8_t)(uint8_t)(v >> (8 * i)); };
+    uint32_t a, b;
+    if constexpr (BITS == 4) a = ((c.w[u] << 4) & 0xF0F0F0F0u) ^ 0x80808080u, b = (c.w[u] & 0xF0F0F0F0u) ^ 0x80808080u;
+    else a = c.w[2 * u] ^ 0x80808080u, b = c.w[2 * u + 1] ^ 0x80808080u;
+    if constexpr (BITS == 4)  // a: k0 k2 k4 k6, b: k1 k3 k5 k7
+        return Frag{{hi16_pair(sb(a, 0), sb(a, 1)), hi16_pair(sb(a, 2), sb(a, 3)), hi16_pair(sb(b, 0), sb(b, 1)),
+                     hi16_pair(sb(b, 2), sb(b, 3))}};
+    else
+        return Frag{{hi16_pair(sb(a, 0), sb(a, 2)), hi16_pair(sb(b, 0), sb(b, 2)), hi16_pair(sb(a, 1), sb(a, 3)),
+                     hi16_pair(sb(b, 1), sb(b, 3))}};
+}
+
+template <int BITS, int SP, int TT, int RT, int NW>
+__global__ void __launch_bounds__(NW *kWave)
+    mix_down_split_kernel(const uint16_t *x, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, int64_t R,
+                          int64_t d, int64_t G, int64_t r, float eps, int64_t Tn, float *h, float *w_in, float *inv_out,
+                          uint32_t ng_max) {
+    using F = xt::Fmt<BITS, SP>;
+    constexpr int TR = 16, TOK = TT * TR, PW = NW / kStreams;
+    extern __shared__ float4v part[];  // [NW][TT][RT + 1][kWave]: the waves' sums, then their squares
+    __shared__ float invs[TOK][kStreams];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int g = lane / 16, j = lane % 16;
+    const uint32_t nrb = (uint32_t)((R + 16 * RT - 1) / (16 * RT));
+    const uint32_t L = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t t0 = (int64_t)(L / nrb) * TOK, r0 = (int64_t)(L % nrb) * 16 * RT, K = kStreams * d;
+    const uint32_t groups = (uint32_t)(K / G), row_bytes = (uint32_t)(K * BITS / 8);
+    auto res = [](const void *p, int64_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+    };
+    // rows past the weight and tokens past the batch repeat the last one (their sums are not stored)
+    const int64_t rows = R - r0 < 16 * RT ? R - r0 : 16 * RT, toks = Tn - t0 < TOK ? Tn - t0 : TOK;
+    const __amdgpu_buffer_rsrc_t rq = res(q + r0 * row_bytes, rows * row_bytes), rs = res(scale + r0 * groups, rows * groups * 2),
+                                 rm = res(minv + r0 * groups, rows * groups * 2);
+    const uint16_t *xb = x + t0 * K;
+    uint32_t wrow[RT];
+    const uint16_t *xp[TT];
 #pragma unroll
-        for (int tt = 0; tt < MT; ++tt) sq[tt] = 0.f;
-        for (int64_t i = 8 * lane; i < d; i += 8 * kWave) {
-            float v[MT][8];
+    for (int t = 0; t < RT; ++t) wrow[t] = (uint32_t)(16 * t + j < rows ? 16 * t + j : rows - 1);
 #pragma unroll
-            for (int tt = 0; tt < MT; ++tt)
-                if (tt < nt) ld8(x + (t0 + tt) * K + (int64_t)wave * d, i, v[tt]);
+    for (int t = 0; t < TT; ++t) {
+        const int tok = TR * t + j;
+        xp[t] = xb + (tok < toks ? tok : toks - 1) * K;
+    }
+    const int stream = wave / PW, steps = (int)(d / SP);
+    const int s0 = steps * (wave % PW) / PW, s1 = steps * (wave % PW + 1) / PW;
+    struct Buf {
+        xt::Codes c[RT];
+        xt::Act8<uint16_t> x[TT][F::NT];
+    };
+    auto fetch = [&](int s, Buf &b) {
+        const uint32_t k = (uint32_t)(stream * d) + (uint32_t)s * SP + g * F::CPL;
 #pragma unroll
-            for (int tt = 0; tt < MT; ++tt)
-                if (tt < nt)
+        for (int t = 0; t < RT; ++t) xt::load_codes<BITS, SP>(rq, wrow[t] * row_bytes, (uint32_t)K, k, b.c[t]);
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) sq[tt] = fmaf(v[tt][k], v[tt][k], sq[tt]);
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int u = 0; u < F::NT; ++u) b.x[t][u].load(xp[t] + k + 8 * u);
+    };
+    // the wave's scales and mins, (scale, min) pairs by group then row: consecutive lanes read consecutive groups of a row
+    // (a 2-byte load a step and row would cost the address path as much as the codes)
+    const uint32_t g0 = (uint32_t)(stream * d + (int64_t)s0 * SP) / (uint32_t)G,
+                   ng = s1 > s0 ? (uint32_t)(stream * d + (int64_t)s1 * SP - 1) / (uint32_t)G - g0 + 1 : 0;
+    uint32_t *sm = reinterpret_cast<uint32_t *>(part) + wave * ng_max * 16 * RT;
+    for (uint32_t i = lane; i < ng * 16 * RT; i += kWave) {
+        const uint32_t row = i / ng, gi = i % ng, wr = row < (uint32_t)rows ? row : (uint32_t)rows - 1, o = (wr * groups + g0 + gi) * 2;
+        const uint32_t sv = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, o, 0, 0),
+                       mv = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rm, o, 0, 0);
+        sm[gi * 16 * RT + row] = sv | mv << 16;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const Frag ones{{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}};
+    float4v tot[TT][RT], acc[TT][RT], sq[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        sq[t] = float4v{0, 0, 0, 0};
+#pragma unroll
+        for (int n = 0; n < RT; ++n) tot[t][n] = acc[t][n] = float4v{0, 0, 0, 0};
+    }
+    auto step = [&](Buf &b, int s, int next) {
+        float4v D[TT][RT], dx[TT];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            dx[t] = float4v{0, 0, 0, 0};
+#pragma unroll
+            for (int n = 0; n < RT; ++n) D[t][n] = float4v{0, 0, 0, 0};
         }
 #pragma unroll
-        for (int tt = 0; tt < MT; ++tt) {
-            const float tot = wave_sum(sq[tt]);
-            if (lane == 0 && tt < nt) invs[tt][wave] = 1.0f / sqrtf(tot / (float)d + eps);
+        for (int u = 0; u < F::NT; ++u) {
+            Frag w[RT];
+#pragma unroll
+            for (int n = 0; n < RT; ++n) w[n] = signed_frag<BITS>(b.c[n], u);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const Frag a = b.x[t][u].frag(j);
+#pragma unroll
+                for (int n = 0; n < RT; ++n) D[t][n] = mfma_bf16(a, w[n], D[t][n]);
+                dx[t] = mfma_bf16(a, ones, dx[t]);
+                sq[t] = mfma_bf16(a, a, sq[t]);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // a group of codes is decoded just before its MFMAs (registers)
         }
+        float sc[RT], mp[RT];
+#pragma unroll
+        for (int n = 0; n < RT; ++n) {
+            const uint32_t w = sm[((uint32_t)(stream * d + (int64_t)s * SP) / (uint32_t)G - g0) * 16 * RT + 16 * n + j];
+            sc[n] = __uint_as_float(w << 16), mp[n] = fmaf(F::MID, sc[n], __uint_as_float(w & 0xFFFF0000u));
+            if constexpr (BITS == 4) sc[n] *= 0.0625f;
+        }
+        if (next < s1) fetch(next, b);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int n = 0; n < RT; ++n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[t][n][i] = fmaf(sc[n], D[t][n][i], fmaf(mp[n], dx[t][i], acc[t][n][i]));
+    };
+    Buf b0, b1;
+    if (s0 < s1) fetch(s0, b0);
+    if (s0 + 1 < s1) fetch(s0 + 1, b1);
+    for (int s = s0; s < s1; s += 2) {
+        step(b0, s, s + 2);
+        if (s + 1 < s1) step(b1, s + 1, s + 3);
+        if (TT == 1 && ((s - s0) % 4 == 2 || s + 2 >= s1))  // sums of sums of four steps: a shorter chain of roundings
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int n = 0; n < RT; ++n) tot[t][n] += acc[t][n], acc[t][n] = float4v{0, 0, 0, 0};
+    }
+    __syncthreads();  // the scales are read: their space takes the sums
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+#pragma unroll
+        for (int n = 0; n < RT; ++n) part[((wave * TT + t) * (RT + 1) + n) * kWave + lane] = TT == 1 ? tot[t][n] : acc[t][n];
+        part[((wave * TT + t) * (RT + 1) + RT) * kWave + lane] = sq[t];
     }
     __syncthreads();
-    if (blockIdx.x == 0 && lane == 0)
-        for (int tt = 0; tt < nt; ++tt) inv[(t0 + tt) * kStreams + wave] = invs[tt][wave];
-    const int64_t row = (int64_t)blockIdx.x * (kWaves / KS) + wave / KS;
-    const int part = wave % KS;
-    if (KS == 1 && row >= R) return;  // after the block's only barrier (KS > 1: the grid holds whole rows)
-    const int64_t grow = row < R ? row : R - 1;
-    const uint8_t *qrow = q + grow * (K * BITS / 8);
-    const int64_t nc = K / kChunk, cps = d / kChunk;  // chunks of the row, chunks a stream
-    float iv[MT][kStreams];
-#pragma unroll
-    for (int tt = 0; tt < MT; ++tt)
-#pragma unroll
-        for (int st = 0; st < kStreams; ++st) iv[tt][st] = tt < nt ? invs[tt][st] : 0.f;
-    float acc[MT];
-#pragma unroll
-    for (int tt = 0; tt < MT; ++tt) acc[tt] = 0.f;
-#pragma unroll 2
-    for (int64_t c = (int64_t)part * kWave + lane; c < nc; c += (int64_t)kWave * KS) {
-        uint32_t w[BITS];
-#pragma unroll
-        for (int i = 0; i < BITS / 4; ++i) {
-            const uint4 u = reinterpret_cast<const uint4 *>(qrow + c * (kChunk * BITS / 8))[i];
-            w[4 * i] = u.x, w[4 * i + 1] = u.y, w[4 * i + 2] = u.z, w[4 * i + 3] = u.w;
-        }
-        const int64_t gi = grow * (K / G) + c * kChunk / G;
-        const float sc = bf16_to_f32(scale[gi]), mn = bf16_to_f32(minv[gi]);
-        const int sg = (int)(c / cps);  // the chunk's stream
-        float cf[kChunk];
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k)
-            cf[k] = (float)((w[k * BITS / 32] >> ((k * BITS) % 32)) & ((1u << BITS) - 1u));
-#pragma unroll
-        for (int tt = 0; tt < MT; ++tt) {
-            if (tt >= nt) break;
-            const T *xc = x + (t0 + tt) * K + c * kChunk;
-            float dot = 0.f, xsum = 0.f;
-#pragma unroll
-            for (int p8 = 0; p8 < kChunk / 8; ++p8) {
-                float v[8];
-                ld8(xc, 8 * p8, v);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) dot = fmaf(v[k], cf[8 * p8 + k], dot), xsum += v[k];
-            }
-            const float s_inv = sg == 0 ? iv[tt][0] : sg == 1 ? iv[tt][1] : sg == 2 ? iv[tt][2] : iv[tt][3];
-            acc[tt] = fmaf(s_inv, fmaf(sc, dot, mn * xsum), acc[tt]);
-        }
+    // element (MFMA row, column) of a wave's tile (t, n)
+    auto at = [&](int w, int t, int n, int row, int col) {
+        return reinterpret_cast<const float *>(&part[((w * TT + t) * (RT + 1) + n) * kWave + row / 4 * 16 + col])[row % 4];
+    };
+    for (int i = threadIdx.x; i < TOK * kStreams; i += NW * kWave) {
+        const int tok = i / kStreams, s = i % kStreams, t = tok / TR, row = tok % TR;
+        float v = 0.f;
+        for (int p = 0; p < PW; ++p) v += at(s * PW + p, t, RT, row, row);
+        const float iv = 1.0f / sqrtf(v / (float)d + eps);
+        invs[tok][s] = iv;
+        if (r0 == 0 && tok < toks) inv_out[(t0 + tok) * kStreams + s] = iv;
     }
-    float tot[MT];
+    __syncthreads();
+    for (int i = threadIdx.x; i < TOK * 16 * RT; i += NW * kWave) {
+        // consecutive threads: 16 weight rows, then tokens (consecutive LDS words, contiguous rows of h)
+        const int col = i % 16, tok = i / 16 % TOK, n = i / (16 * TOK), t = tok / TR, row = tok % TR;
+        const int64_t wr = r0 + 16 * n + col;
+        if (tok >= toks || wr >= R) continue;
+        float a = 0.f;
 #pragma unroll
-    for (int tt = 0; tt < MT; ++tt) tot[tt] = wave_sum(acc[tt]);
-    if constexpr (KS > 1) {
-        if (lane == 0)
-#pragma unroll
-            for (int tt = 0; tt < MT; ++tt) red[wave][tt] = tot[tt];
-        __syncthreads();
-        if (part != 0) return;
-#pragma unroll
-        for (int tt = 0; tt < MT; ++tt) {
+        for (int s = 0; s < kStreams; ++s) {
             float v = 0.f;
-            for (int k = 0; k < KS; ++k) v += red[wave + k][tt];  // part 0's wave: its row's KS waves from here
-            tot[tt] = v;
+#pragma unroll
+            for (int p = 0; p < PW; ++p) v += at(s * PW + p, t, n, row, col);
+            a = fmaf(invs[tok][s], v, a);
+        }
+        const float z = a * 0.25f;
+        if (wr < r) h[(t0 + tok) * r + wr] = z / (1.0f + expf(-z));
+        else w_in[(t0 + tok) * kStreams + (wr - r)] = 2.0f / (1.0f + expf(-z));
+    }
+}
+
+// groups a wave's K range can touch
+template <int SP, int NW> uint32_t down_split_groups(int64_t d, int64_t G) {
+    const int64_t pw = NW / kStreams, steps = (d / SP + pw - 1) / pw;
+    return (uint32_t)((steps * SP + G - 1) / G + 1);
+}
+// the waves' scales and mins, then their sums
+template <int TT, int RT, int NW> size_t down_split_lds(uint32_t ng) {
+    return std::max((size_t)NW * TT * (RT + 1) * kWave * 16, (size_t)NW * ng * 16 * RT * 4);
+}
+
+// ================================================================================================ down: lane dots
+// A block takes MT tokens x RW weight rows, one wave a stream: lane l takes the stream's 8-element chunks l, l + 64, ...
+// - a token's 16 (BF16) or 32 (FP32) bytes and a row's 4 or 8 code bytes, so every load of a wave is contiguous -, a
+// chunk's dot goes s D + m sum(x) into the lane's accumulator of the (token, row), and the token's sum of squares rides
+// along. The lanes' sums meet by a reduce-scatter, the streams' in LDS: a = sum_s inv_s P_s.
+// BF16: v_dot2_f32_bf16 over the codes as bf16 (exact_frag.hpp's offsets, taken out of the dot by the chunk's sum(x)).
+// What bounds it: the vector units (7 instructions per 8 products a row, 8 a token for its sums).
+template <typename V> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, V c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2v, a), __builtin_bit_cast(bf16x2v, b), c, false);
+}
+// the sums of v[p] over the wave for p < P (a power of two, at most 64): lane l ends with that of p = l / (64 / P)
+template <int P> __device__ __forceinline__ float wave_scatter_sum(float (&v)[P]) {
+    const int lane = threadIdx.x % kWave;
+#pragma unroll
+    for (int lvl = 0; lvl < 6; ++lvl) {
+        const int o = kWave / 2 >> lvl, n = P >> lvl;
+        if (n > 1) {
+            const bool up = lane & o;
+#pragma unroll
+            for (int i = 0; i < n / 2; ++i) {
+                const float send = up ? v[i] : v[n / 2 + i];
+                const float keep = up ? v[n / 2 + i] : v[i];
+                v[i] = keep + __shfl_xor(send, o, kWave);
+            }
+        } else {
+            v[0] += __shfl_xor(v[0], o, kWave);
         }
     }
-    if (lane != 0 || row >= R) return;
-    for (int tt = 0; tt < nt; ++tt) {
-        const int64_t t = t0 + tt;
-        const float z = tot[tt] * 0.25f;
-        if (row < r) h[t * r + row] = z / (1.0f + expf(-z));
-        else w_in[t * kStreams + (row - r)] = 2.0f / (1.0f + expf(-z));
+    return v[0];
+}
+
+template <typename T, int BITS, int MT, int RW>
+__global__ void __launch_bounds__(256)
+    mix_down_dot_kernel(const T *x, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, int64_t R, int64_t d,
+                        int64_t G, int64_t r, float eps, int64_t Tn, float *h, float *w_in, float *inv_out) {
+    constexpr bool F32 = std::is_same<T, float>::value;
+    // FP32: Q4 codes 0 .. 15 as they are
+    constexpr float EXTRA = F32 || BITS == 8 ? 0.f : 24.f, MID = BITS == 8 ? 128.f : F32 ? 0.f : 8.f;
+    __shared__ float part[kStreams][MT][RW], sqs[kStreams][MT];
+    const int lane = threadIdx.x % kWave, stream = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t K = kStreams * d, r0 = (int64_t)blockIdx.x * RW, t0 = (int64_t)blockIdx.y * MT;
+    const int nt = (int)(Tn - t0 < MT ? Tn - t0 : MT), nr = (int)(R - r0 < RW ? R - r0 : RW);
+    float acc[MT * RW], sq[MT];
+#pragma unroll
+    for (int i = 0; i < MT * RW; ++i) acc[i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) sq[i] = 0.f;
+    const uint32_t chunks = (uint32_t)(d / 8), k0 = (uint32_t)(stream * d), G32 = (uint32_t)G;
+    for (uint32_t c = lane; c < chunks; c += kWave) {
+        const uint32_t k = k0 + 8 * c;
+        // rows past the weight and tokens past the batch repeat the last one (their sums are not stored)
+        uint32_t w[RW][BITS / 4];
+        uint16_t ws[RW], wm[RW];
+#pragma unroll
+        for (int n = 0; n < RW; ++n) {
+            const int64_t row = r0 + (n < nr ? n : nr - 1);
+            const uint8_t *p = q + row * (K * BITS / 8) + k * BITS / 8;
+            if constexpr (BITS == 4) w[n][0] = *reinterpret_cast<const uint32_t *>(p);
+            else {
+                const uint2 u = *reinterpret_cast<const uint2 *>(p);
+                w[n][0] = u.x, w[n][1] = u.y;
+            }
+            ws[n] = scale[row * (K / G) + k / G32], wm[n] = minv[row * (K / G) + k / G32];
+        }
+        xt::Act8<T> xv[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) xv[t].load(x + (t0 + (t < nt ? t : nt - 1)) * K + k);
+        float sc[RW], mp[RW];
+#pragma unroll
+        for (int n = 0; n < RW; ++n) sc[n] = bf16_to_f32(ws[n]), mp[n] = fmaf(MID, sc[n], bf16_to_f32(wm[n]));
+        if constexpr (F32) {
+            float cf[RW][8];
+#pragma unroll
+            for (int n = 0; n < RW; ++n)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if constexpr (BITS == 4) cf[n][i] = (float)((w[n][0] >> (4 * i)) & 15u);
+                    else cf[n][i] = (float)(int8_t)(uint8_t)((w[n][i / 4] ^ 0x80808080u) >> (8 * (i % 4)));
+                }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const float v[8] = {xv[t].a.x, xv[t].a.y, xv[t].a.z, xv[t].a.w, xv[t].b.x, xv[t].b.y, xv[t].b.z, xv[t].b.w};
+                const float xs = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+                float s = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s = fmaf(v[i], v[i], s);
+                sq[t] += s;
+#pragma unroll
+                for (int n = 0; n < RW; ++n) {
+                    float dot = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) dot = fmaf(v[i], cf[n][i], dot);
+                    acc[t * RW + n] = fmaf(sc[n], dot, fmaf(mp[n], xs, acc[t * RW + n]));
+                }
+            }
+        } else {
+            Frag f[RW];
+#pragma unroll
+            for (int n = 0; n < RW; ++n) {
+                if constexpr (BITS == 4) {  // natural order: 16 + code
+                    const uint32_t e = ((w[n][0] << 3) & 0x78787878u) | 0x80808080u, o = ((w[n][0] >> 1) & 0x78787878u) | 0x80808080u;
+                    const uint32_t m0 = __builtin_amdgcn_perm(o, e, 0x05010400u), m1 = __builtin_amdgcn_perm(o, e, 0x07030602u);
+                    const uint32_t top = 0x41414141u;
+                    f[n] = Frag{{__builtin_amdgcn_perm(top, m0, 0x04010400u), __builtin_amdgcn_perm(top, m0, 0x04030402u),
+                                 __builtin_amdgcn_perm(top, m1, 0x04010400u), __builtin_amdgcn_perm(top, m1, 0x04030402u)}};
+                } else {
+                    auto sb = [](uint32_t v, int i) { return (float)(int8_t)(uint8_t)(v >> (8 * i)); };
+                    const uint32_t a = w[n][0] ^ 0x80808080u, b = w[n][1] ^ 0x80808080u;
+                    f[n] = Frag{{hi16_pair(sb(a, 0), sb(a, 1)), hi16_pair(sb(a, 2), sb(a, 3)), hi16_pair(sb(b, 0), sb(b, 1)),
+                                 hi16_pair(sb(b, 2), sb(b, 3))}};
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const uint32_t v[4] = {xv[t].a.x, xv[t].a.y, xv[t].a.z, xv[t].a.w};
+                float xs = 0.f, s = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xs = dot2(v[i], 0x3F803F80u, xs), s = dot2(v[i], v[i], s);
+                sq[t] += s;
+#pragma unroll
+                for (int n = 0; n < RW; ++n) {
+                    float dot = EXTRA != 0.f ? -EXTRA * xs : 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) dot = dot2(v[i], f[n].d[i], dot);
+                    acc[t * RW + n] = fmaf(sc[n], dot, fmaf(mp[n], xs, acc[t * RW + n]));
+                }
+            }
+        }
     }
+    const float a = wave_scatter_sum<MT * RW>(acc), b = wave_scatter_sum<MT>(sq);
+    if (lane % (kWave / (MT * RW)) == 0) (&part[stream][0][0])[lane / (kWave / (MT * RW))] = a;
+    if (lane % (kWave / MT) == 0) sqs[stream][lane / (kWave / MT)] = b;
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (blockIdx.x == 0 && i < nt * kStreams)
+        inv_out[t0 * kStreams + i] = 1.0f / sqrtf(sqs[i % kStreams][i / kStreams] / (float)d + eps);
+    const int t = i / RW, n = i % RW;
+    if (i >= MT * RW || t >= nt || n >= nr) return;
+    float z = 0.f;
+#pragma unroll
+    for (int s = 0; s < kStreams; ++s) z = fmaf(1.0f / sqrtf(sqs[s][t] / (float)d + eps), part[s][t][n], z);
+    z *= 0.25f;
+    if (r0 + n < r) h[(t0 + t) * r + r0 + n] = z / (1.0f + expf(-z));
+    else w_in[(t0 + t) * kStreams + (r0 + n - r)] = 2.0f / (1.0f + expf(-z));
 }
 
 // ================================================================================================ up: MFMA tiles
@@ -783,7 +1007,36 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
                 " rows are needed");
     STRIX_CHECK(std::isfinite(eps) && eps > 0.f, what, ": eps = ", eps, " (a finite positive value is needed)");
     const bool f32 = act == Act::F32;
-    if (T >= kDownTileMinTokens && d % dn::kK == 0) {  // matrix-core tiles
+    using std::integral_constant;
+    // which kernel, by what each is bound by (see kDownDotTokens)
+    const int64_t cus = device_cus();
+    auto split_blocks = [&](int tt, int rt) { return ((R + 16 * rt - 1) / (16 * rt)) * ((T + 16 * tt - 1) / (16 * tt)); };
+    const bool tiles = d % dn::kK == 0 && (f32 ? T >= kDownTileF32Tokens : split_blocks(2, 4) > cus);
+    const int variant = split_blocks(1, 1) <= cus ? 0 : split_blocks(1, 2) <= cus ? 1 : split_blocks(2, 2) <= cus ? 2 : 3;
+    bool done = false;
+    if (!f32 && !tiles && T > kDownDotTokens) {
+        auto go = [&](auto spc, auto ttc, auto rtc, auto nwc) {
+            constexpr int SP = decltype(spc)::value, TT = decltype(ttc)::value, RT = decltype(rtc)::value, NW = decltype(nwc)::value;
+            const uint32_t ng = down_split_groups<SP, NW>(d, w.G);
+            const size_t lds = down_split_lds<TT, RT, NW>(ng);
+            if (lds > kDownSplitLds) return;  // a stream too wide for the scales' LDS space: the lane dots take it
+            auto k = mix_down_split_kernel<BITS, SP, TT, RT, NW>;
+            allow_lds((const void *)k, lds);
+            k<<<(unsigned)split_blocks(TT, RT), NW * kWave, lds, stream>>>(static_cast<const uint16_t *>(x), w.q, w.scale,
+                                                                          w.minv, R, d, w.G, r, eps, T, h, w_in, inv, ng);
+            done = true;
+        };
+        auto by_variant = [&](auto spc) {
+            if (variant == 0) go(spc, integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 16>{});
+            else if (variant == 1) go(spc, integral_constant<int, 1>{}, integral_constant<int, 2>{}, integral_constant<int, 16>{});
+            else if (variant == 2) go(spc, integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+            else go(spc, integral_constant<int, 2>{}, integral_constant<int, 4>{}, integral_constant<int, 8>{});
+        };
+        if (w.G >= 64 && d % 64 == 0) by_variant(integral_constant<int, 64>{});
+        else by_variant(integral_constant<int, 32>{});
+    }
+    if (done) {
+    } else if (tiles) {  // matrix-core tiles, K staged by the block
         const int64_t nrb = (R + dn::kRows - 1) / dn::kRows, ntt = (T + dn::kTok - 1) / dn::kTok;
         const size_t lds = f32 ? down_tile_lds<BITS, true>() : down_tile_lds<BITS, false>();
         auto go = [&](auto tag, auto gtag) {
@@ -801,36 +1054,21 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
         };
         if (f32) by_g(float{});
         else by_g(uint16_t{});
-    } else {  // vector rows: up to 16 tokens the 4 waves split each row; more tokens share a row's code loads
-        const int mt = T == 1 ? 1 : T <= 2 ? 2 : T <= 4 ? 4 : 8;
-        // up to 16 tokens, 4 waves split each row's K (measured at d 2560, r 320: 16 tokens 29.4 -> 24.3 us, 5 tokens
-        // 21.3 -> 16.2); above, a wave a row
-        const int ks = T <= 16 ? 4 : 1;
-        const int rows_pb = 4 / ks;
-        const dim3 grid((unsigned)((R + rows_pb - 1) / rows_pb), (unsigned)((T + mt - 1) / mt));
-        auto go = [&](auto tag, auto mtag) {
-            using TT = decltype(tag);
-            constexpr int MT = decltype(mtag)::value;
-            if (T == 1)
-                mix_down_rows_kernel<TT, BITS, 1, 4><<<grid, 256, 0, stream>>>(
-                    static_cast<const TT *>(x), w.q, w.scale, w.minv, R, d, w.G, r, eps, T, h, w_in, inv);
-            else if (ks == 4)
-                mix_down_rows_kernel<TT, BITS, MT, 4><<<grid, 256, 0, stream>>>(
-                    static_cast<const TT *>(x), w.q, w.scale, w.minv, R, d, w.G, r, eps, T, h, w_in, inv);
-            else
-                mix_down_rows_kernel<TT, BITS, MT, 1><<<grid, 256, 0, stream>>>(
-                    static_cast<const TT *>(x), w.q, w.scale, w.minv, R, d, w.G, r, eps, T, h, w_in, inv);
+    } else {  // lane dots
+        auto go = [&](auto tag, auto mtc, auto rwc) {
+            using X = decltype(tag);
+            constexpr int MT = decltype(mtc)::value, RW = decltype(rwc)::value;
+            const dim3 grid((unsigned)((R + RW - 1) / RW), (unsigned)((T + MT - 1) / MT));
+            mix_down_dot_kernel<X, BITS, MT, RW><<<grid, 256, 0, stream>>>(static_cast<const X *>(x), w.q, w.scale, w.minv,
+                                                                           R, d, w.G, r, eps, T, h, w_in, inv);
         };
-        auto by_mt = [&](auto tag) {
-            switch (mt) {
-                case 1: go(tag, std::integral_constant<int, 1>{}); break;
-                case 2: go(tag, std::integral_constant<int, 2>{}); break;
-                case 4: go(tag, std::integral_constant<int, 4>{}); break;
-                default: go(tag, std::integral_constant<int, 8>{}); break;
-            }
+        auto by_t = [&](auto tag) {
+            if (T == 1) go(tag, integral_constant<int, 1>{}, integral_constant<int, 1>{});
+            else if (T == 2) go(tag, integral_constant<int, 2>{}, integral_constant<int, 2>{});
+            else go(tag, integral_constant<int, 4>{}, integral_constant<int, 2>{});
         };
-        if (f32) by_mt(float{});
-        else by_mt(uint16_t{});
+        if (f32) by_t(float{});
+        else by_t(uint16_t{});
     }
     STRIX_HIP_CHECK_LAUNCH(what, " Q", BITS, " ", act_str(act), " T=", T, " R=", R, " K=", w.K, " G=", w.G);
 }

@@ -117,3 +117,28 @@ def test_dense_tiles_and_gemm(bits, G, M, N, K):
     lin = moe.linear_q4 if bits == 4 else moe.linear_q8
     assert _rel64(lin(x, w, out_dtype=torch.float32), ref) < 1e-4  # FP32 sums; the GEMM's Q4 codes carry an offset of 128
     assert _rel64(lin(x, w), ref) < 2.0 ** -8  # one BF16 rounding
+
+
+# the down mix's kernels at the ends of their ranges: lane dots of 2 and 3 tokens and a row remainder, split-K tiles of
+# each size (blocks of 16 x 16, 16 x 32, 32 x 32, 32 x 64) with 64- and 32-code steps and streams of a half group, a
+# stream too wide for the split's LDS, FP32 lane dots
+@pytest.mark.parametrize("bits,G,act,T,d,r,inject", [
+    (4, 64, "bf16", 2, 160, 33, False), (8, 32, "bf16", 3, 96, 35, True), (4, 64, "bf16", 33, 160, 20, True),
+    (4, 128, "bf16", 49, 320, 64, False), (8, 64, "bf16", 257, 128, 320, True), (4, 32, "bf16", 400, 96, 320, True),
+    (4, 64, "bf16", 705, 128, 320, True), (8, 64, "bf16", 1500, 64, 320, False), (4, 32, "bf16", 40, 65536, 8, False),
+    (4, 64, "f32", 33, 160, 20, True), (8, 64, "f32", 439, 128, 9, False)])
+def test_mix_down_kernels(bits, G, act, T, d, r, inject):
+    from oracle import hc
+
+    say("mix down", bits, G, act, T, d, r, inject)
+    dt = torch.bfloat16 if act == "bf16" else torch.float32
+    x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, 4 * d)).astype(np.float32)).to(DEV).to(dt)
+    w = _weight(bits, r + (4 if inject else 0), 4 * d, G, 61)
+    h, w_in, inv = moe.hc_mix_down(x, w, r, inject, 1e-6)
+    rows = np.unique(np.concatenate([np.arange(min(T, 40)), np.arange(max(0, T - 40), T)]))
+    hr, wir, invr = hc.hc_mix_down(x.double().cpu().numpy()[rows], _w64(w), d, r, inject, 1e-6)
+    # exact products, FP32 sums of 4 d terms no larger than the result: a few 2^-24 sqrt(4 d)
+    assert _rel64(inv[rows], invr) < 2e-6
+    assert _rel64(h[rows], hr) < 1e-5
+    if inject:
+        assert _rel64(w_in[rows], wir) < 1e-5
