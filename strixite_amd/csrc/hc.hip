@@ -170,8 +170,11 @@ template <int BITS, bool F32> struct Stage {
 };
 }  // namespace dn
 
-template <typename T, int BITS, int G>
-__global__ void __launch_bounds__(dn::kThreads)
+// KH: the block's K in halves (streams 0, 1 and 2, 3), each a group of 4 waves with stage buffers of its own; their totals
+// meet at the end. BF16 takes two (one group alone leaves each SIMD one wave, and a stage's staging, barrier and math
+// follow one another: 104 -> 81 us at 2000 tokens, Q4 g64); the stages of FP32 and of Q8 fill the LDS with one.
+template <typename T, int BITS, int G, int KH>
+__global__ void __launch_bounds__(dn::kThreads * KH)
     mix_down_tile_kernel(const T *x, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, int64_t R,
                          int64_t d, int64_t r, float eps, int64_t Tn, float *h, float *w_in, float *inv_out) {
     using namespace dn;
@@ -179,16 +182,20 @@ __global__ void __launch_bounds__(dn::kThreads)
     using S = Stage<BITS, F32>;
     constexpr int GPS = kK / G;  // groups a stage
     constexpr int WDW = wdw<BITS>();
-    extern __shared__ uint32_t lds[];  // two stages
-    __shared__ float invs[2][kTok];    // by stream parity
+    extern __shared__ uint32_t lds_all[];   // two stages a K half
+    __shared__ float invs_all[KH][2][kTok];  // by stream parity
+    const int half = KH > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / dn::kThreads) : 0;
+    uint32_t *lds = lds_all + half * 2 * S::SIZE;
+    float(&invs)[2][kTok] = invs_all[half];
 
     const int64_t K = kStreams * d;
-    const uint32_t stages = (uint32_t)(K / kK), sps = (uint32_t)(d / kK);  // stages, stages a stream (32-bit: cheap
-                                                                           // division in the loop)
+    const uint32_t stages = (uint32_t)(K / kK) / KH, sps = (uint32_t)(d / kK);  // stages, stages a stream (32-bit: cheap
+                                                                                // division in the loop)
+    const uint32_t st0 = half * stages;  // the half's first stage
     const uint32_t nrb = (uint32_t)((R + kRows - 1) / kRows);
     const uint32_t L = xcd_block(blockIdx.x, gridDim.x);
     const int64_t t0 = (int64_t)(L / nrb) * kTok, rb = (int64_t)(L % nrb) * kRows;
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, n = lane % 16, qd = lane / 16;
+    const int tid = threadIdx.x % dn::kThreads, lane = tid % kWave, wave = tid / kWave, n = lane % 16, qd = lane / 16;
 
     // ---- staging (all threads): registers for the next stage
     constexpr int WP = BITS == 4 ? 3 : 6;  // 16-byte weight pieces a thread a stage
@@ -200,7 +207,7 @@ __global__ void __launch_bounds__(dn::kThreads)
     const int tt = tid / 8, seg = tid % 8;  // the thread's token and 16-k segment of the activation stage
     const int64_t xrow = (t0 + tt < Tn ? t0 + tt : Tn - 1) * K;
     auto load_stage = [&](uint32_t st, Regs &rg) {
-        const int64_t kb = (int64_t)st * kK;
+        const int64_t kb = (int64_t)(st0 + st) * kK;
 #pragma unroll
         for (int i = 0; i < WP; ++i) {
             const int p = tid + dn::kThreads * i;
@@ -285,7 +292,7 @@ __global__ void __launch_bounds__(dn::kThreads)
         if ((st + 1) % sps == 0) {
 #pragma unroll
             for (int o = 1; o < 8; o <<= 1) sq += __shfl_xor(sq, o, kWave);
-            const uint32_t s = st / sps;
+            const uint32_t s = (st0 + st) / sps;
             const float iv = 1.0f / sqrtf(sq / (float)d + eps);
             if (seg == 0) {
                 invs[s & 1][tt] = iv;
@@ -373,7 +380,7 @@ __global__ void __launch_bounds__(dn::kThreads)
                 P[nt][m] = mfma_f32x4(__uint_as_float(sb[S::XS + qd * kTok + 16 * m + n]), mp, P[nt][m]);
         }
         if ((st + 1) % sps == 0) {  // the stream ends: A += inv_s P
-            const int par = (int)((st / sps) & 1);
+            const int par = (int)(((st0 + st) / sps) & 1);
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 const float4 iv = *reinterpret_cast<const float4 *>(&invs[par][16 * m + 4 * qd]);
@@ -405,6 +412,20 @@ __global__ void __launch_bounds__(dn::kThreads)
         if (st + 1 < stages) step(st + 1, rgs[1], rgs[0]);
     }
 
+    if constexpr (KH > 1) {  // the second half's totals to the first (the stages are read: their space takes them)
+        float4v *tot = reinterpret_cast<float4v *>(lds_all);
+        if (half == 1)
+#pragma unroll
+            for (int nt = 0; nt < kTilesPW; ++nt)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) tot[(2 * nt + m) * dn::kThreads + tid] = A[nt][m];
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int nt = 0; nt < kTilesPW; ++nt)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) A[nt][m] += tot[(2 * nt + m) * dn::kThreads + tid];
+    }
     // ---- epilogue: z = a / 4 -> h (rows < r) or the injection gates (rows r .. r + 3)
 #pragma unroll
     for (int nt = 0; nt < kTilesPW; ++nt) {
@@ -423,7 +444,10 @@ __global__ void __launch_bounds__(dn::kThreads)
     }
 }
 
-template <int BITS, bool F32> constexpr size_t down_tile_lds() { return (size_t)2 * dn::Stage<BITS, F32>::SIZE * 4; }
+template <int BITS, bool F32> constexpr int down_tile_halves() { return !F32 && BITS == 4 ? 2 : 1; }
+template <int BITS, bool F32> constexpr size_t down_tile_lds() {
+    return (size_t)down_tile_halves<BITS, F32>() * 2 * dn::Stage<BITS, F32>::SIZE * 4;
+}
 
 // ================================================================================================ down: split-K tiles
 // A block takes TT 16-token tiles against RT tiles of 16 weight rows (BF16 streams), and its NW waves split K: NW / 4 to
@@ -765,10 +789,18 @@ __global__ void __launch_bounds__(256)
 }
 
 // ================================================================================================ up: MFMA tiles
+// 1 / (1 + e^-a). FAST (u in BF16, rounded at 2^-9): the hardware's FP32 exponential and reciprocal, a few 2^-24 off (4
+// instructions for ~40, and there are four gates an output: 2000 tokens at d 2560, r 320 went 90 -> 81 us; u's error against 64 bits unchanged)
+template <bool FAST> __device__ __forceinline__ float gate_of(float a) {
+    if constexpr (FAST) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896340736f));
+    else return 1.0f / (1.0f + expf(-a));
+}
+
 // WAVES column tiles of 16 positions j a block (a wave each), MT 16-token tiles; LDS: h as bf16 hi / mid / lo [16 MT][r + 8]
 // in the paired k order, then its group sums [r / G][16 MT] (FP32)
-template <typename T, int BITS, int MT, int WAVES>
-__global__ void __launch_bounds__(WAVES * kWave)
+// TWO: registers held to what lets two blocks share a CU, for grids of more blocks than CUs
+template <typename T, int BITS, int MT, int WAVES, bool TWO>
+__global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2)))
     mix_up_tile_kernel(const float *h, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, const T *x,
                        const float *norm_w, const float *inv, int64_t d, int64_t r, int64_t G, int64_t Tn, T *u) {
     constexpr int NTHR = WAVES * kWave, TOK = 16 * MT, CB = kChunk * BITS / 8;
@@ -870,7 +902,9 @@ __global__ void __launch_bounds__(WAVES * kWave)
     if constexpr (kHoist) load_epilogue();
 
     // a ring of kAhead chunks in flight: chunk c computes from slot c % kAhead, then that slot loads chunk c + kAhead
-    constexpr int kAhead = 4;  // (8 for the 16-token tiles measured slower: 15.1 against 13.2 us at 1 token)
+    // (8 for the 16-token tiles measured slower: 15.1 against 13.2 us at 1 token; two blocks a CU with 4 ahead spill: 99
+    // us at 2000 tokens, with 2 ahead 72, one block a CU with 4 ahead 81)
+    constexpr int kAhead = TWO ? 2 : 4;
     Ahead ring[kAhead];
 #pragma unroll
     for (int p = 0; p < kAhead; ++p) ld_chunk(p, ring[p]);
@@ -944,7 +978,7 @@ __global__ void __launch_bounds__(WAVES * kWave)
             float sum = 0.f;
 #pragma unroll
             for (int s = 0; s < kStreams; ++s) {
-                const float gate = 1.0f / (1.0f + expf(-acc[s][m][i]));
+                const float gate = gate_of<std::is_same<T, uint16_t>::value>(acc[s][m][i]);
                 sum += gate * (xe[m][i][s] * ie[m][i][s] * nwv[s]);
             }
             st_act(u, t * d + j, sum * 0.25f);
@@ -1042,9 +1076,10 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
         auto go = [&](auto tag, auto gtag) {
             using TT = decltype(tag);
             constexpr int GG = decltype(gtag)::value;
-            auto k = mix_down_tile_kernel<TT, BITS, GG>;
+            constexpr int KH = down_tile_halves<BITS, std::is_same<TT, float>::value>();
+            auto k = mix_down_tile_kernel<TT, BITS, GG, KH>;
             allow_lds((const void *)k, lds);
-            k<<<(unsigned)(nrb * ntt), dn::kThreads, lds, stream>>>(static_cast<const TT *>(x), w.q, w.scale, w.minv,
+            k<<<(unsigned)(nrb * ntt), dn::kThreads * KH, lds, stream>>>(static_cast<const TT *>(x), w.q, w.scale, w.minv,
                                                                     R, d, r, eps, T, h, w_in, inv);
         };
         auto by_g = [&](auto tag) {
@@ -1091,10 +1126,12 @@ void run_mix_up(const float *h, const Weights &w, const void *x, const float *no
     const int MT = small ? 1 : 2, WAVES = small ? 4 : 8;
     const size_t lds = up_tile_lds(MT, w.K, w.G);
     const int64_t njb = (d / 16 + WAVES - 1) / WAVES, ntt = (T + 16 * MT - 1) / (16 * MT);
+    // (Q8 codes beside FP32 streams spill at two blocks a CU: 105 against 103 us at 2000 tokens)
+    const bool two = !small && njb * ntt > device_cus() && !(BITS == 8 && act == Act::F32);
     auto go = [&](auto tag, auto mtag) {
         using TT = decltype(tag);
         constexpr int M = decltype(mtag)::value, WV = M == 1 ? 4 : 8;
-        auto k = mix_up_tile_kernel<TT, BITS, M, WV>;
+        auto k = M == 2 && two ? mix_up_tile_kernel<TT, BITS, M, WV, M == 2> : mix_up_tile_kernel<TT, BITS, M, WV, false>;
         allow_lds((const void *)k, lds);
         k<<<(unsigned)(njb * ntt), WV * kWave, lds, stream>>>(h, w.q, w.scale, w.minv, static_cast<const TT *>(x),
                                                               norm_w, inv, d, w.K, w.G, T, static_cast<TT *>(u));
