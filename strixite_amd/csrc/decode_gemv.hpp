@@ -570,10 +570,15 @@ __global__ void __launch_bounds__((W + 1) * kWave) decode_gate_up_lds_kernel(Dec
 namespace gdn {
 constexpr int kDnStages = 3;                                    // per-wave ring
 template <int KS> constexpr int pos_u4() { return 4 * KS * 17; }  // codes + 16 KS dwords of scales and mins
-// waves a block: 4 (three blocks, 12 waves a CU) at KS = 4; 2 (five blocks, 10 waves) at KS = 5, whose positions are
-// 5,440 bytes (4 waves a block would leave room for two blocks, 8 waves)
-template <int KS> constexpr int waves() { return KS <= 4 ? 4 : 2; }
-template <int KS> constexpr int blocks_per_cu() { return 163840 / (waves<KS>() * kDnStages * pos_u4<KS>() * 16); }
+// waves a block and the blocks that run on a CU together: at KS = 4 three blocks of four (12 waves, by LDS and registers);
+// at KS = 5 two of four: the h rows' registers leave a SIMD two waves. (The waves are dealt their units up front, so
+// a block that waits for another to end makes a second round: with five blocks of two, the LDS's worth, the down of 11
+// tokens at H 2560, I 640 took 26.6 us, so 21.1; held to three waves a SIMD it spills, whose scratch loads the ring's
+// waits then count: 66.)
+template <int KS> constexpr int waves() { return 4; }
+template <int KS> constexpr int blocks_per_cu() {
+    return std::min(KS <= 4 ? 3 : 2, 163840 / (waves<KS>() * kDnStages * pos_u4<KS>() * 16));
+}
 template <int KS> __device__ __forceinline__ int swz(int r) {
     return KS % 2 ? (r >> 2) & 3 : KS % 4 ? (r >> 1) & 7 : r;
 }
@@ -737,6 +742,10 @@ constexpr int kDecGuWaves = 8, kDecGuAhead = 2;  // waves a block; units of load
 constexpr int kDecMaxTiles = 1024;               // M <= 16 tokens x A <= 64 slots
 
 inline bool gate_up_lds_fits(const GemmArgs &ga);
+// the LDS-ring kernels read the scales and mins as dwords straight into LDS
+inline bool scales_dword_aligned(const GemmArgs &ga) {
+    return reinterpret_cast<uintptr_t>(ga.scale) % 4 == 0 && reinterpret_cast<uintptr_t>(ga.minv) % 4 == 0;
+}
 // the LDS-ring down kernel's shapes: Q4 g128, K = 512 or 640 (the benchmark's and the served model's I); it deals its
 // waves to tiles, so every tile needs a wave. Measured on MI355X at H 2560, I 640, 513 experts, 11 slots a token, against
 // the register-fed stream kernels (this and the gate_up at W = 10 together): a layer of 11 tokens 116 -> 86 us, of 1
@@ -744,7 +753,7 @@ inline bool gate_up_lds_fits(const GemmArgs &ga);
 inline bool down_lds_fits(const GemmArgs &ga) {
     const int64_t tiles = std::min(ga.S, ga.S / 16 + ga.E + 2);
     auto waves = [](auto ks) { return gdn::blocks_per_cu<decltype(ks)::value>() * gdn::waves<decltype(ks)::value>(); };
-    if (ga.G != dec::kSpan || ga.N % 16 != 0) return false;
+    if (ga.G != dec::kSpan || ga.N % 16 != 0 || !scales_dword_aligned(ga)) return false;
     if (ga.K == 4 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 4>{}) * device_cus();
     if (ga.K == 5 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 5>{}) * device_cus();
     return false;
@@ -792,7 +801,7 @@ void launch_decode_gate_up_lds(const DecodeArgs &d, SharedJob s, hipStream_t str
 inline bool gate_up_lds_fits(const GemmArgs &ga) {
     const int64_t tiles_bound = std::min(ga.S, ga.S / 16 + ga.E + 2);
     const int64_t upt = ga.N / 32, most_units = (tiles_bound * upt + device_cus() - 1) / device_cus();
-    return ga.G == dec::kSpan && ga.K % 256 == 0 && (ga.K / 256 == 8 || ga.K / 256 == 10 || ga.K / 256 == 12) && (ga.N / 2) % 16 == 0 &&
+    return ga.G == dec::kSpan && scales_dword_aligned(ga) && ga.K % 256 == 0 && (ga.K / 256 == 8 || ga.K / 256 == 10 || ga.K / 256 == 12) && (ga.N / 2) % 16 == 0 &&
            (most_units + upt - 1) / upt + 1 <= gul::kGuMaxBlockTiles && tiles_bound <= kDecMaxTilesL;
 }
 
