@@ -788,7 +788,8 @@ __global__ void __launch_bounds__(1024)
                              GemmArgs sa, int spp, int parts, float *part, int64_t units) {
     extern __shared__ int lds[];
     if (blockIdx.x == 0) {
-        route::topk_route_small_body<NV, false>(logits, ld, M, E, k, ids, coef, L, nbits, ws, err_router, err_route, lds);
+        if (M == 1) route::topk_route_one_body<NV, false>(logits, E, k, ids, coef, L, ws, err_router, err_route, lds);
+        else route::topk_route_small_body<NV, false>(logits, ld, M, E, k, ids, coef, L, nbits, ws, err_router, err_route, lds);
         return;
     }
     // 4 units a block (its other waves exit): the units spread over many CUs

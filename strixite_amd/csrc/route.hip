@@ -25,6 +25,11 @@ __global__ void __launch_bounds__(1024) route_small_kernel(const int32_t *ids, L
     pack_small_body<1, false>(nullptr, 0, ids, 0, (int)L.E, 0, nullptr, nullptr, L, nbits, ws, nullptr, err, lds);
 }
 
+// One block up to kSmallSlots slots (and its LDS), four launches beyond: measured on MI355X (512 experts, us) 9.5 / 17.9
+// at 1100 slots, 14.0 / 19.7 at 4092, 15.7 / 19.7 at 5120, 21.4 / 20.1 at 8140
+constexpr int64_t kSmallSlots = 6144;
+constexpr size_t kSmallLds = 160 * 1024;
+
 // ---- larger S: range histograms, one scan block, placement ------------------------------------------------------------
 // A histogram block takes a range of kRangeChunks chunks, a wave each: the chunk counts meet in LDS, and the block
 // writes each chunk's position within the range and the range's bucket counts. The scan block then has only the
@@ -204,6 +209,14 @@ __global__ void __launch_bounds__(1024)
                               shared_slot);
 }
 
+template <int NV>
+__global__ void __launch_bounds__(256)
+    topk_route_one_kernel(const float *logits, int E, int k, int32_t *ids_out, float *coef_out, Layout L, int32_t *ws,
+                          uint32_t *err_router, uint32_t *err_route, bool shared_slot) {
+    __shared__ __attribute__((aligned(8))) int lds[2 * kWave + 2 * topk::kCandScratch];
+    topk_route_one_body<NV>(logits, E, k, ids_out, coef_out, L, ws, err_router, err_route, lds, shared_slot);
+}
+
 
 }  // namespace
 
@@ -229,8 +242,14 @@ void moe_group_routes(const int32_t *ids, int64_t M, int64_t A, int64_t E, void 
     int nbits = 0;
     while ((1ll << nbits) <= E) ++nbits;  // buckets 0..E
     int32_t *w = static_cast<int32_t *>(ws);
-    if (L.S <= kFusedSlots) {
-        route_small_kernel<<<1, 1024, topk_route_small_lds(L), stream>>>(ids, L, nbits, w, err);
+    const size_t small_lds = topk_route_small_lds(L, false);
+    if (L.S <= kSmallSlots && small_lds <= kSmallLds) {
+        if (small_lds > 64 * 1024) {
+            static const hipError_t granted = hipFuncSetAttribute(reinterpret_cast<const void *>(route_small_kernel),
+                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds);
+            STRIX_HIP_CHECK(granted, fn, ": LDS of ", kSmallLds, " bytes");
+        }
+        route_small_kernel<<<1, 1024, small_lds, stream>>>(ids, L, nbits, w, err);
     } else {
         const unsigned blocks = (unsigned)((L.nch + kWavesPerBlock - 1) / kWavesPerBlock);
         const size_t lds = (size_t)kWavesPerBlock * (E + 1) * 4;
@@ -261,6 +280,11 @@ void moe_topk_group_routes_small(const float *logits, int64_t ld, int64_t M, int
     const size_t lds = route::topk_route_small_lds(L);
     const int nv = E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : E <= 512 ? 8 : 16;
     auto go = [&](auto nvc) {
+        if (M == 1) {
+            topk_route_one_kernel<decltype(nvc)::value><<<1, 256, 0, stream>>>(
+                logits, (int)Es, (int)k, ids, coef, L, static_cast<int32_t *>(ws), err_router, err_route, shared_slot);
+            return;
+        }
         topk_route_small_kernel<decltype(nvc)::value><<<1, 1024, lds, stream>>>(
             logits, ld, (int)M, (int)Es, (int)k, ids, coef, L, nbits, static_cast<int32_t *>(ws), err_router, err_route,
             shared_slot);

@@ -247,9 +247,14 @@ __device__ inline void report_bad(const int32_t *ids, int first_bad, uint32_t *e
 // barrier after a global store or before a dependent global load costs a memory round trip, and a one-block launch
 // is a chain of them otherwise.
 // Phase A: TOPK - wave w takes tokens w, w + 16, ...: top-k of the logits into LDS; else the ids are read into LDS.
-// B: wave w takes slots [64 w, 64 w + 64): histogram. C: block scan of the bucket counts. D: stable placement.
+// B: wave w takes slots [c w, c w + c), c = small_chunk: histogram. C: block scan of the bucket counts. D: stable placement.
 // E: the stores. The workspace layout and contents are those of moe_group_routes.
-constexpr int kFusedSlots = 1024;
+constexpr int kFusedSlots = 1024;  // the one-launch top-k + packing
+// slots a wave of the one-block packing takes (whole 64-slot steps)
+__host__ __device__ inline int small_chunk(int64_t S) {
+    return (int)((S + kSmallWaves * kWave - 1) / (kSmallWaves * kWave)) * kWave;
+}
+__host__ __device__ inline int small_cap(int64_t S) { return kSmallWaves * small_chunk(S); }
 
 // TOPK with shared_slot: each token's slot k is the shared expert (id E_top, coefficient sigmoid(its gate logit at
 // column E_top of the logits); a non-finite one is bad index E_top, strixite kernels/moe_router.hip:108-111), and the
@@ -263,10 +268,11 @@ __device__ inline void pack_small_body(const float *logits, int64_t ld, const in
     const int S = (int)L.S, nb = E + 1, wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, t = threadIdx.x;
     const int Etop = shared_slot ? E - 1 : E, A = k + (shared_slot ? 1 : 0);
     const int nthr = (int)blockDim.x;
+    const int chunk = small_chunk(S), cap = small_cap(S);
     int *sids = lds;                          // [S] ids by slot
-    float *scoef = reinterpret_cast<float *>(sids + kFusedSlots);  // [S] coefficients by slot (TOPK)
-    int *sl = sids + 2 * kFusedSlots;         // [S] slots by position
-    int *cnt = sl + kFusedSlots;              // [16][E + 1] wave counts, then cursors
+    float *scoef = reinterpret_cast<float *>(sids + cap);  // [S] coefficients by slot (TOPK)
+    int *sl = sids + (TOPK ? 2 : 1) * cap;    // [S] slots by position
+    int *cnt = sl + cap;                      // [16][E + 1] wave counts, then cursors
     int *bstart = cnt + kSmallWaves * nb;     // [E + 1] bucket start
     int *btile = bstart + nb;                 // [E + 1] bucket's first 16-slot tile
     int *bcount = btile + nb;                 // [E + 1]
@@ -276,9 +282,9 @@ __device__ inline void pack_small_body(const float *logits, int64_t ld, const in
     int *bad = wsum + scan_lds_ints(7);       // [1]
     // [16][kCandScratch] the waves' top-k candidates (8-byte aligned)
     uint2 *cand = reinterpret_cast<uint2 *>(
-        lds + ((3 * kFusedSlots + kSmallWaves * nb + 4 * nb + L.T16 + scan_lds_ints(7) + 1 + 1) & ~1));
-    // only the waves that hold slots (chunks of 64) count: their counters are the only ones cleared and summed
-    const int nw = (S + kWave - 1) / kWave;
+        lds + ((3 * cap + kSmallWaves * nb + 4 * nb + L.T16 + scan_lds_ints(7) + 1 + 1) & ~1));
+    // only the waves that hold slots count: their counters are the only ones cleared and summed
+    const int nw = (S + chunk - 1) / chunk;
     for (int i = t; i < nw * nb; i += nthr) cnt[i] = 0;
     if (t == 0) *bad = INT_MAX;
     // A
@@ -308,7 +314,7 @@ __device__ inline void pack_small_body(const float *logits, int64_t ld, const in
     }
     __syncthreads();
     // B
-    const int s0 = wave * kWave, s1 = min(s0 + kWave, S);
+    const int s0 = wave * chunk, s1 = min(s0 + chunk, S);
     if (s0 < S) {
         const int fb = chunk_hist(sids, s0, s1, E, nbits, cnt + wave * nb);
         if (lane == 0 && fb != INT_MAX) atomicMin(bad, fb);
@@ -379,11 +385,80 @@ __device__ inline void topk_route_small_body(const float *logits, int64_t ld, in
                               lds, shared_slot);
 }
 
-// LDS bytes pack_small_body needs
-inline size_t topk_route_small_lds(const Layout &L) {
-    const size_t ints = ((size_t)3 * kFusedSlots + (size_t)kSmallWaves * (L.E + 1) + 4 * (size_t)(L.E + 1) +
+// One token (M = 1): its picks are distinct experts, so every bucket holds one slot and a slot's place is its expert's
+// rank among the picks - no histogram, scan or placement. Wave 0 takes the top-k; then every thread counts the picks
+// below its experts. The workspace contents are pack_small_body's. lds: 2 waves of ints, then the top-k's candidates.
+// Measured on MI355X: 7.5 -> 4.4 us at 64 experts, 8.2 -> 6.1 at 512.
+template <int NV, bool PAIRS = true>
+__device__ inline void topk_route_one_body(const float *logits, int E, int k, int32_t *ids_out, float *coef_out, Layout L,
+                                           int32_t *ws, uint32_t *err_router, uint32_t *err_route, int *lds,
+                                           bool shared_slot = false) {
+    const int Etop = shared_slot ? E - 1 : E, A = k + (shared_slot ? 1 : 0), t = threadIdx.x, lane = t % kWave;
+    int *sb = lds;                                             // [A] the slots' buckets
+    uint2 *cand = reinterpret_cast<uint2 *>(lds + 2 * kWave);  // [kCandScratch] the top-k candidates
+    if (t < kWave) {
+        int id;
+        float cf;
+        const float gl = shared_slot ? logits[Etop] : 0.f;
+        int rb = topk::wave_topk<float, NV>(logits, Etop, k, id, cf, cand);
+        if (shared_slot && !isfinite(gl) && Etop < rb) rb = Etop;
+        if (shared_slot && lane == k) id = Etop, cf = 1.0f / (1.0f + expf(-gl));
+        if (rb != INT_MAX) {
+            if (lane == 0 && atomicCAS(&err_router[0], 0u, 1u) == 0u) err_router[1] = 0u, err_router[2] = (uint32_t)rb;
+            id = -1, cf = dev::qnan();
+        }
+        if (lane < A) {
+            sb[lane] = bucket_of(id, E);
+            ids_out[lane] = id, coef_out[lane] = cf;
+        }
+    }
+    __syncthreads();
+    const bool bad = sb[0] == E;  // a non-finite logit: every slot is invalid, one bucket E of A slots
+    for (int e = t; e <= E + 1; e += (int)blockDim.x) {
+        int c = 0;
+        for (int a = 0; a < A; ++a) c += sb[a] < e;
+        ws[L.offsets() + e] = c;
+    }
+    const int tiles = bad ? (A + kTileRows - 1) / kTileRows : A;
+    if (t < A) {
+        int rank = 0;
+        for (int a = 0; a < A; ++a) rank += sb[a] < sb[t] || (sb[a] == sb[t] && a < t);
+        ws[L.slots() + rank] = t;
+        if (!bad) {
+            const int4 rec = make_int4(sb[t], rank, 1, 0);
+            *reinterpret_cast<int4 *>(ws + L.t64_rec() + 4 * rank) = rec;
+            if constexpr (PAIRS) *reinterpret_cast<int4 *>(ws + L.pair_rec() + 4 * rank) = rec;
+        } else if (t == 0) {
+            const int4 rec = make_int4(E, 0, A, 0);
+            *reinterpret_cast<int4 *>(ws + L.t64_rec()) = rec;
+            if constexpr (PAIRS) *reinterpret_cast<int4 *>(ws + L.pair_rec()) = rec;
+        }
+    }
+    // 16-slot tile records {bucket, first, rows, 0, slot[16]}: a thread per (slot, entry)
+    for (int i = t; i < (bad ? tiles : A) * kTileRows; i += (int)blockDim.x) {
+        const int a = i / kTileRows, j = i % kTileRows;
+        int tile = a, b = E, first = a * kTileRows, rows = A - first < kTileRows ? A - first : kTileRows, slot = first + j;
+        if (!bad) {
+            b = sb[a], rows = 1, slot = a, tile = 0;
+            for (int o = 0; o < A; ++o) tile += sb[o] < b;
+            first = tile;
+        }
+        int32_t *rec = ws + L.t16_rec() + kRec16 * tile;
+        if (j == 0) *reinterpret_cast<int4 *>(rec) = make_int4(b, first, rows, 0);
+        rec[4 + j] = j < rows ? slot : -1;
+    }
+    if (t == 0) {
+        ws[0] = tiles, ws[1] = A, ws[2] = (int32_t)L.E, ws[3] = bad ? 1 : A;
+        ws[L.npairs()] = PAIRS ? (bad ? 1 : A) : 0;
+        if (bad && atomicCAS(&err_route[0], 0u, 1u) == 0u) err_route[1] = 0xFFFFFFFFu, err_route[2] = 0u;
+    }
+}
+
+// LDS bytes pack_small_body needs (topk: with the top-k's coefficients and candidates)
+inline size_t topk_route_small_lds(const Layout &L, bool topk = true) {
+    const size_t ints = ((size_t)(topk ? 3 : 2) * small_cap(L.S) + (size_t)kSmallWaves * (L.E + 1) + 4 * (size_t)(L.E + 1) +
                          (size_t)L.T16 + scan_lds_ints(7) + 1 + 1) & ~(size_t)1;
-    return ints * 4 + (size_t)kSmallWaves * topk::kCandScratch * 8;  // + the top-k candidates
+    return ints * 4 + (topk ? (size_t)kSmallWaves * topk::kCandScratch * 8 : 0);  // + the top-k candidates
 }
 // ballot bits a bucket index 0..E takes
 inline int bucket_bits(int64_t E) {

@@ -275,13 +275,14 @@ void launch_router_rows(const uint16_t *x, const uint16_t *w, TY *y, int64_t M, 
         if (vec) router_rows_kernel<TY, MR, true><<<grid, block, 0, stream>>>(x, w, y, M, N, K, TG);
         else router_rows_kernel<TY, MR, false><<<grid, block, 0, stream>>>(x, w, y, M, N, K, TG);
     };
-    if (M <= 64 && vec && K % 512 == 0 && (K / 512 == 4 || K / 512 == 6 || K / 512 == 8)) {
+    if (M <= 64 && vec && K % 512 == 0 && (K / 512 == 4 || K / 512 == 5 || K / 512 == 6 || K / 512 == 8)) {
         // 4 tokens x 1 row a wave (one row a wave keeps enough waves in flight; measured on MI355X at M 16, N 513,
         // K 3072: 4 x 1 5.1 us, 4 x 2 6.0, 4 x 4 8.9, the per-row form with loads in order 8.3)
         constexpr int TT = 4, TE = 1;
         const int64_t per_block = TE * (kThreads / kWave);
         dim3 grid((unsigned)((N + per_block - 1) / per_block), (unsigned)((M + TT - 1) / TT)), block(kThreads);
         if (K / 512 == 4) router_small_kernel<TY, TT, TE, 4><<<grid, block, 0, stream>>>(x, w, y, M, N, K);
+        else if (K / 512 == 5) router_small_kernel<TY, TT, TE, 5><<<grid, block, 0, stream>>>(x, w, y, M, N, K);
         else if (K / 512 == 6) router_small_kernel<TY, TT, TE, 6><<<grid, block, 0, stream>>>(x, w, y, M, N, K);
         else router_small_kernel<TY, TT, TE, 8><<<grid, block, 0, stream>>>(x, w, y, M, N, K);
     } else if (M >= 256 && vec) {

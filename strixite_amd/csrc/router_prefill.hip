@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(kThreads) router_norms_kernel(const uint16_t *
 namespace {
 bool prefill_shape_fits(const void *x, const uint16_t *w, int64_t H, int64_t E, int64_t k) {
     const int64_t nch = H / 512;
-    return H % 512 == 0 && (nch == 2 || nch == 4 || nch == 6 || nch == 8) && E <= 1024 && k <= 32 && k <= E &&
+    return H % 512 == 0 && (nch == 2 || nch == 4 || nch == 5 || nch == 6 || nch == 8) && E <= 1024 && k <= 32 && k <= E &&
            reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
 }
 }  // namespace
@@ -378,6 +378,7 @@ void moe_router_prefill_select(const void *x, const uint16_t *w, const float *bi
     auto by_nch = [&](auto nvc) {
         switch (nch) {
             case 4: go(nvc, std::integral_constant<int, 4>{}); break;
+            case 5: go(nvc, std::integral_constant<int, 5>{}); break;
             case 6: go(nvc, std::integral_constant<int, 6>{}); break;
             case 8: go(nvc, std::integral_constant<int, 8>{}); break;
             default: go(nvc, std::integral_constant<int, 2>{}); break;

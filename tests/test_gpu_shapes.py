@@ -142,3 +142,39 @@ def test_mix_down_kernels(bits, G, act, T, d, r, inject):
     assert _rel64(h[rows], hr) < 1e-5
     if inject:
         assert _rel64(w_in[rows], wir) < 1e-5
+
+
+# the one-block packing past 1024 slots: around its waves' whole steps, its largest, and the sizes beyond
+@pytest.mark.parametrize("M,A,E", [(103, 10, 512), (205, 5, 64), (373, 11, 513), (600, 10, 1023), (6144, 1, 7),
+                                   (6145, 1, 7)])
+def test_group_routes_one_block_sizes(M, A, E):
+    say("packing", M, A, E)
+    rng = np.random.default_rng(M)
+    ids = rng.integers(0, E, (M, A)).astype(np.int32)
+    ids[M // 3, 0], ids[M - 1, A - 1] = -1, E
+    ws, err = moe.moe_group_routes(torch.from_numpy(ids).to(DEV), E)
+    t = moe.route_tables(ws, M, A, E)
+    b = np.where((ids < 0) | (ids >= E), E, ids).ravel()
+    counts = np.bincount(b, minlength=E + 1)
+    assert np.array_equal(t["offsets"].cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+    assert np.array_equal(t["slots"].cpu().numpy(), np.argsort(b, kind="stable"))
+    assert int(t["n_tiles"]) == int(((counts + 15) // 16).sum())
+    assert err.cpu().numpy().tolist() == [1, -1, M // 3 * A]
+
+
+@pytest.mark.parametrize("shared,bits,H,I,E,k", [(True, 4, 512, 256, 32, 4), ("stacked", 4, 2560, 640, 24, 10),
+                                                 (False, 8, 512, 128, 64, 8)])
+def test_one_token_layer_matches_two(shared, bits, H, I, E, k):
+    say("one token", shared, bits, H, I, E, k)
+    layer = moe.MoeLayer.synth(H, E, k, I, seed=7, routed_bits=bits, shared=shared)
+    x = moe.synth_bf16_normal(7, "x", 0, (2, H), 1.0)
+    one, two = layer.forward(x[:1].contiguous()), layer.forward(x)
+    assert torch.equal(one["ids"], two["ids"][:1]) and torch.equal(one["coef"], two["coef"][:1])
+    y1, y2 = one["y"].double().cpu().numpy(), two["y"][:1].double().cpu().numpy()
+    assert np.abs(y1 - y2).max() <= 2.0 ** -7 * np.abs(y2).max()  # one BF16 rounding of each
+    # a non-finite logit: invalid ids, NaN rows, both error words
+    lg = torch.zeros((1, E + (1 if shared else 0)), device=DEV)
+    lg[0, E // 2] = float("inf")
+    bad = layer.forward(x[:1].contiguous(), logits_in=lg)
+    assert (bad["ids"] == -1).all() and torch.isnan(bad["y"]).all()
+    assert bad["err"].cpu().numpy().tolist() == [1, 0, E // 2, 1, -1, 0]
