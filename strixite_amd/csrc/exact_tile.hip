@@ -270,6 +270,37 @@ __global__ void __launch_bounds__(kMaxWaves *kWave)
         if (c0 + 16 * t + j < a.ncol) store(a, y_f32, m, c0 + 16 * t + j, bad ? qnan() : out[t]);
 }
 
+// One token: block (16 output columns), a wave a slot over all of K; the slots' dots meet in LDS. What bounds it: latency
+// (the rows of eight to eleven experts, one round of loads a K step). A launch and the partials' round trip less than
+// down and combine apart: measured on MI355X, H 2048, I 512, 8 slots, Q8: 7.0 + 4.4 -> 7.6 us; H 2560, I 640, 11 slots,
+// Q4: 9.4 + 4.4 -> 8.1.
+template <int FMT, int SP>
+__global__ void __launch_bounds__(kOneTokenSlots *kWave)
+    one_token_down_kernel(Args a, const float *coef, const uint16_t *resid, uint16_t *out) {
+    __shared__ float dots[kOneTokenSlots][16], cf[kOneTokenSlots];
+    __shared__ int bad[kOneTokenSlots];
+    const int lane = threadIdx.x % kWave, slot = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t c0 = (int64_t)blockIdx.x * 16;
+    const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[slot]);
+    const bool nan = id < 0 || id >= a.E;
+    const float c = coef[slot];
+    const uint16_t xr = out != nullptr && threadIdx.x < 16 ? resid[c0 + threadIdx.x] : (uint16_t)0;
+    float4v acc[1];
+    tile_dot<FMT, SP, uint16_t, 1>(a, tile_rows<FMT, false, 1>(a, nan ? 0 : id, c0),
+                                   static_cast<const uint16_t *>(a.x) + (int64_t)slot * a.K, 0, (int)(a.K / SP), acc);
+    if (lane < 16) dots[slot][lane] = acc[0][0];  // MFMA row 0
+    if (lane == 0) cf[slot] = c, bad[slot] = nan;
+    __syncthreads();
+    const int j = threadIdx.x;
+    if (j >= 16) return;
+    float v = 0.f;
+    bool b = false;
+    for (int s = 0; s < (int)a.A; ++s) v = fmaf(cf[s], dots[s][j], v), b = b || bad[s];
+    const uint16_t y = f32_to_bf16(b ? qnan() : v);
+    static_cast<uint16_t *>(a.y)[c0 + j] = y;
+    if (out != nullptr) out[c0 + j] = f32_to_bf16(bf16_to_f32(xr) + bf16_to_f32(y));
+}
+
 int device_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -347,6 +378,16 @@ void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStre
         else
             exact_perslot_combine_kernel<FMT, SP, uint16_t, RT>
                 <<<blocks, nw * kWave, 0, stream>>>(a, coef, false, (int)cbs, (int)bpt, ks);
+    });
+}
+
+void one_token_down(int fmt, const Args &a, const float *coef, const uint16_t *resid, uint16_t *out, hipStream_t stream) {
+    STRIX_CHECK((fmt == 4 || fmt == 8) && a.A >= 1 && a.A <= kOneTokenSlots && a.ncol % 16 == 0, "one-token down: Q", fmt,
+                ", ", a.A, " slots, ", a.ncol, " columns");
+    by_format(fmt, a.G, [&](auto fc, auto sc) {
+        constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value;
+        if constexpr (FMT != 5)
+            one_token_down_kernel<FMT, SP><<<(unsigned)(a.ncol / 16), (unsigned)a.A * kWave, 0, stream>>>(a, coef, resid, out);
     });
 }
 

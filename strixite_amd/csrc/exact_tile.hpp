@@ -32,4 +32,10 @@ void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &
 // NaN row and the error word. x rows are slots; a.S = M; x and y share a dtype.
 void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStream_t stream);
 
+// One token's down, combine and residual in one launch (Q4 or Q8 experts, BF16, at most kOneTokenSlots slots): y [ncol] =
+// sum over the slots, in order with fmaf, of coef[slot] (x[slot] . W[ids[slot]]), rounded to BF16 once; out (optional) =
+// resid + y. An invalid id: NaN. a.x: h [A, K], a.ids [A], a.y: y.
+constexpr int64_t kOneTokenSlots = 16;
+void one_token_down(int fmt, const Args &a, const float *coef, const uint16_t *resid, uint16_t *out, hipStream_t stream);
+
 }  // namespace strix::kernels::xt

@@ -2142,6 +2142,16 @@ void moe_layer_forward(const MoeLayerWeights &w, const void *x, int64_t M, const
             linear_q4_experts_gather_grouped_swiglu(x, w.gate_up, Es, route, L.route_bytes, M, A, h, Act::BF16,
                                                     MoeMath::WmmaBf16, stream, false);
     }
+    // one token without a separate shared expert: down, combine and residual in one launch
+    if (M == 1 && !w.has_shared && inject == nullptr && A <= xt::kOneTokenSlots) {
+        const QV dv = q8 ? qv(dn8) : qv(w.down);
+        check_view(fn, dv, Es);
+        xt::Args t = tile_args(dv, Es, h, y, H);
+        t.A = A, t.S = A, t.ids = ids;
+        xt::one_token_down(dv.bits, t, coef, static_cast<const uint16_t *>(x), static_cast<uint16_t *>(x_out), stream);
+        STRIX_HIP_CHECK_LAUNCH(fn, " M=1 E=", E, " k=", k);
+        return;
+    }
     {
         const QV dv = q8 ? qv(dn8) : qv(w.down);
         check_view(fn, dv, Es);
