@@ -119,6 +119,34 @@ def test_dense_tiles_and_gemm(bits, G, M, N, K):
     assert _rel64(lin(x, w), ref) < 2.0 ** -8  # one BF16 rounding
 
 
+# the exact GEMM's blocks dealt to the XCDs in runs: item counts around multiples of 8, one bucket of all the slots,
+# an empty one, ragged columns, and a slot with an invalid id
+@pytest.mark.parametrize("bits,M,A,E,H,I", [(8, 1090, 1, 1, 128, 128), (8, 520, 2, 3, 192, 144),
+                                            (4, 400, 3, 6, 128, 64), (8, 610, 2, 5, 320, 272)])
+def test_exact_gemm_items(bits, M, A, E, H, I):
+    say("exact gemm", bits, M, A, E, H, I)
+    gu, dn = _weight(bits, E * 2 * I, H, 64, 71), _weight(bits, E * H, I // 64 * 64, 64, 72)
+    K = dn.K
+    x = _bf16(orc.gen_bf16_normal(orc.tensor_key(10, "x"), 1.0, (M, H)))
+    h = _bf16(orc.gen_bf16_normal(orc.tensor_key(11, "x"), 1.0, (M * A, K)))
+    ids = np.random.default_rng(M).integers(0, max(1, E - 1), size=(M, A)).astype(np.int32)  # the last expert: no slot
+    ids[M // 2, A - 1] = E
+    tid = torch.from_numpy(ids).to(DEV)
+    ws, _ = moe.moe_group_routes(tid, E)
+    ex = moe.MOE_MATH_WMMA_BF16
+    got = moe.experts_gather_grouped_swiglu(x, gu, E, ws, M, A, math=ex)
+    pt = torch.full((M * A, H), 7.0, dtype=torch.float32, device=DEV)
+    moe.experts_combine_grouped(h, dn, E, tid, torch.ones((M, A), device=DEV), ws, M, A, partial=pt, math=ex)
+    flat = ids.ravel()
+    good, bad = np.flatnonzero(flat < E), np.flatnonzero(flat >= E)
+    X, Hd, g64, d64 = x.double().cpu().numpy(), h.double().cpu().numpy(), _w64(gu), _w64(dn)
+    z = np.stack([X[s // A] @ g64[flat[s] * 2 * I:(flat[s] + 1) * 2 * I].T for s in good])
+    p = np.stack([Hd[s] @ d64[flat[s] * H:(flat[s] + 1) * H].T for s in good])
+    assert _rel64(got[good], z[:, :I] / (1 + np.exp(-z[:, :I])) * z[:, I:]) < 2.0 ** -8  # one BF16 rounding
+    assert _rel64(pt[good], p) < 1e-4  # FP32 sums; Q4 codes carry an offset of 128
+    assert torch.isnan(got[bad].float()).all() and torch.isnan(pt[bad]).all()
+
+
 # the down mix's kernels at the ends of their ranges: lane dots of 2 and 3 tokens and a row remainder, split-K tiles of
 # each size (blocks of 16 x 16, 16 x 32, 32 x 32, 32 x 64) with 64- and 32-code steps and streams of a half group, a
 # stream too wide for the split's LDS, FP32 lane dots
