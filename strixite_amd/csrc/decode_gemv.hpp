@@ -748,8 +748,8 @@ inline bool scales_dword_aligned(const GemmArgs &ga) {
 }
 // the LDS-ring down kernel's shapes: Q4 g128, K = 512 or 640 (the benchmark's and the served model's I); it deals its
 // waves to tiles, so every tile needs a wave. Measured on MI355X at H 2560, I 640, 513 experts, 11 slots a token, against
-// the register-fed stream kernels (this and the gate_up at W = 10 together): a layer of 11 tokens 116 -> 86 us, of 1
-// token 40.0 -> 33.5, of 333 tokens 526 -> 366
+// the register-fed stream kernels (this and the gate_up at W = 10 together, the rest of the layer as it was): a layer of 11
+// tokens 116 -> 86 us, of 1 token 40.0 -> 33.5, of 333 tokens 526 -> 366
 inline bool down_lds_fits(const GemmArgs &ga) {
     const int64_t tiles = std::min(ga.S, ga.S / 16 + ga.E + 2);
     auto waves = [](auto ks) { return gdn::blocks_per_cu<decltype(ks)::value>() * gdn::waves<decltype(ks)::value>(); };

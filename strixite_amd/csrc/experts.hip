@@ -268,10 +268,6 @@ __device__ __forceinline__ RawItem load_raw(const GemmArgs &a, int64_t item, int
         const int32_t *rec = a.ws + route::t16_rec_at(a.S, a.E) + route::kRec16 * (int64_t)tile;
         r.expert = rec[0];
         r.my = rec[4 + j];
-    } else if constexpr (MODE == DENSE) {
-        const int32_t st = (int32_t)tile * 16, rows = a.M - st < 16 ? (int32_t)(a.M - st) : 16;
-        r.expert = 0;
-        r.my = j < rows ? st + j : -1;
     } else {
         r.expert = a.ids[tile];
         r.my = j == 0 ? (int32_t)tile : -1;
@@ -287,7 +283,7 @@ __device__ __forceinline__ Item<RT> make_item(const GemmArgs &a, const RawItem &
     it.valid = item < n_items;
     const uint32_t tile = (uint32_t)item / (uint32_t)col_blocks, cb = (uint32_t)item % (uint32_t)col_blocks;
     const int32_t id = __builtin_amdgcn_readfirstlane(raw.expert);
-    it.nan = MODE != DENSE && (id < 0 || id >= a.E);
+    it.nan = id < 0 || id >= a.E;
     const uint32_t expert = it.nan ? 0u : (uint32_t)id;
     it.expert = expert;
     if constexpr (MODE == PERSLOT) {
@@ -1187,9 +1183,9 @@ void launch_gemm_v(const GemmArgs &a, int64_t tiles_bound, const SharedJob &sh, 
     const int64_t blocks = std::max<int64_t>(1, std::min(want, cap)) + sh.blocks;
     // 32-bit buffer offsets: the weight view and the activations must each stay below 2 GiB
     const int64_t q_bytes = a.N * a.E * a.K * BITS / 8, s_bytes = a.N * a.E * (a.K / a.G) * 2;
-    const int64_t x_rows = MODE == GROUPED ? (XROW_DIV ? a.S / a.A : a.S) : MODE == DENSE ? a.M : (XROW_DIV ? a.M : a.M * a.A);
+    const int64_t x_rows = MODE == GROUPED ? (XROW_DIV ? a.S / a.A : a.S) : (XROW_DIV ? a.M : a.M * a.A);
     const int64_t x_bytes = x_rows * a.K * 2;
-    const int64_t y_rows = MODE == GROUPED ? a.S : MODE == DENSE ? a.M : a.M * a.A;
+    const int64_t y_rows = MODE == GROUPED ? a.S : a.M * a.A;
     const int64_t y_bytes = y_rows * a.ldy * (EPI == EPI_F32 ? 4 : 2);
     STRIX_CHECK(q_bytes < (1ll << 31) && s_bytes < (1ll << 31) && x_bytes < (1ll << 31) && y_bytes < (1ll << 31),
                 "expert kernels: weight (", q_bytes, " B), activation (", x_bytes, " B) or output (", y_bytes,
