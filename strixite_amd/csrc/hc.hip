@@ -789,13 +789,6 @@ __global__ void __launch_bounds__(256)
 }
 
 // ================================================================================================ up: MFMA tiles
-// 1 / (1 + e^-a). FAST (u in BF16, rounded at 2^-9): the hardware's FP32 exponential and reciprocal, a few 2^-24 off (4
-// instructions for ~40, and there are four gates an output: 2000 tokens at d 2560, r 320 went 90 -> 81 us; u's error against 64 bits unchanged)
-template <bool FAST> __device__ __forceinline__ float gate_of(float a) {
-    if constexpr (FAST) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896340736f));
-    else return 1.0f / (1.0f + expf(-a));
-}
-
 // WAVES column tiles of 16 positions j a block (a wave each), MT 16-token tiles; LDS: h as bf16 hi / mid / lo [16 MT][r + 8]
 // in the paired k order, then its group sums [r / G][16 MT] (FP32)
 // TWO: registers held to what lets two blocks share a CU, for grids of more blocks than CUs
@@ -978,7 +971,7 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
             float sum = 0.f;
 #pragma unroll
             for (int s = 0; s < kStreams; ++s) {
-                const float gate = gate_of<std::is_same<T, uint16_t>::value>(acc[s][m][i]);
+                const float gate = 1.0f / (1.0f + expf(-acc[s][m][i]));
                 sum += gate * (xe[m][i][s] * ie[m][i][s] * nwv[s]);
             }
             st_act(u, t * d + j, sum * 0.25f);

@@ -206,3 +206,16 @@ def test_one_token_layer_matches_two(shared, bits, H, I, E, k):
     bad = layer.forward(x[:1].contiguous(), logits_in=lg)
     assert (bad["ids"] == -1).all() and torch.isnan(bad["y"]).all()
     assert bad["err"].cpu().numpy().tolist() == [1, 0, E // 2, 1, -1, 0]
+
+
+# u in BF16 is the FP32 u rounded once: the same gates, products and sums on BF16-valued streams in either dtype (a gate
+# a few 2^-24 off rounds some of these outputs the other way)
+@pytest.mark.parametrize("bits,G,T,d,r", [(4, 64, 700, 2560, 320), (8, 64, 600, 1024, 128), (4, 32, 9, 2560, 96)])
+def test_mix_up_bf16_is_the_rounded_fp32(bits, G, T, d, r):
+    say("mix up bf16", bits, G, T, d, r)
+    x = _bf16(orc.gen_bf16_normal(orc.tensor_key(12, "x"), 1.0, (T, 4 * d)))
+    rng = np.random.default_rng(T)
+    w = _weight(bits, 4 * d, r, G, 81)  # any codes: both calls read them chunk-major
+    h, inv, nw = (torch.from_numpy(a.astype(np.float32)).to(DEV) for a in
+                  (rng.standard_normal((T, r)), rng.uniform(0.5, 1.5, (T, 4)), rng.standard_normal(4 * d) * 0.1))
+    assert torch.equal(moe.hc_mix_up(h, w, x, nw, inv), moe.hc_mix_up(h, w, x.float(), nw, inv).to(torch.bfloat16))
