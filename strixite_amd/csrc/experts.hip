@@ -2035,8 +2035,9 @@ void moe_layer_forward(const MoeLayerWeights &w, const void *x, int64_t M, const
         a.M = M;
         GemmArgs b = make_args(dv, 1, sh_h, sh_s, H);
         b.M = M;
-        if (M >= kSharedGemmMinTokens && H % gemm::BK == 0 && I % gemm::BK == 0 && gv.G % gemm::BK == 0 &&
-            dv.G % gemm::BK == 0) {
+        // (a row of more than kMaxGroups groups is not the GEMM's: its scales and mins would not fit the block's LDS)
+        auto gemm_takes = [](const QV &v) { return v.K % gemm::BK == 0 && v.G % gemm::BK == 0 && v.K / v.G <= gemm::kMaxGroups; };
+        if (M >= kSharedGemmMinTokens && gemm_takes(gv) && gemm_takes(dv)) {
             launch_expert_gemm<8, DENSE, EPI_SWIGLU, false, false>(a, sh_stream);
             launch_expert_gemm<8, DENSE, EPI_BF16, false, false>(b, sh_stream);
         } else {

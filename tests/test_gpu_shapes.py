@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import oracle as orc
-from gpu_util import qspec, rel_err, to_np
+from gpu_util import oracle_weights, qspec, rel_err, to_np
 from strixite_amd import moe
 
 pytestmark = pytest.mark.gpu
@@ -219,3 +219,16 @@ def test_mix_up_bf16_is_the_rounded_fp32(bits, G, T, d, r):
     h, inv, nw = (torch.from_numpy(a.astype(np.float32)).to(DEV) for a in
                   (rng.standard_normal((T, r)), rng.uniform(0.5, 1.5, (T, 4)), rng.standard_normal(4 * d) * 0.1))
     assert torch.equal(moe.hc_mix_up(h, w, x, nw, inv), moe.hc_mix_up(h, w, x.float(), nw, inv).to(torch.bfloat16))
+
+
+# a separate shared expert whose rows hold more groups than the GEMM's (H 4096, g 64), on either side of the sizes that
+# go to the GEMM
+@pytest.mark.parametrize("M", [100, 130])
+def test_layer_shared_expert_of_many_groups(M):
+    say("shared expert, H 4096", M)
+    layer = moe.MoeLayer.synth(4096, 8, 2, 128, seed=5)
+    x = moe.synth_bf16_normal(5, "x", 0, (M, 4096), 1.0)
+    out = layer.forward(x)
+    o = orc.moe_layer(oracle_weights(layer), to_np(x)[:16])
+    assert np.array_equal(to_np(out["ids"])[:16], o["ids"])
+    assert rel_err(to_np(out["y"])[:16], o["y"]) < 1e-2  # the layer tests' tolerance
