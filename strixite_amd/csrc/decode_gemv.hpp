@@ -823,14 +823,9 @@ template <int SPW>
 void launch_decode_gate_up_spw(const DecodeArgs &d, const SharedJob &s, hipStream_t stream) {
     constexpr int W = kDecGuWaves, R = kDecGuAhead;
     const size_t lds = dec_gu_lds<W, SPW>(kDecMaxTiles);
-    static thread_local bool attr = false;
-    if (!attr) {
-        for (const void *k : {reinterpret_cast<const void *>(decode_gate_up_kernel<W, SPW, R, 0>),
-                              reinterpret_cast<const void *>(decode_gate_up_kernel<W, SPW, R, 1>)})
-            STRIX_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                            "decode gate_up: LDS of ", lds, " bytes");
-        attr = true;
-    }
+    const void *kern = s.blocks > 0 ? reinterpret_cast<const void *>(decode_gate_up_kernel<W, SPW, R, 1>)
+                                    : reinterpret_cast<const void *>(decode_gate_up_kernel<W, SPW, R, 0>);
+    STRIX_HIP_CHECK(allow_lds(kern, lds), "decode gate_up: LDS of ", lds, " bytes");
     const unsigned blocks = (unsigned)(device_cus() + s.blocks);
     if (s.blocks > 0) decode_gate_up_kernel<W, SPW, R, 1><<<blocks, W * kWave, lds, stream>>>(d, s);
     else decode_gate_up_kernel<W, SPW, R, 0><<<blocks, W * kWave, lds, stream>>>(d, s);

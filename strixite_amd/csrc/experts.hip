@@ -14,6 +14,7 @@
 // served layout: q4g128, q8g64).
 #include "common.hpp"
 #include "exact_tile.hpp"
+#include "lds_grant.hpp"
 #include "route_small.hpp"
 #include "router_small.hpp"
 

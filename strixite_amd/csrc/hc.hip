@@ -38,11 +38,10 @@
 // * Split-K tiles and lane dots (down mix, smaller batches): described at mix_down_split_kernel and mix_down_dot_kernel.
 #include "common.hpp"
 #include "exact_frag.hpp"
+#include "lds_grant.hpp"
 
 #include <algorithm>
 #include <cmath>
-#include <mutex>
-#include <vector>
 
 namespace strix::kernels {
 
@@ -984,20 +983,6 @@ inline size_t up_tile_lds(int MT, int64_t r, int64_t G) {
 }
 
 // ================================================================================================ launchers
-// Raises a tile kernel's dynamic LDS allowance to `bytes` when it is below (kept per kernel, so a launch that needs
-// no more than before makes no runtime call).
-void allow_lds(const void *kernel, size_t bytes) {
-    static std::mutex mu;
-    static std::vector<std::pair<const void *, size_t>> granted;
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = std::find_if(granted.begin(), granted.end(), [&](const auto &e) { return e.first == kernel; });
-    if (it != granted.end() && it->second >= bytes) return;
-    STRIX_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes),
-                    "hc mix: allowing ", bytes, " bytes of LDS");
-    if (it != granted.end()) it->second = bytes;
-    else granted.emplace_back(kernel, bytes);
-}
-
 struct Weights {  // either format's arrays
     const uint8_t *q;
     const uint16_t *scale, *minv;
@@ -1048,7 +1033,7 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
             const size_t lds = down_split_lds<TT, RT, NW>(ng);
             if (lds > kDownSplitLds) return;  // a stream too wide for the scales' LDS space: the lane dots take it
             auto k = mix_down_split_kernel<BITS, SP, TT, RT, NW>;
-            allow_lds((const void *)k, lds);
+            STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
             k<<<(unsigned)split_blocks(TT, RT), NW * kWave, lds, stream>>>(static_cast<const uint16_t *>(x), w.q, w.scale,
                                                                           w.minv, R, d, w.G, r, eps, T, h, w_in, inv, ng);
             done = true;
@@ -1071,7 +1056,7 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
             constexpr int GG = decltype(gtag)::value;
             constexpr int KH = down_tile_halves<BITS, std::is_same<TT, float>::value>();
             auto k = mix_down_tile_kernel<TT, BITS, GG, KH>;
-            allow_lds((const void *)k, lds);
+            STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
             k<<<(unsigned)(nrb * ntt), dn::kThreads * KH, lds, stream>>>(static_cast<const TT *>(x), w.q, w.scale, w.minv,
                                                                     R, d, r, eps, T, h, w_in, inv);
         };
@@ -1125,7 +1110,7 @@ void run_mix_up(const float *h, const Weights &w, const void *x, const float *no
         using TT = decltype(tag);
         constexpr int M = decltype(mtag)::value, WV = M == 1 ? 4 : 8;
         auto k = M == 2 && two ? mix_up_tile_kernel<TT, BITS, M, WV, M == 2> : mix_up_tile_kernel<TT, BITS, M, WV, false>;
-        allow_lds((const void *)k, lds);
+        STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
         k<<<(unsigned)(njb * ntt), WV * kWave, lds, stream>>>(h, w.q, w.scale, w.minv, static_cast<const TT *>(x),
                                                               norm_w, inv, d, w.K, w.G, T, static_cast<TT *>(u));
     };

@@ -7,6 +7,7 @@
 // equal buckets in lane order and one leader lane updates the bucket's count - no atomics, so the placement is the
 // stable order by construction. Small S (<= 16 chunks) runs as one 1024-thread block with everything in LDS; larger S
 // as three launches (chunk histograms, scan, placement) through the workspace.
+#include "lds_grant.hpp"
 #include "route_small.hpp"
 
 #include <type_traits>
@@ -244,11 +245,9 @@ void moe_group_routes(const int32_t *ids, int64_t M, int64_t A, int64_t E, void 
     int32_t *w = static_cast<int32_t *>(ws);
     const size_t small_lds = topk_route_small_lds(L, false);
     if (L.S <= kSmallSlots && small_lds <= kSmallLds) {
-        if (small_lds > 64 * 1024) {
-            static const hipError_t granted = hipFuncSetAttribute(reinterpret_cast<const void *>(route_small_kernel),
-                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds);
-            STRIX_HIP_CHECK(granted, fn, ": LDS of ", kSmallLds, " bytes");
-        }
+        if (small_lds > 64 * 1024)
+            STRIX_HIP_CHECK(allow_lds(reinterpret_cast<const void *>(route_small_kernel), kSmallLds), fn, ": LDS of ",
+                            kSmallLds, " bytes");
         route_small_kernel<<<1, 1024, small_lds, stream>>>(ids, L, nbits, w, err);
     } else {
         const unsigned blocks = (unsigned)((L.nch + kWavesPerBlock - 1) / kWavesPerBlock);
