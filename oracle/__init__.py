@@ -28,10 +28,10 @@ TENSOR = {  # tensor ids of the seeded generator (shared with strixite_amd/csrc/
 
 
 def build(force: bool = False) -> None:
-    """Compiles liboracle_moe.so (and, where /root/reference exists, oracle/_ref) with the Makefile here."""
+    """Compiles liboracle_moe.so (and, where /root/reference holds the formats' sources, oracle/_ref) with the Makefile here."""
     if force or not os.path.exists(_LIB):
         subprocess.run(["make", "-s", "-C", _HERE] + (["-B"] if force else []) + ["all"], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/formats/q4.cpp"):
         subprocess.run(["make", "-s", "-C", _HERE, "ref"], check=True)
 
 
