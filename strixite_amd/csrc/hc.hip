@@ -12,7 +12,7 @@
 //     j])), W_up [4 d, r] chunk-major (32-code chunk c of row n at q[(c N + n) * 16] (Q4) or [(c N + n) * 32] (Q8),
 //     group g's scale / min at [g N + n]; strixite formats/q4.hpp:43-55).
 //
-// The kernels, chosen by the token count (kDownDotTokens):
+// The kernels, chosen by the sizes (hc_plan.hpp):
 //
 // * Matrix-core tiles (the up mix from 1 token; the down mix of large batches with d % 128 == 0). Weights enter the
 //   bf16 MFMA (v_mfma_f32_16x16x32_bf16) as their exact integer codes and each quantization group's partial product D is
@@ -38,6 +38,7 @@
 // * Split-K tiles and lane dots (down mix, smaller batches): described at mix_down_split_kernel and mix_down_dot_kernel.
 #include "common.hpp"
 #include "exact_frag.hpp"
+#include "hc_plan.hpp"
 #include "lds_grant.hpp"
 
 #include <algorithm>
@@ -50,16 +51,6 @@ namespace {
 using namespace strix::dev;
 constexpr int kWave = 64, kStreams = 4, kChunk = 32;
 constexpr int64_t kMaxR = 1024, kMaxTokens = 65535, kMaxD = 1 << 20;
-// The down mix's kernels (us on MI355X at d 2560, r 320, Q4 g64):
-// - lane dots up to this many BF16 tokens: 4.3 at 1 token, 6.1 at 4, 10.2 at 16, 19 at 40, 27 at 64, in proportion;
-// - split-K tiles above, as long as their blocks are at most the CUs (16 tokens x 16 rows a block 18 us flat, 16 x 32 24,
-//   32 x 32 36, 32 x 64 50): a block's time is its K walk, whatever the grid;
-// - then the staged tiles, flat in T until their blocks pass the CUs.
-// FP32 streams (three MFMA rows or products a value): lane dots (20 at 40 tokens, 99 at 255) up to the staged tiles' 168.
-// Before: vector rows 5.6 / 12 / 24 / 35 / 45, 146 at 255 tokens (FP32 43 at 16, 426 at 255), staged tiles 104 from 256.
-constexpr int64_t kDownDotTokens = 32, kDownTileF32Tokens = 440;
-constexpr size_t kDownSplitLds = 160 * 1024 - 1024;
-
 int device_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -158,6 +149,7 @@ constexpr int kRows = kWaves * kTilesPW * 16;          // weight rows a block
 constexpr int kTok = 32;                               // tokens a block: two 16-token MFMA tiles
 constexpr int kK = 128;                                // k a stage
 constexpr int kAdw = kK / 2 + 4;                       // dwords of a staged activation row (bf16, padded)
+static_assert(kRows == hcp::kStageRows && kTok == hcp::kStageTok && kK == hcp::kStageK, "the plan's block sizes");
 template <int BITS> constexpr int wdw() { return BITS == 4 ? 20 : 36; }  // dwords of a staged weight row (padded)
 // stage layout in dwords: W [kRows][wdw] | A hi [kTok][kAdw] | A lo (F32) | xs [4][kTok] | sc [kRows][4] |
 // mp [kRows][4]
@@ -631,16 +623,6 @@ __global__ void __launch_bounds__(NW *kWave)
     }
 }
 
-// groups a wave's K range can touch
-template <int SP, int NW> uint32_t down_split_groups(int64_t d, int64_t G) {
-    const int64_t pw = NW / kStreams, steps = (d / SP + pw - 1) / pw;
-    return (uint32_t)((steps * SP + G - 1) / G + 1);
-}
-// the waves' scales and mins, then their sums
-template <int TT, int RT, int NW> size_t down_split_lds(uint32_t ng) {
-    return std::max((size_t)NW * TT * (RT + 1) * kWave * 16, (size_t)NW * ng * 16 * RT * 4);
-}
-
 // ================================================================================================ down: lane dots
 // A block takes MT tokens x RW weight rows, one wave a stream: lane l takes the stream's 8-element chunks l, l + 64, ...
 // - a token's 16 (BF16) or 32 (FP32) bytes and a row's 4 or 8 code bytes, so every load of a wave is contiguous -, a
@@ -977,11 +959,6 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
         }
 }
 
-inline size_t up_tile_lds(int MT, int64_t r, int64_t G) {
-    const int64_t ngr4 = (r / G + 3) / 4 * 4;
-    return (size_t)(3 * 16 * MT * (r / 2 + 4) + ngr4 * 16 * MT) * 4;
-}
-
 // ================================================================================================ launchers
 struct Weights {  // either format's arrays
     const uint8_t *q;
@@ -1020,35 +997,27 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
     STRIX_CHECK(std::isfinite(eps) && eps > 0.f, what, ": eps = ", eps, " (a finite positive value is needed)");
     const bool f32 = act == Act::F32;
     using std::integral_constant;
-    // which kernel, by what each is bound by (see kDownDotTokens)
-    const int64_t cus = device_cus();
-    auto split_blocks = [&](int tt, int rt) { return ((R + 16 * rt - 1) / (16 * rt)) * ((T + 16 * tt - 1) / (16 * tt)); };
-    const bool tiles = d % dn::kK == 0 && (f32 ? T >= kDownTileF32Tokens : split_blocks(2, 4) > cus);
-    const int variant = split_blocks(1, 1) <= cus ? 0 : split_blocks(1, 2) <= cus ? 1 : split_blocks(2, 2) <= cus ? 2 : 3;
-    bool done = false;
-    if (!f32 && !tiles && T > kDownDotTokens) {
-        auto go = [&](auto spc, auto ttc, auto rtc, auto nwc) {
-            constexpr int SP = decltype(spc)::value, TT = decltype(ttc)::value, RT = decltype(rtc)::value, NW = decltype(nwc)::value;
-            const uint32_t ng = down_split_groups<SP, NW>(d, w.G);
-            const size_t lds = down_split_lds<TT, RT, NW>(ng);
-            if (lds > kDownSplitLds) return;  // a stream too wide for the scales' LDS space: the lane dots take it
-            auto k = mix_down_split_kernel<BITS, SP, TT, RT, NW>;
+    const hcp::DownPlan plan = hcp::plan_down(f32, w.G, T, R, d, device_cus());
+    if (plan.kernel == hcp::Down::Split) {
+        auto go = [&](auto spc, auto vc) {
+            constexpr int SP = decltype(spc)::value;
+            constexpr hcp::Split S = hcp::kSplits[decltype(vc)::value];
+            const size_t lds = hcp::split_lds(S, d, w.G);
+            auto k = mix_down_split_kernel<BITS, SP, S.TT, S.RT, S.NW>;
             STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
-            k<<<(unsigned)split_blocks(TT, RT), NW * kWave, lds, stream>>>(static_cast<const uint16_t *>(x), w.q, w.scale,
-                                                                          w.minv, R, d, w.G, r, eps, T, h, w_in, inv, ng);
-            done = true;
+            k<<<(unsigned)hcp::split_blocks(S, T, R), S.NW * kWave, lds, stream>>>(
+                static_cast<const uint16_t *>(x), w.q, w.scale, w.minv, R, d, w.G, r, eps, T, h, w_in, inv,
+                hcp::split_groups(S, d, w.G));
         };
-        auto by_variant = [&](auto spc) {
-            if (variant == 0) go(spc, integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 16>{});
-            else if (variant == 1) go(spc, integral_constant<int, 1>{}, integral_constant<int, 2>{}, integral_constant<int, 16>{});
-            else if (variant == 2) go(spc, integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
-            else go(spc, integral_constant<int, 2>{}, integral_constant<int, 4>{}, integral_constant<int, 8>{});
+        auto by_split = [&](auto spc) {
+            if (plan.split == 0) go(spc, integral_constant<int, 0>{});
+            else if (plan.split == 1) go(spc, integral_constant<int, 1>{});
+            else if (plan.split == 2) go(spc, integral_constant<int, 2>{});
+            else go(spc, integral_constant<int, 3>{});
         };
-        if (w.G >= 64 && d % 64 == 0) by_variant(integral_constant<int, 64>{});
-        else by_variant(integral_constant<int, 32>{});
-    }
-    if (done) {
-    } else if (tiles) {  // matrix-core tiles, K staged by the block
+        if (hcp::split_step(d, w.G) == 64) by_split(integral_constant<int, 64>{});
+        else by_split(integral_constant<int, 32>{});
+    } else if (plan.kernel == hcp::Down::Tiles) {  // matrix-core tiles, K staged by the block
         const int64_t nrb = (R + dn::kRows - 1) / dn::kRows, ntt = (T + dn::kTok - 1) / dn::kTok;
         const size_t lds = f32 ? down_tile_lds<BITS, true>() : down_tile_lds<BITS, false>();
         auto go = [&](auto tag, auto gtag) {
@@ -1098,14 +1067,10 @@ void run_mix_up(const float *h, const Weights &w, const void *x, const float *no
     STRIX_CHECK(reinterpret_cast<uintptr_t>(h) % 16 == 0, what, ": h must start on a 16-byte boundary");
     const int64_t es = act == Act::F32 ? 4 : 2;
     STRIX_CHECK(disjoint(u, T * d * es, x, T * H * d * es), what, ": u and the streams x overlap");
-    // 16-token tiles of 4 waves a block up to 16 tokens, 32-token tiles of 8 waves above (the h tile shared by more
-    // columns); 32-token tiles of h fit the LDS up to r = 768
-    const bool small = T <= 16 || w.K > 768;
+    const auto [small, two] = hcp::plan_up(BITS, act == Act::F32, T, d, w.K, device_cus());
     const int MT = small ? 1 : 2, WAVES = small ? 4 : 8;
-    const size_t lds = up_tile_lds(MT, w.K, w.G);
+    const size_t lds = hcp::up_lds(MT, w.K, w.G);
     const int64_t njb = (d / 16 + WAVES - 1) / WAVES, ntt = (T + 16 * MT - 1) / (16 * MT);
-    // (Q8 codes beside FP32 streams spill at two blocks a CU: 105 against 103 us at 2000 tokens)
-    const bool two = !small && njb * ntt > device_cus() && !(BITS == 8 && act == Act::F32);
     auto go = [&](auto tag, auto mtag) {
         using TT = decltype(tag);
         constexpr int M = decltype(mtag)::value, WV = M == 1 ? 4 : 8;

@@ -1,0 +1,83 @@
+// Which kernel of the hyper-connection mix (hc.hip) a call takes: host arithmetic on its sizes alone.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+namespace strix::kernels::hcp {
+
+// ---- down ------------------------------------------------------------------------------------------------------------
+// The kernels (us on MI355X at d 2560, r 320, Q4 g64):
+// - lane dots up to this many BF16 tokens: 4.3 at 1 token, 6.1 at 4, 10.2 at 16, 19 at 40, 27 at 64, in proportion;
+// - split-K tiles above, as long as their blocks are at most the CUs (16 tokens x 16 rows a block 18 us flat, 16 x 32 24,
+//   32 x 32 36, 32 x 64 50): a block's time is its K walk, whatever the grid;
+// - then the staged tiles, flat in T until their blocks pass the CUs.
+// FP32 streams (three MFMA rows or products a value): lane dots (20 at 40 tokens, 99 at 255) up to the staged tiles' 168.
+// Before: vector rows 5.6 / 12 / 24 / 35 / 45, 146 at 255 tokens (FP32 43 at 16, 426 at 255), staged tiles 104 from 256.
+constexpr int64_t kDownDotTokens = 32, kDownTileF32Tokens = 440;
+constexpr size_t kDownSplitLds = 160 * 1024 - 1024;
+constexpr int64_t kStageK = 128, kStageRows = 192, kStageTok = 32;  // the staged tiles: k a stage, rows and tokens a block
+
+enum class Down { Dots, Split, Tiles };
+
+// A split-K block: TT 16-token tiles x RT 16-row tiles, NW waves
+struct Split {
+    int TT, RT, NW;
+};
+constexpr Split kSplits[4] = {{1, 1, 16}, {1, 2, 16}, {2, 2, 8}, {2, 4, 8}};
+
+inline int64_t split_blocks(const Split &s, int64_t T, int64_t R) {
+    return ((R + 16 * s.RT - 1) / (16 * s.RT)) * ((T + 16 * s.TT - 1) / (16 * s.TT));
+}
+// codes a K step of the split-K tiles
+inline int split_step(int64_t d, int64_t G) { return G >= 64 && d % 64 == 0 ? 64 : 32; }
+// groups a wave's K range can touch
+inline uint32_t split_groups(const Split &s, int64_t d, int64_t G) {
+    const int64_t sp = split_step(d, G), pw = s.NW / 4, steps = (d / sp + pw - 1) / pw;
+    return (uint32_t)((steps * sp + G - 1) / G + 1);
+}
+// the waves' scales and mins, then their sums
+inline size_t split_lds(const Split &s, int64_t d, int64_t G) {
+    return std::max((size_t)s.NW * s.TT * (s.RT + 1) * 64 * 16, (size_t)s.NW * split_groups(s, d, G) * 16 * s.RT * 4);
+}
+
+struct DownPlan {
+    Down kernel;
+    int split;  // of kSplits
+};
+
+inline DownPlan plan_down(bool f32, int64_t G, int64_t T, int64_t R, int64_t d, int64_t cus) {
+    const bool tiles = d % kStageK == 0 && (f32 ? T >= kDownTileF32Tokens : split_blocks(kSplits[3], T, R) > cus);
+    if (tiles) return {Down::Tiles, 0};
+    if (f32 || T <= kDownDotTokens) return {Down::Dots, 0};
+    int v = 0;  // the first whose blocks are at most the CUs
+    while (v < 3 && split_blocks(kSplits[v], T, R) > cus) ++v;
+    // a stream too wide for the scales' LDS space: the lane dots take it
+    if (split_lds(kSplits[v], d, G) > kDownSplitLds) return {Down::Dots, 0};
+    return {Down::Split, v};
+}
+
+// ---- up --------------------------------------------------------------------------------------------------------------
+// LDS of a block's MT 16-token tiles of h: three bf16 pieces and the group sums
+inline size_t up_lds(int MT, int64_t r, int64_t G) {
+    const int64_t ngr4 = (r / G + 3) / 4 * 4;
+    return (size_t)(3 * 16 * MT * (r / 2 + 4) + ngr4 * 16 * MT) * 4;
+}
+
+struct UpPlan {
+    bool small;  // 16-token tiles of 4 waves a block (else 32-token tiles of 8 waves)
+    bool two;    // the variant of two blocks a CU
+};
+
+// 16-token tiles of 4 waves a block up to 16 tokens, 32-token tiles of 8 waves above (the h tile shared by more
+// columns); 32-token tiles of h fit the LDS up to r = 768
+inline UpPlan plan_up(int bits, bool f32, int64_t T, int64_t d, int64_t r, int64_t cus) {
+    const bool small = T <= 16 || r > 768;
+    const int64_t MT = small ? 1 : 2, waves = small ? 4 : 8;
+    const int64_t blocks = (d / 16 + waves - 1) / waves * ((T + 16 * MT - 1) / (16 * MT));
+    // (Q8 codes beside FP32 streams spill at two blocks a CU: 105 against 103 us at 2000 tokens)
+    return {small, !small && blocks > cus && !(bits == 8 && f32)};
+}
+
+}  // namespace strix::kernels::hcp

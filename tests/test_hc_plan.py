@@ -1,0 +1,61 @@
+"""The hyper-connection mix's choice of a kernel (strixite_amd/csrc/hc_plan.hpp) on the CPU, at 256 CUs."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include "hc_plan.hpp"
+#include <cstdio>
+using namespace strix::kernels::hcp;
+int main() {
+    char what;
+    long bits, f32, G, T, r, d;
+    while (std::scanf(" %c %ld %ld %ld %ld %ld %ld", &what, &bits, &f32, &G, &T, &r, &d) == 7) {
+        if (what == 'd') {
+            const DownPlan p = plan_down(f32, G, T, r, d, 256);
+            const char *name[] = {"dots", "split", "tiles"};
+            std::printf("%s %d %ld %zu\n", name[(int)p.kernel], p.split, (long)split_blocks(kSplits[p.split], T, r),
+                        split_lds(kSplits[p.split], d, G));
+        } else {
+            const UpPlan p = plan_up(bits, f32, T, d, r, 256);
+            std::printf("%s%s 0 0 %zu\n", p.small ? "small" : "wide", p.two ? " two" : " one", up_lds(p.small ? 1 : 2, r, G));
+        }
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    tmp = tmp_path_factory.mktemp("plan")
+    (tmp / "p.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++20", "-O1", "-I", os.path.join(ROOT, "strixite_amd", "csrc"), str(tmp / "p.cpp"), "-o",
+                    str(tmp / "p")], check=True)
+
+    def ask(cases):  # (kind, bits, f32, G, T, rows (up: rank), d)
+        text = "\n".join(" ".join(str(int(v) if not isinstance(v, str) else v) for v in c) for c in cases)
+        out = subprocess.run([str(tmp / "p")], input=text, check=True, capture_output=True, text=True).stdout.splitlines()
+        assert len(out) == len(cases)
+        return [line.split() for line in out]
+
+    return ask
+
+
+def test_down_plans_can_run(plan):
+    """Split-K blocks fit the LDS and the CUs, staged tiles have whole stages."""
+    cases = [("d", bits, f32, G, T, R, d) for bits in (4, 8) for f32 in (0, 1) for G in (32, 64, 128)
+             for T in (1, 2, 32, 33, 255, 256, 441, 1000, 4000, 65535) for R in (1, 20, 324, 1028)
+             for d in (32, 96, 128, 160, 2560, 4096, 10240, 65536) if (4 * d) % G == 0]
+    for c, (kernel, split, blocks, lds) in zip(cases, plan(cases)):
+        _, _, f32, _, T, _, d = c
+        if kernel == "split":
+            assert not f32 and T > 32 and int(lds) <= 159 * 1024, c
+            assert int(blocks) <= 256 or (split == "3" and d % 128), c
+        elif kernel == "tiles":
+            assert d % 128 == 0, c
