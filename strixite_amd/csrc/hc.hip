@@ -997,7 +997,7 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
     STRIX_CHECK(std::isfinite(eps) && eps > 0.f, what, ": eps = ", eps, " (a finite positive value is needed)");
     const bool f32 = act == Act::F32;
     using std::integral_constant;
-    const hcp::DownPlan plan = hcp::plan_down(f32, w.G, T, R, d, device_cus());
+    const hcp::DownPlan plan = hcp::plan_down(BITS, f32, w.G, T, R, d, device_cus());
     if (plan.kernel == hcp::Down::Split) {
         auto go = [&](auto spc, auto vc) {
             constexpr int SP = decltype(spc)::value;

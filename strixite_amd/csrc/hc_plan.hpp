@@ -13,9 +13,9 @@ namespace strix::kernels::hcp {
 // - split-K tiles above, as long as their blocks are at most the CUs (16 tokens x 16 rows a block 18 us flat, 16 x 32 24,
 //   32 x 32 36, 32 x 64 50): a block's time is its K walk, whatever the grid;
 // - then the staged tiles, flat in T until their blocks pass the CUs.
-// FP32 streams (three MFMA rows or products a value): lane dots (20 at 40 tokens, 99 at 255) up to the staged tiles' 168.
+// FP32 streams (three MFMA rows or products a value): the cheaper of lane dots and staged tiles (dots_beat_tiles).
 // Before: vector rows 5.6 / 12 / 24 / 35 / 45, 146 at 255 tokens (FP32 43 at 16, 426 at 255), staged tiles 104 from 256.
-constexpr int64_t kDownDotTokens = 32, kDownTileF32Tokens = 440;
+constexpr int64_t kDownDotTokens = 32;
 constexpr size_t kDownSplitLds = 160 * 1024 - 1024;
 constexpr int64_t kStageK = 128, kStageRows = 192, kStageTok = 32;  // the staged tiles: k a stage, rows and tokens a block
 
@@ -42,13 +42,25 @@ inline size_t split_lds(const Split &s, int64_t d, int64_t G) {
     return std::max((size_t)s.NW * s.TT * (s.RT + 1) * 64 * 16, (size_t)s.NW * split_groups(s, d, G) * 16 * s.RT * 4);
 }
 
+// FP32 streams: the lane dots' time is in proportion to tokens x rows x (d + 530) (the reductions at a row's end cost as
+// much as 530 more codes), x 1.5 with Q8 codes; the staged tiles' to the stages of K times the rounds their blocks take on
+// the CUs (one a CU). kTileUnits: what d's worth of stages costs in units of the dots' (0.323e-6 us), from 69 us at d 1024
+// and 171 at 2560 (Q4), 182 (Q8). Measured on MI355X, Q4 g64, us, dots / tiles: d 2560, r 320, 400 tokens 134 / 172, r
+// 384, 439 tokens 171 / 174, r 768, 256 tokens 203 / 168, r 1020, 300 tokens 296 / 175; d 1024, r 320, 439 tokens 75 / 69;
+// Q8, d 2560, r 384, 256 and 439 tokens 155 and 239 / 182.
+inline bool dots_beat_tiles(int bits, int64_t T, int64_t R, int64_t d, int64_t cus) {
+    constexpr int64_t kTileUnits[2] = {200000, 147000};  // Q4, Q8 (the dots' 1.5 taken out)
+    const int64_t blocks = ((R + kStageRows - 1) / kStageRows) * ((T + kStageTok - 1) / kStageTok);
+    return T * R * (d + 530) < (blocks + cus - 1) / cus * d * kTileUnits[bits == 8];
+}
+
 struct DownPlan {
     Down kernel;
     int split;  // of kSplits
 };
 
-inline DownPlan plan_down(bool f32, int64_t G, int64_t T, int64_t R, int64_t d, int64_t cus) {
-    const bool tiles = d % kStageK == 0 && (f32 ? T >= kDownTileF32Tokens : split_blocks(kSplits[3], T, R) > cus);
+inline DownPlan plan_down(int bits, bool f32, int64_t G, int64_t T, int64_t R, int64_t d, int64_t cus) {
+    const bool tiles = d % kStageK == 0 && (f32 ? !dots_beat_tiles(bits, T, R, d, cus) : split_blocks(kSplits[3], T, R) > cus);
     if (tiles) return {Down::Tiles, 0};
     if (f32 || T <= kDownDotTokens) return {Down::Dots, 0};
     int v = 0;  // the first whose blocks are at most the CUs

@@ -154,7 +154,10 @@ def test_exact_gemm_items(bits, M, A, E, H, I):
     (4, 64, "bf16", 2, 160, 33, False), (8, 32, "bf16", 3, 96, 35, True), (4, 64, "bf16", 33, 160, 20, True),
     (4, 128, "bf16", 49, 320, 64, False), (8, 64, "bf16", 257, 128, 320, True), (4, 32, "bf16", 400, 96, 320, True),
     (4, 64, "bf16", 705, 128, 320, True), (8, 64, "bf16", 1500, 64, 320, False), (4, 32, "bf16", 40, 65536, 8, False),
-    (4, 64, "f32", 33, 160, 20, True), (8, 64, "f32", 439, 128, 9, False)])
+    (4, 64, "f32", 33, 160, 20, True), (8, 64, "f32", 439, 128, 9, False),
+    # FP32 staged tiles, either format and each group size: ragged rows and tokens, one and three stages a stream
+    (4, 64, "f32", 500, 128, 1020, True), (8, 64, "f32", 449, 384, 700, False), (4, 32, "f32", 300, 384, 1001, True),
+    (8, 128, "f32", 1001, 128, 321, False)])
 def test_mix_down_kernels(bits, G, act, T, d, r, inject):
     from oracle import hc
 

@@ -16,7 +16,7 @@ int main() {
     long bits, f32, G, T, r, d;
     while (std::scanf(" %c %ld %ld %ld %ld %ld %ld", &what, &bits, &f32, &G, &T, &r, &d) == 7) {
         if (what == 'd') {
-            const DownPlan p = plan_down(f32, G, T, r, d, 256);
+            const DownPlan p = plan_down(bits, f32, G, T, r, d, 256);
             const char *name[] = {"dots", "split", "tiles"};
             std::printf("%s %d %ld %zu\n", name[(int)p.kernel], p.split, (long)split_blocks(kSplits[p.split], T, r),
                         split_lds(kSplits[p.split], d, G));
@@ -59,3 +59,14 @@ def test_down_plans_can_run(plan):
             assert int(blocks) <= 256 or (split == "3" and d % 128), c
         elif kernel == "tiles":
             assert d % 128 == 0, c
+
+
+def test_fp32_crossing_moves_with_the_rows(plan):
+    """FP32 streams: lane dots cost tokens x rows, the staged tiles a K walk whatever the tokens, so the crossing in tokens
+    falls as the rows grow (measured pairs of the kernels' times: dots cheaper below, tiles above)."""
+    pairs = [(4, 2560, 68, 700, 8000), (4, 2560, 324, 400, 700), (4, 2560, 388, 400, 500), (4, 2560, 772, 128, 256),
+             (4, 2560, 1024, 128, 256), (8, 2560, 388, 256, 439), (4, 1024, 324, 256, 439), (8, 2560, 1024, 64, 256)]
+    below = plan([("d", b, 1, 64, lo, R, d) for b, d, R, lo, hi in pairs])
+    above = plan([("d", b, 1, 64, hi, R, d) for b, d, R, lo, hi in pairs])
+    assert [p[0] for p in below] == ["dots"] * len(pairs)
+    assert [p[0] for p in above] == ["tiles"] * len(pairs)
