@@ -13,7 +13,8 @@ namespace strix::kernels::hcp {
 // - split-K tiles above, as long as their blocks are at most the CUs (16 tokens x 16 rows a block 18 us flat, 16 x 32 24,
 //   32 x 32 36, 32 x 64 50): a block's time is its K walk, whatever the grid;
 // - then the staged tiles, flat in T until their blocks pass the CUs.
-// FP32 streams (three MFMA rows or products a value): the cheaper of lane dots and staged tiles (dots_beat_tiles).
+// FP32 streams (three MFMA rows or products a value), and streams too wide for the split-K tiles' LDS: the cheaper of lane
+// dots and staged tiles (dots_beat_tiles).
 // Before: vector rows 5.6 / 12 / 24 / 35 / 45, 146 at 255 tokens (FP32 43 at 16, 426 at 255), staged tiles 104 from 256.
 constexpr int64_t kDownDotTokens = 32;
 constexpr size_t kDownSplitLds = 160 * 1024 - 1024;
@@ -42,16 +43,17 @@ inline size_t split_lds(const Split &s, int64_t d, int64_t G) {
     return std::max((size_t)s.NW * s.TT * (s.RT + 1) * 64 * 16, (size_t)s.NW * split_groups(s, d, G) * 16 * s.RT * 4);
 }
 
-// FP32 streams: the lane dots' time is in proportion to tokens x rows x (d + 530) (the reductions at a row's end cost as
-// much as 530 more codes), x 1.5 with Q8 codes; the staged tiles' to the stages of K times the rounds their blocks take on
-// the CUs (one a CU). kTileUnits: what d's worth of stages costs in units of the dots' (0.323e-6 us), from 69 us at d 1024
-// and 171 at 2560 (Q4), 182 (Q8). Measured on MI355X, Q4 g64, us, dots / tiles: d 2560, r 320, 400 tokens 134 / 172, r
-// 384, 439 tokens 171 / 174, r 768, 256 tokens 203 / 168, r 1020, 300 tokens 296 / 175; d 1024, r 320, 439 tokens 75 / 69;
-// Q8, d 2560, r 384, 256 and 439 tokens 155 and 239 / 182.
-inline bool dots_beat_tiles(int bits, int64_t T, int64_t R, int64_t d, int64_t cus) {
-    constexpr int64_t kTileUnits[2] = {200000, 147000};  // Q4, Q8 (the dots' 1.5 taken out)
+// The lane dots' time is in proportion to tokens x rows x (d + 530) (the reductions at a row's end cost as much as 530 more
+// codes), FP32 Q8 x 1.5; the staged tiles' to the stages of K times the rounds their blocks take on the CUs (one a CU).
+// kTileUnits: what d's worth of stages costs in units of the dots' (0.323e-6 us), the dots' 1.5 taken out. Measured on
+// MI355X, us, dots / tiles:
+// - FP32, d 2560, Q4 g64: r 320, 400 tokens 134 / 172, r 384, 439 tokens 171 / 174, r 768, 256 tokens 203 / 168, r 1020,
+//   300 tokens 296 / 175; d 1024, r 320, 439 tokens 75 / 69; Q8, r 384, 256 and 439 tokens 155 and 239 / 182;
+// - BF16, r 320, 1000 tokens: Q4 g32 d 5120 511 / 155, Q4 g64 d 10240 945 / 292, Q8 g32 d 5120 525 / 295.
+inline bool dots_beat_tiles(int bits, bool f32, int64_t T, int64_t R, int64_t d, int64_t cus) {
+    constexpr int64_t kTileUnits[2][2] = {{94000, 178000}, {200000, 147000}};  // [f32][Q8]
     const int64_t blocks = ((R + kStageRows - 1) / kStageRows) * ((T + kStageTok - 1) / kStageTok);
-    return T * R * (d + 530) < (blocks + cus - 1) / cus * d * kTileUnits[bits == 8];
+    return T * R * (d + 530) < (blocks + cus - 1) / cus * d * kTileUnits[f32][bits == 8];
 }
 
 struct DownPlan {
@@ -60,14 +62,17 @@ struct DownPlan {
 };
 
 inline DownPlan plan_down(int bits, bool f32, int64_t G, int64_t T, int64_t R, int64_t d, int64_t cus) {
-    const bool tiles = d % kStageK == 0 && (f32 ? !dots_beat_tiles(bits, T, R, d, cus) : split_blocks(kSplits[3], T, R) > cus);
-    if (tiles) return {Down::Tiles, 0};
-    if (f32 || T <= kDownDotTokens) return {Down::Dots, 0};
-    int v = 0;  // the first whose blocks are at most the CUs
-    while (v < 3 && split_blocks(kSplits[v], T, R) > cus) ++v;
-    // a stream too wide for the scales' LDS space: the lane dots take it
-    if (split_lds(kSplits[v], d, G) > kDownSplitLds) return {Down::Dots, 0};
-    return {Down::Split, v};
+    const bool stages = d % kStageK == 0;  // the staged tiles take the shape
+    if (!f32) {
+        if (T <= kDownDotTokens) return {Down::Dots, 0};
+        int v = 0;  // the first whose blocks are at most the CUs
+        while (v < 3 && split_blocks(kSplits[v], T, R) > cus) ++v;
+        const bool fits = split_lds(kSplits[v], d, G) <= kDownSplitLds;
+        if (fits && (!stages || split_blocks(kSplits[v], T, R) <= cus)) return {Down::Split, v};
+        if (fits) return {Down::Tiles, 0};
+        // a stream too wide for the scales' LDS space
+    }
+    return {stages && !dots_beat_tiles(bits, f32, T, R, d, cus) ? Down::Tiles : Down::Dots, 0};
 }
 
 // ---- up --------------------------------------------------------------------------------------------------------------

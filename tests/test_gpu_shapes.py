@@ -157,7 +157,9 @@ def test_exact_gemm_items(bits, M, A, E, H, I):
     (4, 64, "f32", 33, 160, 20, True), (8, 64, "f32", 439, 128, 9, False),
     # FP32 staged tiles, either format and each group size: ragged rows and tokens, one and three stages a stream
     (4, 64, "f32", 500, 128, 1020, True), (8, 64, "f32", 449, 384, 700, False), (4, 32, "f32", 300, 384, 1001, True),
-    (8, 128, "f32", 1001, 128, 321, False)])
+    (8, 128, "f32", 1001, 128, 321, False),
+    # BF16 streams too wide for the split-K tiles' LDS, at a token count whose lane dots would cost more than the tiles
+    (4, 32, "bf16", 1000, 5120, 316, True)])
 def test_mix_down_kernels(bits, G, act, T, d, r, inject):
     from oracle import hc
 

@@ -70,3 +70,12 @@ def test_fp32_crossing_moves_with_the_rows(plan):
     above = plan([("d", b, 1, 64, hi, R, d) for b, d, R, lo, hi in pairs])
     assert [p[0] for p in below] == ["dots"] * len(pairs)
     assert [p[0] for p in above] == ["tiles"] * len(pairs)
+
+
+def test_streams_too_wide_for_the_split_go_to_the_cheaper_kernel(plan):
+    """BF16 streams whose split-K scale table does not fit the LDS: staged tiles where their K walk costs less than the lane
+    dots' tokens x rows, the lane dots for few tokens and where a stream has no whole stages."""
+    cases = [(4, 32, 1000, 324, 5120), (8, 32, 1000, 324, 5120), (4, 64, 1000, 324, 10240), (8, 64, 1000, 324, 10240),
+             (4, 32, 1000, 324, 8192), (4, 32, 40, 8, 65536), (4, 32, 1000, 324, 5152)]
+    got = plan([("d", b, 0, G, T, R, d) for b, G, T, R, d in cases])
+    assert [p[0] for p in got] == ["tiles"] * 5 + ["dots"] * 2
