@@ -162,8 +162,8 @@ template <int BITS, bool F32> struct Stage {
 }  // namespace dn
 
 // KH: the block's K in halves (streams 0, 1 and 2, 3), each a group of 4 waves with stage buffers of its own; their totals
-// meet at the end. BF16 takes two (one group alone leaves each SIMD one wave, and a stage's staging, barrier and math
-// follow one another: 104 -> 81 us at 2000 tokens, Q4 g64); the stages of FP32 and of Q8 fill the LDS with one.
+// meet at the end (one group alone leaves each SIMD of its CU one wave, and a stage's staging, barrier and math follow one
+// another). hcp::tile_halves says when.
 template <typename T, int BITS, int G, int KH>
 __global__ void __launch_bounds__(dn::kThreads * KH)
     mix_down_tile_kernel(const T *x, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, int64_t R,
@@ -433,11 +433,6 @@ __global__ void __launch_bounds__(dn::kThreads * KH)
                 else w_in[t * kStreams + (row - r)] = 2.0f / (1.0f + expf(-z));
             }
     }
-}
-
-template <int BITS, bool F32> constexpr int down_tile_halves() { return !F32 && BITS == 4 ? 2 : 1; }
-template <int BITS, bool F32> constexpr size_t down_tile_lds() {
-    return (size_t)down_tile_halves<BITS, F32>() * 2 * dn::Stage<BITS, F32>::SIZE * 4;
 }
 
 // ================================================================================================ down: split-K tiles
@@ -1018,16 +1013,21 @@ void run_mix_down(const void *x, const Weights &w, int64_t T, int64_t H, int64_t
         if (hcp::split_step(d, w.G) == 64) by_split(integral_constant<int, 64>{});
         else by_split(integral_constant<int, 32>{});
     } else if (plan.kernel == hcp::Down::Tiles) {  // matrix-core tiles, K staged by the block
-        const int64_t nrb = (R + dn::kRows - 1) / dn::kRows, ntt = (T + dn::kTok - 1) / dn::kTok;
-        const size_t lds = f32 ? down_tile_lds<BITS, true>() : down_tile_lds<BITS, false>();
         auto go = [&](auto tag, auto gtag) {
-            using TT = decltype(tag);
+            using X = decltype(tag);
             constexpr int GG = decltype(gtag)::value;
-            constexpr int KH = down_tile_halves<BITS, std::is_same<TT, float>::value>();
-            auto k = mix_down_tile_kernel<TT, BITS, GG, KH>;
-            STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
-            k<<<(unsigned)(nrb * ntt), dn::kThreads * KH, lds, stream>>>(static_cast<const TT *>(x), w.q, w.scale, w.minv,
-                                                                    R, d, r, eps, T, h, w_in, inv);
+            constexpr bool F32 = std::is_same<X, float>::value;
+            auto run = [&](auto khc) {
+                constexpr int KH = decltype(khc)::value;
+                constexpr size_t lds = (size_t)KH * 2 * dn::Stage<BITS, F32>::SIZE * 4;
+                auto k = mix_down_tile_kernel<X, BITS, GG, KH>;
+                STRIX_HIP_CHECK(allow_lds((const void *)k, lds), what, ": LDS of ", lds, " bytes");
+                k<<<(unsigned)hcp::tile_blocks(T, R), dn::kThreads * KH, lds, stream>>>(
+                    static_cast<const X *>(x), w.q, w.scale, w.minv, R, d, r, eps, T, h, w_in, inv);
+            };
+            if constexpr (BITS == 4 && !F32)
+                if (plan.halves == 2) return run(integral_constant<int, 2>{});
+            run(integral_constant<int, 1>{});
         };
         auto by_g = [&](auto tag) {
             if (w.G == 32) go(tag, std::integral_constant<int, 32>{});

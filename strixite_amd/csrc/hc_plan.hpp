@@ -43,6 +43,10 @@ inline size_t split_lds(const Split &s, int64_t d, int64_t G) {
     return std::max((size_t)s.NW * s.TT * (s.RT + 1) * 64 * 16, (size_t)s.NW * split_groups(s, d, G) * 16 * s.RT * 4);
 }
 
+inline int64_t tile_blocks(int64_t T, int64_t R) {
+    return ((R + kStageRows - 1) / kStageRows) * ((T + kStageTok - 1) / kStageTok);
+}
+
 // The lane dots' time is in proportion to tokens x rows x (d + 530) (the reductions at a row's end cost as much as 530 more
 // codes), FP32 Q8 x 1.5; the staged tiles' to the stages of K times the rounds their blocks take on the CUs (one a CU).
 // kTileUnits: what d's worth of stages costs in units of the dots' (0.323e-6 us), the dots' 1.5 taken out. Measured on
@@ -52,27 +56,37 @@ inline size_t split_lds(const Split &s, int64_t d, int64_t G) {
 // - BF16, r 320, 1000 tokens: Q4 g32 d 5120 511 / 155, Q4 g64 d 10240 945 / 292, Q8 g32 d 5120 525 / 295.
 inline bool dots_beat_tiles(int bits, bool f32, int64_t T, int64_t R, int64_t d, int64_t cus) {
     constexpr int64_t kTileUnits[2][2] = {{94000, 178000}, {200000, 147000}};  // [f32][Q8]
-    const int64_t blocks = ((R + kStageRows - 1) / kStageRows) * ((T + kStageTok - 1) / kStageTok);
-    return T * R * (d + 530) < (blocks + cus - 1) / cus * d * kTileUnits[f32][bits == 8];
+    return T * R * (d + 530) < (tile_blocks(T, R) + cus - 1) / cus * d * kTileUnits[f32][bits == 8];
 }
 
 struct DownPlan {
     Down kernel;
-    int split;  // of kSplits
+    int split;   // of kSplits
+    int halves;  // staged tiles: K in halves, a wave group each
 };
+
+// K in halves fills a CU that has one block (BF16 streams, Q4: the stages of FP32 and of Q8 fill the LDS with one). Where
+// the blocks pass the CUs, two blocks of one half share a CU and do the same without the totals' exchange, except with
+// groups of 32, whose four rescales a stage leave a group of waves more to hide. Measured on MI355X at d 2560, two halves /
+// one, us: Q4 g64, r 320, 2000 tokens (126 blocks) 81 / 104, r 384, 4000 (375) 164 / 153, r 768, 2000 (315) 166 / 154, 6000
+// 333 / 305; g128, r 768, 2000 140 / 132; g32, r 384, 4000 165 / 172, r 768, 6000 332 / 338.
+inline int tile_halves(int bits, bool f32, int64_t G, int64_t T, int64_t R, int64_t cus) {
+    return !f32 && bits == 4 && (G == 32 || tile_blocks(T, R) <= cus) ? 2 : 1;
+}
 
 inline DownPlan plan_down(int bits, bool f32, int64_t G, int64_t T, int64_t R, int64_t d, int64_t cus) {
     const bool stages = d % kStageK == 0;  // the staged tiles take the shape
     if (!f32) {
-        if (T <= kDownDotTokens) return {Down::Dots, 0};
+        if (T <= kDownDotTokens) return {Down::Dots, 0, 1};
         int v = 0;  // the first whose blocks are at most the CUs
         while (v < 3 && split_blocks(kSplits[v], T, R) > cus) ++v;
         const bool fits = split_lds(kSplits[v], d, G) <= kDownSplitLds;
-        if (fits && (!stages || split_blocks(kSplits[v], T, R) <= cus)) return {Down::Split, v};
-        if (fits) return {Down::Tiles, 0};
+        if (fits && (!stages || split_blocks(kSplits[v], T, R) <= cus)) return {Down::Split, v, 1};
+        if (fits) return {Down::Tiles, 0, tile_halves(bits, f32, G, T, R, cus)};
         // a stream too wide for the scales' LDS space
     }
-    return {stages && !dots_beat_tiles(bits, f32, T, R, d, cus) ? Down::Tiles : Down::Dots, 0};
+    if (stages && !dots_beat_tiles(bits, f32, T, R, d, cus)) return {Down::Tiles, 0, tile_halves(bits, f32, G, T, R, cus)};
+    return {Down::Dots, 0, 1};
 }
 
 // ---- up --------------------------------------------------------------------------------------------------------------

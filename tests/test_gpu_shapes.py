@@ -159,7 +159,11 @@ def test_exact_gemm_items(bits, M, A, E, H, I):
     (4, 64, "f32", 500, 128, 1020, True), (8, 64, "f32", 449, 384, 700, False), (4, 32, "f32", 300, 384, 1001, True),
     (8, 128, "f32", 1001, 128, 321, False),
     # BF16 streams too wide for the split-K tiles' LDS, at a token count whose lane dots would cost more than the tiles
-    (4, 32, "bf16", 1000, 5120, 316, True)])
+    (4, 32, "bf16", 1000, 5120, 316, True),
+    # BF16 staged tiles: K in halves of one and of six stages with each group size, one half past the CUs, Q8
+    (4, 32, "bf16", 1500, 128, 400, True), (4, 64, "bf16", 1200, 384, 385, False), (4, 128, "bf16", 1500, 128, 400, True),
+    (4, 64, "bf16", 1601, 128, 1021, False), (4, 128, "bf16", 1601, 384, 1001, True), (8, 32, "bf16", 1500, 128, 400, True),
+    (8, 64, "bf16", 1200, 384, 385, False), (8, 128, "bf16", 1500, 128, 401, True)])
 def test_mix_down_kernels(bits, G, act, T, d, r, inject):
     from oracle import hc
 

@@ -18,8 +18,8 @@ int main() {
         if (what == 'd') {
             const DownPlan p = plan_down(bits, f32, G, T, r, d, 256);
             const char *name[] = {"dots", "split", "tiles"};
-            std::printf("%s %d %ld %zu\n", name[(int)p.kernel], p.split, (long)split_blocks(kSplits[p.split], T, r),
-                        split_lds(kSplits[p.split], d, G));
+            std::printf("%s %d %ld %zu %d\n", name[(int)p.kernel], p.split, (long)split_blocks(kSplits[p.split], T, r),
+                        split_lds(kSplits[p.split], d, G), p.halves);
         } else {
             const UpPlan p = plan_up(bits, f32, T, d, r, 256);
             std::printf("%s%s 0 0 %zu\n", p.small ? "small" : "wide", p.two ? " two" : " one", up_lds(p.small ? 1 : 2, r, G));
@@ -52,7 +52,7 @@ def test_down_plans_can_run(plan):
     cases = [("d", bits, f32, G, T, R, d) for bits in (4, 8) for f32 in (0, 1) for G in (32, 64, 128)
              for T in (1, 2, 32, 33, 255, 256, 441, 1000, 4000, 65535) for R in (1, 20, 324, 1028)
              for d in (32, 96, 128, 160, 2560, 4096, 10240, 65536) if (4 * d) % G == 0]
-    for c, (kernel, split, blocks, lds) in zip(cases, plan(cases)):
+    for c, (kernel, split, blocks, lds, _) in zip(cases, plan(cases)):
         _, _, f32, _, T, _, d = c
         if kernel == "split":
             assert not f32 and T > 32 and int(lds) <= 159 * 1024, c
@@ -79,3 +79,12 @@ def test_streams_too_wide_for_the_split_go_to_the_cheaper_kernel(plan):
              (4, 32, 1000, 324, 8192), (4, 32, 40, 8, 65536), (4, 32, 1000, 324, 5152)]
     got = plan([("d", b, 0, G, T, R, d) for b, G, T, R, d in cases])
     assert [p[0] for p in got] == ["tiles"] * 5 + ["dots"] * 2
+
+
+def test_staged_tiles_take_k_in_halves_only_in_one_round_of_blocks(plan):
+    """Q4, BF16: two halves of K where the blocks are at most the CUs (and with groups of 32), one where two blocks share a CU;
+    one for Q8 and FP32 streams."""
+    cases = [(4, 0, 64, 2000, 324), (4, 0, 64, 4000, 388), (4, 0, 128, 2000, 772), (4, 0, 32, 4000, 388), (8, 0, 64, 2000, 324),
+             (4, 1, 64, 2000, 324)]
+    got = plan([("d", b, f, G, T, R, 2560) for b, f, G, T, R in cases])
+    assert [(p[0], p[4]) for p in got] == [("tiles", v) for v in "211211"]
