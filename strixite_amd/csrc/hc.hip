@@ -767,7 +767,7 @@ __global__ void __launch_bounds__(256)
 // ================================================================================================ up: MFMA tiles
 // WAVES column tiles of 16 positions j a block (a wave each), MT 16-token tiles; LDS: h as bf16 hi / mid / lo [16 MT][r + 8]
 // in the paired k order, then its group sums [r / G][16 MT] (FP32)
-// TWO: registers held to what lets two blocks share a CU, for grids of more blocks than CUs
+// TWO: registers held to what lets two blocks share a CU (hcp::plan_up says when)
 template <typename T, int BITS, int MT, int WAVES, bool TWO>
 __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2)))
     mix_up_tile_kernel(const float *h, const uint8_t *q, const uint16_t *scale, const uint16_t *minv, const T *x,
@@ -872,7 +872,7 @@ __global__ void __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per
 
     // a ring of kAhead chunks in flight: chunk c computes from slot c % kAhead, then that slot loads chunk c + kAhead
     // (8 for the 16-token tiles measured slower: 15.1 against 13.2 us at 1 token; two blocks a CU with 4 ahead spill: 99
-    // us at 2000 tokens, with 2 ahead 72, one block a CU with 4 ahead 81)
+    // us at 2000 tokens, r 320, Q4 g64, with 2 ahead 83, one block a CU with 4 ahead 91)
     constexpr int kAhead = TWO ? 2 : 4;
     Ahead ring[kAhead];
 #pragma unroll
@@ -1067,7 +1067,7 @@ void run_mix_up(const float *h, const Weights &w, const void *x, const float *no
     STRIX_CHECK(reinterpret_cast<uintptr_t>(h) % 16 == 0, what, ": h must start on a 16-byte boundary");
     const int64_t es = act == Act::F32 ? 4 : 2;
     STRIX_CHECK(disjoint(u, T * d * es, x, T * H * d * es), what, ": u and the streams x overlap");
-    const auto [small, two] = hcp::plan_up(BITS, act == Act::F32, T, d, w.K, device_cus());
+    const auto [small, two] = hcp::plan_up(BITS, act == Act::F32, T, d, w.K, w.G, device_cus());
     const int MT = small ? 1 : 2, WAVES = small ? 4 : 8;
     const size_t lds = hcp::up_lds(MT, w.K, w.G);
     const int64_t njb = (d / 16 + WAVES - 1) / WAVES, ntt = (T + 16 * MT - 1) / (16 * MT);

@@ -102,13 +102,17 @@ struct UpPlan {
 };
 
 // 16-token tiles of 4 waves a block up to 16 tokens, 32-token tiles of 8 waves above (the h tile shared by more
-// columns); 32-token tiles of h fit the LDS up to r = 768
-inline UpPlan plan_up(int bits, bool f32, int64_t T, int64_t d, int64_t r, int64_t cus) {
+// columns); 32-token tiles of h fit the LDS up to r = 768.
+// Two blocks a CU, at half the registers and a ring of two chunks: where there are more blocks than CUs and the LDS holds
+// two tiles of h (r about 410); Q8 only beside short rows and BF16 streams (its ring is twice the registers). Measured on
+// MI355X, d 2560, g 64, 2000 tokens, two / one, us: Q4 r 320 83 / 91, r 384 93 / 95, r 448 119 / 117, r 768 177 / 158, FP32
+// streams r 320 78 / 88, r 768 182 / 164; Q8 r 64 49 / 53, r 128 61 / 61, r 320 101 / 99, r 448 163 / 122, FP32 105 / 103.
+inline UpPlan plan_up(int bits, bool f32, int64_t T, int64_t d, int64_t r, int64_t G, int64_t cus) {
     const bool small = T <= 16 || r > 768;
     const int64_t MT = small ? 1 : 2, waves = small ? 4 : 8;
     const int64_t blocks = (d / 16 + waves - 1) / waves * ((T + 16 * MT - 1) / (16 * MT));
-    // (Q8 codes beside FP32 streams spill at two blocks a CU: 105 against 103 us at 2000 tokens)
-    return {small, !small && blocks > cus && !(bits == 8 && f32)};
+    const bool pays = bits == 4 || (!f32 && r <= 128);
+    return {small, !small && blocks > cus && pays && 2 * up_lds(2, r, G) <= 160 * 1024};
 }
 
 }  // namespace strix::kernels::hcp

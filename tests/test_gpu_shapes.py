@@ -219,7 +219,8 @@ def test_one_token_layer_matches_two(shared, bits, H, I, E, k):
 
 # u in BF16 is the FP32 u rounded once: the same gates, products and sums on BF16-valued streams in either dtype (a gate
 # a few 2^-24 off rounds some of these outputs the other way)
-@pytest.mark.parametrize("bits,G,T,d,r", [(4, 64, 700, 2560, 320), (8, 64, 600, 1024, 128), (4, 32, 9, 2560, 96)])
+@pytest.mark.parametrize("bits,G,T,d,r", [(4, 64, 700, 2560, 320), (8, 64, 600, 1024, 128), (4, 32, 9, 2560, 96),
+                                           (8, 64, 500, 2560, 128), (4, 64, 500, 2560, 512)])
 def test_mix_up_bf16_is_the_rounded_fp32(bits, G, T, d, r):
     say("mix up bf16", bits, G, T, d, r)
     x = _bf16(orc.gen_bf16_normal(orc.tensor_key(12, "x"), 1.0, (T, 4 * d)))
@@ -241,3 +242,26 @@ def test_layer_shared_expert_of_many_groups(M):
     o = orc.moe_layer(oracle_weights(layer), to_np(x)[:16])
     assert np.array_equal(to_np(out["ids"])[:16], o["ids"])
     assert rel_err(to_np(out["y"])[:16], o["y"]) < 1e-2  # the layer tests' tolerance
+
+
+# the up mix's variants: two blocks a CU and one, either format and dtype, ragged tokens, ranks on either side of the LDS
+# that two blocks leave, group counts past the min terms held in registers
+@pytest.mark.parametrize("bits,G,act,T,d,r", [(4, 64, "bf16", 497, 2560, 384), (4, 32, "f32", 497, 2560, 352),
+                                              (8, 64, "bf16", 515, 2560, 128), (8, 32, "f32", 515, 2560, 96),
+                                              (4, 64, "bf16", 431, 2560, 448), (8, 128, "bf16", 431, 2560, 768)])
+def test_mix_up_kernels(bits, G, act, T, d, r):
+    from oracle import hc
+
+    say("mix up", bits, G, act, T, d, r)
+    dt = torch.bfloat16 if act == "bf16" else torch.float32
+    rng = np.random.default_rng(T)
+    x = torch.from_numpy(rng.standard_normal((T, 4 * d)).astype(np.float32)).to(DEV).to(dt)
+    h, inv, nw = (torch.from_numpy(a.astype(np.float32)).to(DEV) for a in
+                  (rng.standard_normal((T, r)), rng.uniform(0.5, 1.5, (T, 4)), rng.standard_normal(4 * d) * 0.1))
+    q, s, m = orc.gen_q(bits, orc.tensor_key(82, "gu_q"), orc.tensor_key(82, "gu_s"), 4 * d, r, G)
+    w64 = hc.weights64(bits, q, s, m, 4 * d, r, G)
+    u = moe.hc_mix_up(h, moe.QWeight.from_host(bits, *hc.to_chunk_major(bits, q, s, m, 4 * d, r, G), 4 * d, r, G), x, nw, inv)
+    rows = np.unique(np.concatenate([np.arange(40), np.arange(T - 40, T)]))
+    np64 = [t.double().cpu().numpy() for t in (h, x, nw, inv)]
+    ref = hc.hc_mix_up(np64[0][rows], w64, np64[1][rows], np64[2], np64[3][rows], d)
+    assert _rel64(u[rows], ref) < (2.0 ** -8 if act == "bf16" else 1e-4)  # one rounding of u; the gates' sums in FP32

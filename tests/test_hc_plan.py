@@ -21,7 +21,7 @@ int main() {
             std::printf("%s %d %ld %zu %d\n", name[(int)p.kernel], p.split, (long)split_blocks(kSplits[p.split], T, r),
                         split_lds(kSplits[p.split], d, G), p.halves);
         } else {
-            const UpPlan p = plan_up(bits, f32, T, d, r, 256);
+            const UpPlan p = plan_up(bits, f32, T, d, r, G, 256);
             std::printf("%s%s 0 0 %zu\n", p.small ? "small" : "wide", p.two ? " two" : " one", up_lds(p.small ? 1 : 2, r, G));
         }
     }
@@ -88,3 +88,14 @@ def test_staged_tiles_take_k_in_halves_only_in_one_round_of_blocks(plan):
              (4, 1, 64, 2000, 324)]
     got = plan([("d", b, f, G, T, R, 2560) for b, f, G, T, R in cases])
     assert [(p[0], p[4]) for p in got] == [("tiles", v) for v in "211211"]
+
+
+def test_up_mix_shares_a_cu_only_where_the_lds_holds_two_blocks(plan):
+    """The two-block variant: more blocks than CUs, twice the h tile within the 160 KB LDS, and not where it measured slower."""
+    cases = [("u", bits, f32, G, T, r, 2560) for bits in (4, 8) for f32 in (0, 1) for G in (32, 64, 128)
+             for T in (16, 17, 500, 2000) for r in (128, 320, 384, 448, 512, 768, 896) if r % G == 0]
+    for c, (tile, blocks, _, _, lds) in zip(cases, plan(cases)):
+        _, bits, f32, _, T, r, _ = c
+        assert (tile == "small") == (T == 16 or r > 768), c
+        want = tile == "wide" and T >= 500 and r <= 384 and (bits == 4 or (not f32 and r <= 128))
+        assert (blocks == "two") == want and (not want or 2 * int(lds) <= 160 * 1024), c
