@@ -269,6 +269,10 @@ __device__ __forceinline__ RawItem load_raw(const GemmArgs &a, int64_t item, int
         const int32_t *rec = a.ws + route::t16_rec_at(a.S, a.E) + route::kRec16 * (int64_t)tile;
         r.expert = rec[0];
         r.my = rec[4 + j];
+    } else if constexpr (MODE == DENSE) {
+        const int32_t st = (int32_t)tile * 16, rows = a.M - st < 16 ? (int32_t)(a.M - st) : 16;
+        r.expert = 0;
+        r.my = j < rows ? st + j : -1;
     } else {
         r.expert = a.ids[tile];
         r.my = j == 0 ? (int32_t)tile : -1;
@@ -284,7 +288,7 @@ __device__ __forceinline__ Item<RT> make_item(const GemmArgs &a, const RawItem &
     it.valid = item < n_items;
     const uint32_t tile = (uint32_t)item / (uint32_t)col_blocks, cb = (uint32_t)item % (uint32_t)col_blocks;
     const int32_t id = __builtin_amdgcn_readfirstlane(raw.expert);
-    it.nan = id < 0 || id >= a.E;
+    it.nan = MODE != DENSE && (id < 0 || id >= a.E);
     const uint32_t expert = it.nan ? 0u : (uint32_t)id;
     it.expert = expert;
     if constexpr (MODE == PERSLOT) {
@@ -1184,9 +1188,9 @@ void launch_gemm_v(const GemmArgs &a, int64_t tiles_bound, const SharedJob &sh, 
     const int64_t blocks = std::max<int64_t>(1, std::min(want, cap)) + sh.blocks;
     // 32-bit buffer offsets: the weight view and the activations must each stay below 2 GiB
     const int64_t q_bytes = a.N * a.E * a.K * BITS / 8, s_bytes = a.N * a.E * (a.K / a.G) * 2;
-    const int64_t x_rows = MODE == GROUPED ? (XROW_DIV ? a.S / a.A : a.S) : (XROW_DIV ? a.M : a.M * a.A);
+    const int64_t x_rows = MODE == GROUPED ? (XROW_DIV ? a.S / a.A : a.S) : MODE == DENSE ? a.M : (XROW_DIV ? a.M : a.M * a.A);
     const int64_t x_bytes = x_rows * a.K * 2;
-    const int64_t y_rows = MODE == GROUPED ? a.S : a.M * a.A;
+    const int64_t y_rows = MODE == GROUPED ? a.S : MODE == DENSE ? a.M : a.M * a.A;
     const int64_t y_bytes = y_rows * a.ldy * (EPI == EPI_F32 ? 4 : 2);
     STRIX_CHECK(q_bytes < (1ll << 31) && s_bytes < (1ll << 31) && x_bytes < (1ll << 31) && y_bytes < (1ll << 31),
                 "expert kernels: weight (", q_bytes, " B), activation (", x_bytes, " B) or output (", y_bytes,
@@ -1770,6 +1774,15 @@ namespace {
 // stream kernel that walked K alone: 56), at 130 34 / 62, 200 41 / 62, 300 55 / 62, 500 72 / 62 (tiles for the down only:
 // 73); H 3072, I 2048, Q4 at 100 73 / 79, at 130 97 / 78.
 constexpr int64_t kDenseTileOutputs = 400000;
+// Groups of 32, which the GEMM does not take: past kDenseTileOutputs (at K up to 512, past 280000) and up to K 2048 the
+// stream kernel, whose waves walk K alone over 16 tokens x 32 rows: a short walk, and it converts a code once for both. From
+// there on the tiles' split of K makes up for it. Measured on MI355X, stream / tiles, us: Q4 K 512, N 3072 at 100 tokens
+// 12.0 / 14.4, at 500 23 / 40, at 2000 72 / 141; K 1024, N 4096 at 128 29 / 32, at 2000 394 / 457; K 2048, N 4096 (Q8) at 500
+// 201 / 207; K 3072, N 4096 at 700 440 / 405; within the tiles' range K 512, N 512 at 500 12.0 / 11.4, K 1024, N 1024 at 300
+// 29 / 25.
+bool dense_streams(int64_t M, int64_t N, int64_t K, int64_t G) {
+    return G == 32 && K <= 2048 && M * N > (K <= 512 ? 280000 : kDenseTileOutputs);
+}
 
 // y [M, N] = x [M, K] . dequant(W)^T for one Q4 or Q8 weight, FP32 accumulation, y stored in out_act
 void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64_t M, Act act, Act out_act,
@@ -1803,7 +1816,16 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
         };
         if (v.bits == 4) go(std::integral_constant<int, 4>{});
         else go(std::integral_constant<int, 8>{});
-    } else {
+    } else if (dense_streams(M, v.N, v.K, v.G)) {
+        auto go = [&](auto bits) {
+            constexpr int B = decltype(bits)::value;
+            const int64_t tiles = (M + 15) / 16;
+            if (out_act == Act::F32) launch_gemm_s<B, 32, DENSE, EPI_F32, false, false, false>(a, tiles, stream, nullptr);
+            else launch_gemm_s<B, 32, DENSE, EPI_BF16, false, false, false>(a, tiles, stream, nullptr);
+        };
+        if (v.bits == 4) go(std::integral_constant<int, 4>{});
+        else go(std::integral_constant<int, 8>{});
+} else {
         xt::Args t = tile_args(v, 1, x, y, v.N);
         t.A = 1, t.S = M;
         xt::project(v.bits, xt::DENSE, false, Act::BF16, out_act, t, stream);

@@ -108,7 +108,10 @@ def test_fp32_router_rows_match_bf16_bits():
 
 # dense BF16 on either side of the tiles' and the GEMM's sizes, with a remainder of the 16-token tiles
 @pytest.mark.parametrize("bits,G,M,N,K", [(8, 64, 17, 1040, 3072), (4, 128, 111, 96, 512), (8, 64, 113, 4096, 2048),
-                                          (4, 64, 300, 1024, 2048), (8, 32, 1, 16, 96)])
+                                          (4, 64, 300, 1024, 2048), (8, 32, 1, 16, 96),
+                                          # groups of 32 past the tiles' outputs: the stream kernel, up to K 2048
+                                          (4, 32, 555, 528, 512), (8, 32, 421, 992, 1024), (4, 32, 131, 3088, 2048),
+                                          (8, 32, 131, 3088, 2080)])
 def test_dense_tiles_and_gemm(bits, G, M, N, K):
     say("dense", bits, G, M, N, K)
     w = _weight(bits, N, K, G, 51)
