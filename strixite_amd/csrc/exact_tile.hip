@@ -227,47 +227,58 @@ __global__ void __launch_bounds__(kMaxWaves *kWave)
     }
 }
 
-// Block (token, column block), the token's slots one after another as exact_tile_kernel's one-row tiles (MFMA rows 0, 5
-// and 10 of an FP32 slot, row 0 of a BF16 one), their dots summed with the coefficients.
-template <int FMT, int SP, typename TX, int RT>
-__global__ void __launch_bounds__(kMaxWaves *kWave)
-    exact_perslot_combine_kernel(Args a, const float *coef, bool y_f32, int cbs, int bpt, int ks) {
-    __shared__ float4v red[2][kMaxWaves][RT][kWave];
+// Block (token, 16 output columns): ks waves split K of a slot, sg slots at a time (kCombineWaves waves at most), each as
+// exact_tile_kernel's one-row tile (MFMA rows 0, 5 and 10 of an FP32 slot, row 0 of a BF16 one), the slots' dots summed with
+// the coefficients in slot order. What bounds it: latency, a round of K's walk for every sg slots. Measured on MI355X, H
+// 3072, I 512, 10 slots a token, Q4 g128, FP32: 12 us at 1 token, 26 at 4 (a slot a round 44 and 47, a wave an output 20 and
+// 67).
+constexpr int kCombineWaves = 16;
+template <int FMT, int SP, typename TX>
+__global__ void __launch_bounds__(kCombineWaves *kWave)
+    exact_perslot_combine_kernel(Args a, const float *coef, bool y_f32, int cbs, int ks, int sg) {
+    constexpr bool F32 = std::is_same_v<TX, float>;
+    __shared__ float red[2][kCombineWaves][kWave];  // lane (g, j), g < 3: MFMA row 5 g of column j
+    __shared__ float cf[kWave];
+    __shared__ int32_t sid[kWave];
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int g = lane / 16, j = lane % 16, nw = (int)(blockDim.x / kWave);
-    const int64_t m = blockIdx.x / (uint32_t)bpt;
-    const int cb = (int)(blockIdx.x % (uint32_t)bpt) * (nw / ks) + (ks > 1 ? 0 : wave);
-    const int64_t c0 = (int64_t)cb * 16 * RT;
-    if (cb >= cbs) return;  // ks = 1 only (its waves meet no barrier)
-    const int spans = (int)(a.K / SP), part = ks > 1 ? wave : 0;
-    float out[RT] = {};
-    bool bad = false;
-    for (int64_t s = 0; s < a.A; ++s) {
-        const int64_t slot = m * a.A + s;
-        const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[slot]);
-        const bool nan = id < 0 || id >= a.E;
-        if (nan && blockIdx.x % (uint32_t)bpt == 0 && threadIdx.x == 0) report(a.err, id, slot);
-        bad = bad || nan;
-        const float cf = coef[slot];
-        float4v acc[RT];
-        tile_dot<FMT, SP, TX, RT>(a, tile_rows<FMT, false, RT>(a, nan ? 0 : id, c0),
-                                  static_cast<const TX *>(a.x) + slot * a.K, spans * part / ks, spans * (part + 1) / ks, acc);
-        float4v(&rb)[kMaxWaves][RT][kWave] = red[s & 1];  // two buffers: one barrier a slot
-#pragma unroll
-        for (int t = 0; t < RT; ++t) rb[wave][t][lane] = acc[t];
-        if (ks > 1) __syncthreads();
-        else {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-#pragma unroll
-        for (int t = 0; t < RT; ++t) out[t] = fmaf(cf, tile_sum<TX, RT>(rb, ks > 1 ? 0 : wave, ks, t, 0, j), out[t]);
+    const int g = lane / 16, j = lane % 16, sub = wave / ks, part = wave % ks, A = (int)a.A;
+    const int64_t m = blockIdx.x / (uint32_t)cbs, c0 = (int64_t)(blockIdx.x % (uint32_t)cbs) * 16;
+    if ((int)threadIdx.x < A) {  // A is at most 64: the first wave
+        sid[threadIdx.x] = a.ids[m * A + threadIdx.x];
+        cf[threadIdx.x] = coef[m * A + threadIdx.x];
     }
-    if (g != 0 || (ks > 1 && wave != 0)) return;
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-        if (c0 + 16 * t + j < a.ncol) store(a, y_f32, m, c0 + 16 * t + j, bad ? qnan() : out[t]);
+    const int spans = (int)(a.K / SP);
+    float out = 0.f;
+    bool bad = false;
+    for (int s0 = 0, round = 0; s0 < A; s0 += sg, ++round) {
+        float(&rb)[kCombineWaves][kWave] = red[round & 1];  // two buffers: one barrier a round
+        if (s0 + sub < A) {
+            const int64_t slot = m * A + s0 + sub;
+            const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[slot]);
+            float4v acc[1];
+            tile_dot<FMT, SP, TX, 1>(a, tile_rows<FMT, false, 1>(a, id < 0 || id >= a.E ? 0 : id, c0),
+                                     static_cast<const TX *>(a.x) + slot * a.K, spans * part / ks, spans * (part + 1) / ks,
+                                     acc);
+            rb[wave][lane] = g == 0 ? acc[0][0] : g == 1 ? acc[0][1] : acc[0][2];
+        }
+        __syncthreads();
+        if (threadIdx.x >= 16) continue;
+        for (int s = 0; s < sg && s0 + s < A; ++s) {
+            auto row_sum = [&](int i) {  // the parts in wave order
+                float v = rb[s * ks][i];
+                for (int w = 1; w < ks; ++w) v += rb[s * ks + w][i];
+                return v;
+            };
+            float v = row_sum(j);
+            if constexpr (F32) v += row_sum(16 + j) + row_sum(32 + j);
+            out = fmaf(cf[s0 + s], v, out);
+            const int32_t id = sid[s0 + s];
+            const bool nan = id < 0 || id >= a.E;
+            if (nan && !bad && c0 == 0 && threadIdx.x == 0) report(a.err, id, m * A + s0 + s);  // the token's first
+            bad = bad || nan;
+        }
+    }
+    if (threadIdx.x < 16 && c0 + j < a.ncol) store(a, y_f32, m, c0 + j, bad ? qnan() : out);
 }
 
 // One token: block (16 output columns), a wave a slot over all of K; the slots' dots meet in LDS. What bounds it: latency
@@ -366,18 +377,18 @@ void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &
 }
 
 void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStream_t stream) {
+    const int64_t cbs = (a.ncol + 15) / 16;
+    STRIX_CHECK(a.A >= 1 && a.A <= kWave && a.S * cbs < (1ll << 31), "exact per-slot combine: ", a.S, " tokens of ", a.A,
+                " slots, ", a.ncol, " columns");
     by_format(fmt, a.G, [&](auto fc, auto sc) {
-        constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value, RT = 2;
-        const int ks = split_of(a.K / SP), nw = ks > 1 ? ks : 4;
-        const int64_t cbs = (a.ncol + 16 * RT - 1) / (16 * RT), bpt = ks > 1 ? cbs : (cbs + nw - 1) / nw;
-        STRIX_CHECK(a.S * bpt < (1ll << 31), "exact per-slot combine: ", a.S, " x ", a.ncol, " outputs, too many");
-        const unsigned blocks = (unsigned)(a.S * bpt);
-        if (act == Act::F32)
-            exact_perslot_combine_kernel<FMT, SP, float, RT>
-                <<<blocks, nw * kWave, 0, stream>>>(a, coef, true, (int)cbs, (int)bpt, ks);
-        else
-            exact_perslot_combine_kernel<FMT, SP, uint16_t, RT>
-                <<<blocks, nw * kWave, 0, stream>>>(a, coef, false, (int)cbs, (int)bpt, ks);
+        constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value;
+        const int ks = split_of(a.K / SP), sg = (int)std::min<int64_t>(a.A, kCombineWaves / ks);
+        auto go = [&](auto tx) {
+            exact_perslot_combine_kernel<FMT, SP, decltype(tx)>
+                <<<(unsigned)(a.S * cbs), ks * sg * kWave, 0, stream>>>(a, coef, act == Act::F32, (int)cbs, ks, sg);
+        };
+        if (act == Act::F32) go(float{});
+        else go(uint16_t{});
     });
 }
 

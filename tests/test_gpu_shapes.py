@@ -268,3 +268,29 @@ def test_mix_up_kernels(bits, G, act, T, d, r):
     np64 = [t.double().cpu().numpy() for t in (h, x, nw, inv)]
     ref = hc.hc_mix_up(np64[0][rows], w64, np64[1][rows], np64[2], np64[3][rows], d)
     assert _rel64(u[rows], ref) < (2.0 ** -8 if act == "bf16" else 1e-4)  # one rounding of u; the gates' sums in FP32
+
+
+# the per-slot combine: K whole, split over 4 and over 8 waves, slots within one round of waves and past it, a ragged
+# column end; the grouped combine's bits, float64, the first invalid id of a token reported
+@pytest.mark.parametrize("G,K,A,N", [(128, 512, 17, 48), (128, 512, 5, 16), (128, 1024, 9, 32), (32, 1024, 3, 80)])
+def test_perslot_combine_rounds(G, K, A, N):
+    say("per-slot combine", G, K, A, N)
+    M, E = 3, 24
+    w = _weight(4, E * N, K, G, 91)
+    w64 = _w64(w)
+    rng = np.random.default_rng(K + A)
+    h = torch.from_numpy(rng.standard_normal((M * A, K)).astype(np.float32)).to(DEV)
+    coef = torch.from_numpy(rng.random((M, A)).astype(np.float32)).to(DEV)
+    ids = np.stack([rng.permutation(E)[:A] for _ in range(M)]).astype(np.int32)
+    ids[1, A - 2], ids[1, A - 1] = E, -1
+    tid = torch.from_numpy(ids).to(DEV)
+    ws, _ = moe.moe_group_routes(tid, E)
+    err = moe.zero_err()
+    y = moe.experts_combine(h, w, E, tid, coef, err)
+    yg = moe.experts_combine_grouped(h, w, E, tid, coef, ws, M, A)
+    assert err.cpu().numpy().tolist() == [1, E, A + A - 2]
+    assert torch.isnan(y[1]).all() and torch.equal(torch.nan_to_num(y, nan=7.0), torch.nan_to_num(yg, nan=7.0))
+    h64, c64 = h.double().cpu().numpy(), coef.double().cpu().numpy()
+    for m in (0, 2):
+        ref = sum(c64[m, a] * (h64[m * A + a] @ w64[ids[m, a] * N:(ids[m, a] + 1) * N].T) for a in range(A))
+        assert _rel64(y[m], ref) < 2e-5  # exact products, FP32 sums whose terms reach a few times the result
