@@ -312,6 +312,112 @@ __global__ void __launch_bounds__(kOneTokenSlots *kWave)
     if (out != nullptr) out[c0 + j] = f32_to_bf16(bf16_to_f32(xr) + bf16_to_f32(y));
 }
 
+// ---- small calls: a wave an output element ------------------------------------------------------------------------------
+// Lane l takes the row's 32-code chunks l, l + 64, ...: acc = s (x . codes) + m sum(x) a chunk, FP32 with fmaf, the codes
+// about the middle of their range as in the tiles, then a butterfly over the lanes. Every load of a row is in flight at once, so a call whose outputs do not fill the chip costs one
+// round trip, where a tile's waves walk K two steps at a time; a row's codes are converted once an output, so its time grows
+// with the outputs from there (lanes_take).
+template <int FMT> struct ChunkCodes {
+    static constexpr int W = FMT == 5 ? 4 : FMT;
+    uint32_t w[W], hi;
+    // chunk c of the row at p (FMT 5: low plane [K / 2], then bit 4 of code k at bit k % 8 of byte k / 8)
+    __device__ __forceinline__ void load(const uint8_t *p, int64_t K, int64_t c) {
+#pragma unroll
+        for (int i = 0; i < W / 4; ++i) {
+            const uint4 u = *reinterpret_cast<const uint4 *>(p + c * (4 * W) + 16 * i);
+            w[4 * i] = u.x, w[4 * i + 1] = u.y, w[4 * i + 2] = u.z, w[4 * i + 3] = u.w;
+        }
+        if constexpr (FMT == 5) hi = *reinterpret_cast<const uint32_t *>(p + K / 2 + c * 4);
+    }
+    __device__ __forceinline__ float code(int i) const {
+        constexpr int bits = FMT == 8 ? 8 : 4, per = 32 / bits;
+        uint32_t n = (w[i / per] >> (bits * (i % per))) & ((1u << bits) - 1u);
+        if constexpr (FMT == 5) n |= ((hi >> i) & 1u) << 4;
+        return (float)n - Fmt<FMT, 32>::MID;  // exact
+    }
+};
+
+// the dot of an activation row with a weight row, in every lane
+template <int FMT, typename TX> __device__ __forceinline__ float lane_dot(const Args &a, const TX *xr, int64_t wrow) {
+    const int64_t row_bytes = FMT == 8 ? a.K : FMT == 4 ? a.K / 2 : a.K / 2 + a.K / 8, groups = a.K / a.G;
+    float acc = 0.f;
+    for (int64_t c = threadIdx.x % kWave; c < a.K / 32; c += kWave) {
+        ChunkCodes<FMT> cc;
+        cc.load(a.q + wrow * row_bytes, a.K, c);
+        const int64_t gi = wrow * groups + c * 32 / a.G;
+        const float s = bf16_to_f32(a.scale[gi]), m = fmaf(Fmt<FMT, 32>::MID, s, bf16_to_f32(a.minv[gi]));
+        float dot[4], xs[4];  // eight codes each: short chains of roundings
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            float v[8];
+            if constexpr (std::is_same_v<TX, float>) {
+                const float4 u = *reinterpret_cast<const float4 *>(xr + c * 32 + 8 * p),
+                             w = *reinterpret_cast<const float4 *>(xr + c * 32 + 8 * p + 4);
+                v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = w.x, v[5] = w.y, v[6] = w.z, v[7] = w.w;
+            } else {
+                const uint4 u = *reinterpret_cast<const uint4 *>(xr + c * 32 + 8 * p);
+                const uint32_t d[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(i % 2 ? d[i / 2] & 0xffff0000u : d[i / 2] << 16);
+            }
+            dot[p] = v[0] * cc.code(8 * p), xs[p] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+#pragma unroll
+            for (int i = 1; i < 8; ++i) dot[p] = fmaf(v[i], cc.code(8 * p + i), dot[p]);
+        }
+        acc = fmaf(s, (dot[0] + dot[1]) + (dot[2] + dot[3]), fmaf(m, (xs[0] + xs[1]) + (xs[2] + xs[3]), acc));
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kWave);
+    return acc;
+}
+
+constexpr int kLaneBlock = 256;
+
+// output row r of a grouped workspace is position r: its bucket by bisection of the offsets
+template <int FMT, bool SWI, typename TX>
+__global__ void __launch_bounds__(kLaneBlock) lane_rows_kernel(Args a, int mode, bool y_f32) {
+    const uint32_t item = blockIdx.x * (kLaneBlock / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (item >= (uint32_t)(a.S * a.ncol)) return;  // whole wave; no barrier in this kernel (lanes_take: few outputs)
+    const uint32_t r = item / (uint32_t)a.ncol, j = item % (uint32_t)a.ncol;
+    uint32_t row = r;  // DENSE: A is 1
+    int32_t expert = 0;
+    if (mode == GROUPED) {
+        int32_t lo = 0, hi = (int32_t)a.E;  // buckets 0 .. E (E: invalid ids)
+        while (lo < hi) {
+            const int32_t mid = (lo + hi + 1) / 2;
+            if (a.ws[4 + mid] <= (int32_t)r) lo = mid;
+            else hi = mid - 1;
+        }
+        row = (uint32_t)a.ws[route::Layout{a.S, a.E, 0, 0, 0}.slots() + r], expert = lo;
+    } else if (mode == PERSLOT) {
+        expert = a.ids[r];
+        if ((expert < 0 || expert >= a.E) && j == 0 && threadIdx.x % kWave == 0) report(a.err, expert, r);
+    }
+    const bool nan = expert < 0 || expert >= a.E;
+    const int64_t w0 = (nan ? 0 : expert) * a.N + j;
+    const TX *xr = static_cast<const TX *>(a.x) + (int64_t)(row / (uint32_t)a.A) * a.K;
+    float v = lane_dot<FMT, TX>(a, xr, w0);
+    if constexpr (SWI) v = silu(v) * lane_dot<FMT, TX>(a, xr, w0 + a.ncol);
+    if (threadIdx.x % kWave == 0) store(a, y_f32, row, j, nan ? qnan() : v);
+}
+
+template <int FMT, typename TX>
+__global__ void __launch_bounds__(kLaneBlock) lane_perslot_combine_kernel(Args a, const float *coef, bool y_f32) {
+    const uint32_t item = blockIdx.x * (kLaneBlock / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (item >= (uint32_t)(a.S * a.ncol)) return;  // whole wave; no barrier in this kernel
+    const int64_t m = item / (uint32_t)a.ncol, n = item % (uint32_t)a.ncol;
+    float out = 0.f;
+    bool bad = false;
+    for (int64_t slot = m * a.A; slot < (m + 1) * a.A; ++slot) {
+        const int32_t id = a.ids[slot];
+        const bool nan = id < 0 || id >= a.E;
+        if (nan && n == 0 && threadIdx.x % kWave == 0) report(a.err, id, slot);
+        bad = bad || nan;
+        out = fmaf(coef[slot], lane_dot<FMT, TX>(a, static_cast<const TX *>(a.x) + slot * a.K, (nan ? 0 : id) * a.N + n), out);
+    }
+    if (threadIdx.x % kWave == 0) store(a, y_f32, m, n, bad ? qnan() : out);
+}
+
 int device_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -342,9 +448,41 @@ template <typename F> void by_format(int fmt, int64_t G, F &&f) {
     }
 }
 
+// Whether a call is small enough for a wave an output element (dots: outputs, FP32 SwiGLU's twice; BF16: Q5 only, the dense
+// BF16 calls' tiles being faster at every size). That form's time grows with dots x (K + 600), the tiles' with the K steps a
+// wave walks (about 0.9 us each, 1.5 where eight waves split K), from about one start each. Measured on MI355X, wave / tiles,
+// us: dense FP32, Q4 g128, N 1024, K 3072 at 4 tokens 9.9 / 12.2, at 8 16 / 13.6; N 3072, K 512 at 2 6.3 / 8.2, at 6 11.8 /
+// 10.2; N 4096, K 4096 at 1 11 / 13, at 2 19 / 14; Q4 g32, N 1024, K 3072 at 12 23 / 27, at 16 28 / 27; Q8 g64, N 640, K 5120
+// at 12 24 / 28, at 16 29 / 28; FP32 gate_up of 4 slots, H 2048, I 512, Q8 8.1 / 12.4, of 16 23 / 22; BF16 Q5 of 8 slots
+// 8.8 / 9.9. By the slots' count and the shape alone, so that a per-slot call and a grouped one take the same form (the same
+// bits). Error against 64 bits (2-norm, FP32): 0.9e-7 to 1.1e-7, the tiles 0.6e-7 to 1.3e-7.
+bool lanes_take(int fmt, Act act, int64_t K, int64_t G, int64_t dots) {
+    if (act != Act::F32 && fmt != 5) return false;
+    const int64_t span = fmt == 8 ? std::min<int64_t>(G, 64) : G, spans = K / span, ks = split_of(spans);
+    return dots < (1 << 24) && dots * (K + 600) < 400000 * (4 + (spans + ks - 1) / ks * (ks == 8 ? 15 : 9));
+}
+template <typename F> void by_lanes(int fmt, Act act, F &&f) {
+    using std::integral_constant;
+    auto by_act = [&](auto fc) {
+        if (act == Act::F32) f(fc, float{});
+        else f(fc, uint16_t{});
+    };
+    if (fmt == 5) by_act(integral_constant<int, 5>{});
+    else if (fmt == 4) f(integral_constant<int, 4>{}, float{});  // BF16: Q5 only (lanes_take)
+    else f(integral_constant<int, 8>{}, float{});
+}
+
 }  // namespace
 
 void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &a, hipStream_t stream) {
+    if (lanes_take(fmt, x_act, a.K, a.G, a.S * a.ncol * (swiglu && x_act == Act::F32 ? 2 : 1))) {
+        const unsigned blocks = (unsigned)((a.S * a.ncol + kLaneBlock / kWave - 1) / (kLaneBlock / kWave));
+        return by_lanes(fmt, x_act, [&](auto fc, auto tx) {
+            auto k = swiglu ? lane_rows_kernel<decltype(fc)::value, true, decltype(tx)>
+                            : lane_rows_kernel<decltype(fc)::value, false, decltype(tx)>;
+            k<<<blocks, kLaneBlock, 0, stream>>>(a, (int)mode, y_act == Act::F32);
+        });
+    }
     const int64_t tr = x_act == Act::F32 ? tile_rows_of<float>() : tile_rows_of<uint16_t>();
     const int64_t tiles = mode == GROUPED ? std::min(a.S, a.S / 16 + a.E + 2) : mode == DENSE ? (a.S + tr - 1) / tr : a.S;
     by_format(fmt, a.G, [&](auto fc, auto sc) {
@@ -377,6 +515,13 @@ void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &
 }
 
 void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStream_t stream) {
+    if (lanes_take(fmt, act, a.K, a.G, a.S * a.A * a.ncol)) {  // as the grouped down of the same slots
+        const unsigned blocks = (unsigned)((a.S * a.ncol + kLaneBlock / kWave - 1) / (kLaneBlock / kWave));
+        return by_lanes(fmt, act, [&](auto fc, auto tx) {
+            lane_perslot_combine_kernel<decltype(fc)::value, decltype(tx)>
+                <<<blocks, kLaneBlock, 0, stream>>>(a, coef, act == Act::F32);
+        });
+    }
     const int64_t cbs = (a.ncol + 15) / 16;
     STRIX_CHECK(a.A >= 1 && a.A <= kWave && a.S * cbs < (1ll << 31), "exact per-slot combine: ", a.S, " tokens of ", a.A,
                 " slots, ", a.ncol, " columns");

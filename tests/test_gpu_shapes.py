@@ -294,3 +294,38 @@ def test_perslot_combine_rounds(G, K, A, N):
     for m in (0, 2):
         ref = sum(c64[m, a] * (h64[m * A + a] @ w64[ids[m, a] * N:(ids[m, a] + 1) * N].T) for a in range(A))
         assert _rel64(y[m], ref) < 2e-5  # exact products, FP32 sums whose terms reach a few times the result
+
+
+# the wave an output element of small calls and the tiles, on either side of the line between them: FP32 dense (K of one and
+# several rounds of the lanes, a ragged last one, each format), and Q5 experts in BF16 grouped and per slot
+@pytest.mark.parametrize("bits,G,K,N,M", [(4, 128, 128, 16, 1), (4, 64, 2112, 48, 9), (4, 64, 2112, 48, 90), (8, 64, 4160, 32, 3),
+                                          (8, 32, 96, 64, 40), (8, 64, 512, 1024, 1), (8, 64, 512, 1024, 30)])
+def test_small_fp32_dense(bits, G, K, N, M):
+    say("small fp32 dense", bits, G, K, N, M)
+    w = _weight(bits, N, K, G, 95)
+    x = torch.from_numpy(np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)).to(DEV)
+    ref = x.double().cpu().numpy() @ _w64(w).T
+    lin = moe.linear_q4 if bits == 4 else moe.linear_q8
+    y = lin(x, w, out_dtype=torch.float32)
+    assert _rel64(y, ref) < 2e-5  # FP32 sums of up to 4160 terms
+    assert torch.equal(lin(x, w, out_dtype=torch.bfloat16), y.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,A", [(1, 3), (40, 3)])
+def test_small_q5_bf16_experts(M, A):
+    from oracle import q5
+
+    say("small q5", M, A)
+    E, H, I = 8, 2176, 64
+    N = E * 2 * I
+    q, s, m = q5.quantize((np.random.default_rng(1).standard_normal((N, H)) * 0.05).astype(np.float32), 128)
+    gu, g64 = moe.QWeight.from_host(5, q, s, m, N, H, 128), q5.weights64(q, s, m, N, H, 128)
+    x = _bf16(orc.gen_bf16_normal(orc.tensor_key(13, "x"), 1.0, (M, H)))
+    ids = np.stack([np.random.default_rng(m).permutation(E)[:A] for m in range(M)]).astype(np.int32)
+    tid = torch.from_numpy(ids).to(DEV)
+    ws, _ = moe.moe_group_routes(tid, E)
+    h = moe.experts_gather_grouped_swiglu(x, gu, E, ws, M, A)
+    X = x.double().cpu().numpy()
+    z = np.stack([X[s // A] @ g64[e * 2 * I:(e + 1) * 2 * I].T for s, e in enumerate(ids.ravel())])
+    assert _rel64(h, z[:, :I] / (1 + np.exp(-z[:, :I])) * z[:, I:]) < 2.0 ** -8  # one BF16 rounding
+    assert torch.equal(moe.experts_gather(x, gu, E, tid, moe.zero_err(), swiglu=True), h)
