@@ -185,10 +185,9 @@ __global__ void __launch_bounds__(kThreads)
 // (one round trip for the row and its MR tokens), and the waves of a block share a weight row through L1. VEC: K % 8 == 0
 // and 16-byte aligned rows; else element loads. Measured on MI355X at M 40, N 513, K 3072: 20 us (a wave a token and
 // row with element loads: 178).
-template <typename TY, int MR, bool VEC>
+template <typename TY, int MR, bool VEC, int NB = 2>
 __global__ void __launch_bounds__(kThreads)
     router_f32x_kernel(const float *x, const uint16_t *w, TY *y, int64_t M, int64_t N, int64_t K) {
-    constexpr int NB = 2;
     const int lane = threadIdx.x % kWave;
     const int64_t groups = (M + MR - 1) / MR, item = (int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave;
     if (item >= N * groups) return;  // whole wave; no barrier in this kernel
@@ -200,6 +199,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int64_t c = cb + (int64_t)b * kWave < chunks ? cb + (int64_t)b * kWave : cb;  // past the end: not added
+            [[maybe_unused]] const int left = (int)(K - c * 8 < 8 ? K - c * 8 : 8);  // a ragged end re-reads, adds not
             if constexpr (VEC) {
                 const uint4 u = *reinterpret_cast<const uint4 *>(wr + c * 8);
                 const uint32_t d[4] = {u.x, u.y, u.z, u.w};
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kThreads)
                 for (int i = 0; i < 8; ++i) wv[b][i] = __uint_as_float(i % 2 ? d[i / 2] & 0xffff0000u : d[i / 2] << 16);
             } else {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) wv[b][i] = c * 8 + i < K ? bf16_to_f32(wr[c * 8 + i]) : 0.f;
+                for (int i = 0; i < 8; ++i) wv[b][i] = bf16_to_f32(wr[c * 8 + (i < left ? i : 0)]);
             }
 #pragma unroll
             for (int r = 0; r < MR; ++r) {
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kThreads)
                     for (int i = 0; i < 8; ++i) xv[r][b][i] = e[i];
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) xv[r][b][i] = c * 8 + i < K ? xr[i] : 0.f;
+                    for (int i = 0; i < 8; ++i) xv[r][b][i] = xr[i < left ? i : 0];
                 }
             }
         }
@@ -227,11 +227,12 @@ __global__ void __launch_bounds__(kThreads)
         for (int b = 0; b < NB; ++b) {
             const int64_t c = cb + (int64_t)b * kWave;
             if (c >= chunks) break;
+            [[maybe_unused]] const int left = (int)(K - c * 8 < 8 ? K - c * 8 : 8);
 #pragma unroll
             for (int r = 0; r < MR; ++r)
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    if (VEC || c * 8 + i < K) acc[r] = fmaf(xv[r][b][i], wv[b][i], acc[r]);
+                    if (VEC || i < left) acc[r] = fmaf(xv[r][b][i], wv[b][i], acc[r]);
         }
     }
 #pragma unroll
@@ -250,15 +251,19 @@ __global__ void __launch_bounds__(kThreads)
 template <typename TY>
 void launch_router_f32x(const float *x, const uint16_t *w, TY *y, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
     const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
-    auto go = [&](auto mr) {
-        constexpr int MR = decltype(mr)::value;
-        const int64_t blocks = (N * ((M + MR - 1) / MR) + kThreads / kWave - 1) / (kThreads / kWave);
+    auto go = [&](auto kern, int64_t mr) {
+        const int64_t blocks = (N * ((M + mr - 1) / mr) + kThreads / kWave - 1) / (kThreads / kWave);
         STRIX_CHECK(blocks < (1ll << 31), "linear_bf16w: M = ", M, ", N = ", N, " too large for the FP32-activation path");
-        if (vec) router_f32x_kernel<TY, MR, true><<<(unsigned)blocks, kThreads, 0, stream>>>(x, w, y, M, N, K);
-        else router_f32x_kernel<TY, MR, false><<<(unsigned)blocks, kThreads, 0, stream>>>(x, w, y, M, N, K);
+        kern<<<(unsigned)blocks, kThreads, 0, stream>>>(x, w, y, M, N, K);
     };
-    if (M == 1) go(std::integral_constant<int, 1>{});
-    else go(std::integral_constant<int, 4>{});
+    // Element loads: a token a wave and a chunk at a time until the waves fill the chip (four tokens' elements are a longer
+    // chain of loads, and two chunks' are no fewer). Measured on MI355X, us, one token a wave / four: N 65, K 1003, 4 tokens
+    // 5.9 / 12.1, 16 8.3 / 12.2, 300 56 / 44; N 64, K 2044, 16 tokens 8.4 / 20.5, 40 19 / 21; N 513, K 3071, 16 73 / 74, 40 168 /
+    // 143.
+    if (!vec && M * N <= 8192) go(router_f32x_kernel<TY, 1, false, 1>, 1);
+    else if (!vec) go(router_f32x_kernel<TY, 4, false>, 4);
+    else if (M == 1) go(router_f32x_kernel<TY, 1, true>, 1);
+    else go(router_f32x_kernel<TY, 4, true>, 4);
 }
 
 template <typename TY>

@@ -99,7 +99,7 @@ def test_fp32_router_rows_match_bf16_bits():
     say("fp32 router")
     # FP32 x holding BF16 values: the canonical order's bits, with token counts around the four-token groups, chunk
     # counts that leave lanes without a last chunk, and rows that are not 16-byte aligned
-    for M, N, K in [(1, 33, 2560), (2, 5, 520), (5, 17, 1000), (9, 4, 1003)]:
+    for M, N, K in [(1, 33, 2560), (2, 5, 520), (5, 17, 1000), (9, 4, 1003), (130, 65, 1003)]:
         rng = np.random.default_rng(M)
         x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
         w = torch.from_numpy(rng.standard_normal((N, K)).astype(np.float32)).to(DEV).to(torch.bfloat16)
