@@ -13,6 +13,7 @@
 // A span (Q4: 128 codes, Q8: 64) never crosses a group: Q4 needs G = 128, Q8 G = 64 or 128 (the reference's
 // served layout: q4g128, q8g64).
 #include "common.hpp"
+#include "dense_plan.hpp"
 #include "exact_tile.hpp"
 #include "lds_grant.hpp"
 #include "route_small.hpp"
@@ -1767,23 +1768,6 @@ void swiglu(const void *gu, void *h, int64_t rows, int64_t I, Act act, hipStream
 }
 
 namespace {
-// Dense projections of fewer than 64 tokens, or of M N up to this, take the exact 16-row tiles (K split over a block's
-// waves), larger ones the LDS-tiled GEMM of 64-token tiles. The GEMM's blocks walk K alone, a time in proportion to K
-// until they fill the chip; the tiles convert the weights' codes once for 16 tokens, a time in proportion to M N K.
-// Measured on MI355X (gate_up + SwiGLU + down of one FFN, tiles / GEMM): H 3072, I 512, Q8 g64 at 100 tokens 26 us (the
-// stream kernel that walked K alone: 56), at 130 34 / 62, 200 41 / 62, 300 55 / 62, 500 72 / 62 (tiles for the down only:
-// 73); H 3072, I 2048, Q4 at 100 73 / 79, at 130 97 / 78.
-constexpr int64_t kDenseTileOutputs = 400000;
-// Groups of 32, which the GEMM does not take: past kDenseTileOutputs (at K up to 512, past 280000) and up to K 2048 the
-// stream kernel, whose waves walk K alone over 16 tokens x 32 rows: a short walk, and it converts a code once for both. From
-// there on the tiles' split of K makes up for it. Measured on MI355X, stream / tiles, us: Q4 K 512, N 3072 at 100 tokens
-// 12.0 / 14.4, at 500 23 / 40, at 2000 72 / 141; K 1024, N 4096 at 128 29 / 32, at 2000 394 / 457; K 2048, N 4096 (Q8) at 500
-// 201 / 207; K 3072, N 4096 at 700 440 / 405; within the tiles' range K 512, N 512 at 500 12.0 / 11.4, K 1024, N 1024 at 300
-// 29 / 25.
-bool dense_streams(int64_t M, int64_t N, int64_t K, int64_t G) {
-    return G == 32 && K <= 2048 && M * N > (K <= 512 ? 280000 : kDenseTileOutputs);
-}
-
 // y [M, N] = x [M, K] . dequant(W)^T for one Q4 or Q8 weight, FP32 accumulation, y stored in out_act
 void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64_t M, Act act, Act out_act,
                       hipStream_t stream) {
@@ -1808,7 +1792,9 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
     STRIX_CHECK(disjoint(y, M * v.N * oes, x, M * v.K * 2), fn, ": y overlaps x");
     GemmArgs a = make_args(v, 1, x, y, v.N);
     a.M = M;
-    if (M >= 64 && M * v.N > kDenseTileOutputs && v.K % gemm::BK == 0 && v.G % gemm::BK == 0 && v.K / v.G <= gemm::kMaxGroups) {
+    const bool gemm_ok = v.K % gemm::BK == 0 && v.G % gemm::BK == 0 && v.K / v.G <= gemm::kMaxGroups;
+    const dnp::Dense kernel = dnp::plan(v.bits, v.G, M, v.N, v.K, out_act == Act::F32, gemm_ok);
+    if (kernel == dnp::Dense::Gemm) {
         auto go = [&](auto bits) {
             constexpr int B = decltype(bits)::value;
             if (out_act == Act::F32) launch_expert_gemm<B, DENSE, EPI_F32, false, false>(a, stream);
@@ -1816,16 +1802,10 @@ void dense_projection(const char *fn, const QV &v, const void *x, void *y, int64
         };
         if (v.bits == 4) go(std::integral_constant<int, 4>{});
         else go(std::integral_constant<int, 8>{});
-    } else if (dense_streams(M, v.N, v.K, v.G)) {
-        auto go = [&](auto bits) {
-            constexpr int B = decltype(bits)::value;
-            const int64_t tiles = (M + 15) / 16;
-            if (out_act == Act::F32) launch_gemm_s<B, 32, DENSE, EPI_F32, false, false, false>(a, tiles, stream, nullptr);
-            else launch_gemm_s<B, 32, DENSE, EPI_BF16, false, false, false>(a, tiles, stream, nullptr);
-        };
-        if (v.bits == 4) go(std::integral_constant<int, 4>{});
-        else go(std::integral_constant<int, 8>{});
-} else {
+    } else if (kernel == dnp::Dense::Stream) {
+        if (out_act == Act::F32) launch_bits<DENSE, EPI_F32, false, false, false>(v.bits, a, (M + 15) / 16, stream);
+        else launch_bits<DENSE, EPI_BF16, false, false, false>(v.bits, a, (M + 15) / 16, stream);
+    } else {
         xt::Args t = tile_args(v, 1, x, y, v.N);
         t.A = 1, t.S = M;
         xt::project(v.bits, xt::DENSE, false, Act::BF16, out_act, t, stream);

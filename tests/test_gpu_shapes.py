@@ -122,6 +122,22 @@ def test_dense_tiles_and_gemm(bits, G, M, N, K):
     assert _rel64(lin(x, w), ref) < 2.0 ** -8  # one BF16 rounding
 
 
+# each kernel that dense_plan.hpp chooses from, at ragged tokens and columns: the stream kernel of each format and group size
+# past the tiles' outputs, the GEMM (Q4 and Q8, groups of one and two K steps, its tokens' and columns' remainders)
+@pytest.mark.parametrize("bits,G,M,N,K", [(8, 64, 85, 4112, 1024), (4, 64, 113, 4096, 1024), (8, 128, 77, 4112, 2048),
+                                          (4, 128, 100, 4112, 2048), (4, 64, 70, 8208, 1024), (4, 64, 333, 2064, 1088),
+                                          (4, 128, 300, 4112, 1024), (8, 64, 700, 1040, 1088), (8, 128, 400, 2064, 2176)])
+def test_dense_stream_and_gemm(bits, G, M, N, K):
+    say("dense plan", bits, G, M, N, K)
+    w = _weight(bits, N, K, G, 52)
+    x = _bf16(orc.gen_bf16_normal(orc.tensor_key(14, "x"), 1.0, (M, K)))
+    rows = np.unique(np.concatenate([np.arange(min(M, 20)), np.arange(max(0, M - 20), M)]))
+    ref = x.double().cpu().numpy()[rows] @ _w64(w).T
+    lin = moe.linear_q4 if bits == 4 else moe.linear_q8
+    assert _rel64(lin(x, w, out_dtype=torch.float32)[rows], ref) < 1e-4  # FP32 sums; Q4 codes carry an offset of 128
+    assert _rel64(lin(x, w)[rows], ref) < 2.0 ** -8  # one BF16 rounding
+
+
 # the exact GEMM's blocks dealt to the XCDs in runs: item counts around multiples of 8, one bucket of all the slots,
 # an empty one, ragged columns, and a slot with an invalid id
 @pytest.mark.parametrize("bits,M,A,E,H,I", [(8, 1090, 1, 1, 128, 128), (8, 520, 2, 3, 192, 144),
