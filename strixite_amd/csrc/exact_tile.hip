@@ -67,34 +67,66 @@ __device__ __forceinline__ Rows<RT> tile_rows(const Args &a, int64_t expert, int
     return r;
 }
 
+// LDS between the lanes of one wave
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // acc[t] = the tile's sums over K steps [s0, s1): lane (g, j) holds rows 4 g .. 4 g + 3 against weight row j of tile t.
 // xp: the activation row of MFMA row lane % 16 (any row for an unused one: rows do not mix, and nobody reads its sums).
+// sm: the wave's own LDS for the scales and mins of kWindow groups, [group][row] pairs. (Loaded as 2 bytes a row and step
+// they were half of a step's loads, each a cache line a row for 2 bytes of it: per-slot gate_up of 80 slots, H 2560, I 1024,
+// Q4 g32, FP32 303 us, now 124; 32 slots of Q5 g64, BF16, H 3072, I 1024 105, now 66; FP32 gate_up and down of 40 tokens at H
+// 3072, I 512, Q4 g128 with the rest of their sublayer 320, now 286.)
+constexpr int kWindow = 16;
+template <int RT> constexpr int scale_words() { return kWindow * 16 * RT; }
 template <int FMT, int SP, typename TX, int RT>
 __device__ __forceinline__ void tile_dot(const Args &a, const Rows<RT> &rw, const TX *xp, int s0, int s1,
-                                         float4v (&acc)[RT]) {
+                                         uint32_t *sm, float4v (&acc)[RT]) {
     using F = Fmt<FMT, SP>;
     const int g = threadIdx.x % kWave / 16;
     const uint32_t row_bytes = (uint32_t)(FMT == 8 ? a.K : FMT == 4 ? a.K / 2 : a.K / 2 + a.K / 8);
     const uint32_t groups = (uint32_t)(a.K / a.G), G = (uint32_t)a.G;
     struct Buf {
         Codes c[RT];
-        uint16_t s[RT], m[RT];
         Act8<TX> x[F::NT];
     };
     auto fetch = [&](int s, Buf &b) {
-        const uint32_t k = (uint32_t)s * SP + g * F::CPL, gi = (uint32_t)s * SP / G;
+        const uint32_t k = (uint32_t)s * SP + g * F::CPL;
 #pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            load_codes<FMT, SP>(rw.q[t], rw.j[t] * row_bytes, (uint32_t)a.K, k, b.c[t]);
-            b.s[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.s[t], (rw.j[t] * groups + gi) * 2, 0, 0);
-            b.m[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.m[t], (rw.j[t] * groups + gi) * 2, 0, 0);
-        }
+        for (int t = 0; t < RT; ++t) load_codes<FMT, SP>(rw.q[t], rw.j[t] * row_bytes, (uint32_t)a.K, k, b.c[t]);
 #pragma unroll
         for (int u = 0; u < F::NT; ++u) {
             b.x[u].load(xp + k + 8 * u);
         }
     };
-    auto step = [&](Buf &b, int next) {
+    // the scales and mins of groups [w0, w0 + kWindow) that the wave's steps reach: consecutive lanes read consecutive groups of
+    // a row. Rows past a tile's last one read zeros (their sums are not stored).
+    uint32_t w0 = 0, w1 = 0;
+    const uint32_t g_end = s1 > s0 ? ((uint32_t)s1 * SP - 1) / G + 1 : 0;
+    auto stage = [&](uint32_t first) {
+        w0 = first, w1 = first + kWindow;
+        const uint32_t n = (w1 < g_end ? w1 : g_end) - w0;
+        const int sh = n > 8 ? 4 : n > 4 ? 3 : n > 2 ? 2 : n > 1 ? 1 : 0;
+        wave_sync();  // what the space held has been read
+        for (uint32_t i0 = 0; i0 < 16u << sh; i0 += kWave) {
+            // (lanes past the 16 rows and groups past the last repeat or read what nobody takes)
+            const uint32_t i = i0 + threadIdx.x % kWave, row = (i >> sh) % 16, gi = i & ((1u << sh) - 1);
+            const uint32_t o = (row * groups + w0 + gi) * 2;
+            uint16_t sv[RT], mv[RT];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                sv[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.s[t], o, 0, 0);
+                mv[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw.m[t], o, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) sm[gi * 16 * RT + 16 * t + row] = sv[t] | (uint32_t)mv[t] << 16;
+        }
+        wave_sync();
+    };
+    auto step = [&](Buf &b, int s, int next) {
         const Frag ones{{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}};
         float4v d[RT], dx = {0, 0, 0, 0};  // dx: the activations' own sums
 #pragma unroll
@@ -110,8 +142,9 @@ __device__ __forceinline__ void tile_dot(const Args &a, const Rows<RT> &rw, cons
         float sc[RT], mp[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
-            sc[t] = bf16_to_f32(b.s[t]);
-            mp[t] = fmaf(F::MID, sc[t], bf16_to_f32(b.m[t]));
+            const uint32_t w = sm[((uint32_t)s * SP / G - w0) * 16 * RT + 16 * t + threadIdx.x % 16];
+            sc[t] = __uint_as_float(w << 16);
+            mp[t] = fmaf(F::MID, sc[t], __uint_as_float(w & 0xFFFF0000u));
         }
         if (next < s1) fetch(next, b);
 #pragma unroll
@@ -128,9 +161,11 @@ __device__ __forceinline__ void tile_dot(const Args &a, const Rows<RT> &rw, cons
     if (s0 < s1) fetch(s0, b0);
     if (s0 + 1 < s1) fetch(s0 + 1, b1);
     for (int s = s0; s < s1; s += 2) {
-        step(b0, s + 2);
-        if (s + 1 < s1) step(b1, s + 3);
+        if (((uint32_t)s + 1) * SP / G >= w1) stage((uint32_t)s * SP / G);  // (the first pair: w1 is 0)
+        step(b0, s, s + 2);
+        if (s + 1 < s1) step(b1, s + 1, s + 3);
     }
+    wave_sync();  // the scales are read: the space is the caller's again
 }
 
 __device__ __forceinline__ void store(const Args &a, bool f32, int64_t row, int64_t col, float v) {
@@ -201,15 +236,12 @@ __global__ void __launch_bounds__(kMaxWaves *kWave)
         const int my = __shfl(rec, r0 + (xi < n ? xi : 0), kWave);
         const TX *xp = static_cast<const TX *>(a.x) + (int64_t)((uint32_t)my / (uint32_t)a.A) * a.K;
         float4v acc[RT];
-        tile_dot<FMT, SP, TX, RT>(a, rw, xp, spans * part / ks, spans * (part + 1) / ks, acc);
+        tile_dot<FMT, SP, TX, RT>(a, rw, xp, spans * part / ks, spans * (part + 1) / ks,
+                                  reinterpret_cast<uint32_t *>(red[wave]), acc);  // the scales where its sums will go
 #pragma unroll
         for (int t = 0; t < RT; ++t) red[wave][t][lane] = acc[t];
         if (ks > 1) __syncthreads();
-        else {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
+        else wave_sync();
         // ks > 1: wave t finishes column tile t; else each wave its own. Lane (g, j): rows g, g + 4, ... of column j
         for (int r = 0; r < n; r += 4) {
             const int row = __shfl(rec, r0 + (r + g < n ? r + g : 0), kWave);
@@ -238,6 +270,7 @@ __global__ void __launch_bounds__(kCombineWaves *kWave)
     exact_perslot_combine_kernel(Args a, const float *coef, bool y_f32, int cbs, int ks, int sg) {
     constexpr bool F32 = std::is_same_v<TX, float>;
     __shared__ float red[2][kCombineWaves][kWave];  // lane (g, j), g < 3: MFMA row 5 g of column j
+    __shared__ uint32_t sm[kCombineWaves][scale_words<1>()];
     __shared__ float cf[kWave];
     __shared__ int32_t sid[kWave];
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -258,7 +291,7 @@ __global__ void __launch_bounds__(kCombineWaves *kWave)
             float4v acc[1];
             tile_dot<FMT, SP, TX, 1>(a, tile_rows<FMT, false, 1>(a, id < 0 || id >= a.E ? 0 : id, c0),
                                      static_cast<const TX *>(a.x) + slot * a.K, spans * part / ks, spans * (part + 1) / ks,
-                                     acc);
+                                     sm[wave], acc);
             rb[wave][lane] = g == 0 ? acc[0][0] : g == 1 ? acc[0][1] : acc[0][2];
         }
         __syncthreads();
@@ -290,6 +323,7 @@ __global__ void __launch_bounds__(kOneTokenSlots *kWave)
     one_token_down_kernel(Args a, const float *coef, const uint16_t *resid, uint16_t *out) {
     __shared__ float dots[kOneTokenSlots][16], cf[kOneTokenSlots];
     __shared__ int bad[kOneTokenSlots];
+    __shared__ uint32_t sm[kOneTokenSlots][scale_words<1>()];
     const int lane = threadIdx.x % kWave, slot = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t c0 = (int64_t)blockIdx.x * 16;
     const int32_t id = __builtin_amdgcn_readfirstlane(a.ids[slot]);
@@ -298,7 +332,7 @@ __global__ void __launch_bounds__(kOneTokenSlots *kWave)
     const uint16_t xr = out != nullptr && threadIdx.x < 16 ? resid[c0 + threadIdx.x] : (uint16_t)0;
     float4v acc[1];
     tile_dot<FMT, SP, uint16_t, 1>(a, tile_rows<FMT, false, 1>(a, nan ? 0 : id, c0),
-                                   static_cast<const uint16_t *>(a.x) + (int64_t)slot * a.K, 0, (int)(a.K / SP), acc);
+                                   static_cast<const uint16_t *>(a.x) + (int64_t)slot * a.K, 0, (int)(a.K / SP), sm[slot], acc);
     if (lane < 16) dots[slot][lane] = acc[0][0];  // MFMA row 0
     if (lane == 0) cf[slot] = c, bad[slot] = nan;
     __syncthreads();
