@@ -363,11 +363,20 @@ template <int FMT> struct ChunkCodes {
         }
         if constexpr (FMT == 5) hi = *reinterpret_cast<const uint32_t *>(p + K / 2 + c * 4);
     }
+    // code i about the middle of its range, as a signed field: its top bit turned over
+    __device__ __forceinline__ void centre() {
+        if constexpr (FMT == 5) hi = ~hi;
+        else
+#pragma unroll
+            for (int i = 0; i < W; ++i) w[i] ^= FMT == 8 ? 0x80808080u : 0x88888888u;
+    }
     __device__ __forceinline__ float code(int i) const {
         constexpr int bits = FMT == 8 ? 8 : 4, per = 32 / bits;
-        uint32_t n = (w[i / per] >> (bits * (i % per))) & ((1u << bits) - 1u);
-        if constexpr (FMT == 5) n |= ((hi >> i) & 1u) << 4;
-        return (float)n - Fmt<FMT, 32>::MID;  // exact
+        const uint32_t v = w[i / per];
+        const int at = bits * (i % per);
+        if constexpr (FMT == 5)  // n - 16: the low plane's four bits, and -16 where bit 4 is clear
+            return (float)((int32_t)((v >> at) & 15u) | ((int32_t)(hi << (31 - i)) >> 31) * 16);
+        else return (float)((int32_t)(v << (32 - bits - at)) >> (32 - bits));
     }
 };
 
@@ -378,6 +387,7 @@ template <int FMT, typename TX> __device__ __forceinline__ float lane_dot(const 
     for (int64_t c = threadIdx.x % kWave; c < a.K / 32; c += kWave) {
         ChunkCodes<FMT> cc;
         cc.load(a.q + wrow * row_bytes, a.K, c);
+        cc.centre();
         const int64_t gi = wrow * groups + c * 32 / a.G;
         const float s = bf16_to_f32(a.scale[gi]), m = fmaf(Fmt<FMT, 32>::MID, s, bf16_to_f32(a.minv[gi]));
         float dot[4], xs[4];  // eight codes each: short chains of roundings
