@@ -348,8 +348,8 @@ __global__ void __launch_bounds__(kOneTokenSlots *kWave)
 
 // ---- small calls: a wave an output element ------------------------------------------------------------------------------
 // Lane l takes the row's 32-code chunks l, l + 64, ...: acc = s (x . codes) + m sum(x) a chunk, FP32 with fmaf, the codes
-// about the middle of their range as in the tiles, then a butterfly over the lanes. Every load of a row is in flight at once, so a call whose outputs do not fill the chip costs one
-// round trip, where a tile's waves walk K two steps at a time; a row's codes are converted once an output, so its time grows
+// about the middle of their range as in the tiles, then a butterfly over the lanes. Every load of a row is in flight at once,
+// so a call whose outputs do not fill the chip costs one round trip, where a tile's waves walk K two steps at a time; a row's codes are converted once an output, so its time grows
 // with the outputs from there (lanes_take).
 template <int FMT> struct ChunkCodes {
     static constexpr int W = FMT == 5 ? 4 : FMT;
@@ -492,18 +492,22 @@ template <typename F> void by_format(int fmt, int64_t G, F &&f) {
     }
 }
 
-// Whether a call is small enough for a wave an output element (dots: outputs, FP32 SwiGLU's twice; BF16: Q5 only, the dense
-// BF16 calls' tiles being faster at every size). That form's time grows with dots x (K + 600), the tiles' with the K steps a
-// wave walks (about 0.9 us each, 1.5 where eight waves split K), from about one start each. Measured on MI355X, wave / tiles,
-// us: dense FP32, Q4 g128, N 1024, K 3072 at 4 tokens 9.9 / 12.2, at 8 16 / 13.6; N 3072, K 512 at 2 6.3 / 8.2, at 6 11.8 /
-// 10.2; N 4096, K 4096 at 1 11 / 13, at 2 19 / 14; Q4 g32, N 1024, K 3072 at 12 23 / 27, at 16 28 / 27; Q8 g64, N 640, K 5120
-// at 12 24 / 28, at 16 29 / 28; FP32 gate_up of 4 slots, H 2048, I 512, Q8 8.1 / 12.4, of 16 23 / 22; BF16 Q5 of 8 slots
-// 8.8 / 9.9. By the slots' count and the shape alone, so that a per-slot call and a grouped one take the same form (the same
-// bits). Error against 64 bits (2-norm, FP32): 0.9e-7 to 1.1e-7, the tiles 0.6e-7 to 1.3e-7.
-bool lanes_take(int fmt, Act act, int64_t K, int64_t G, int64_t dots) {
-    if (act != Act::F32 && fmt != 5) return false;
+// Whether a call is small enough for a wave an output element (dots: outputs, SwiGLU's twice; BF16: Q5 only, the dense BF16
+// calls' tiles being faster at every size). That form's time grows with dots x (K + 1400), 0.55 of that with BF16 activations,
+// the tiles' with the K steps a wave walks (about 0.25 us each, 0.55 where eight waves split K), from about one start each; over
+// 900 calls of 1 to 80 slots the line's choice is 1.016 of the better form's time on average. Measured on MI355X, wave / tiles,
+// us: dense FP32, Q4 g128, N 1024, K 3072 at 4 tokens 9.9 / 12.2, at 8 16 / 13.6; N 4096, K 4096 at 1 11 / 13, at 2 19 / 14; Q8
+// g64, N 640, K 5120 at 12 24 / 28; FP32 gate_up of 4 slots, H 2048, I 512, Q8 8.1 / 12.4, of 16 23 / 22; per-slot down of 7
+// slots, K 128, N 3072, Q4 g32 12.7 / 6.1. And Q5 in groups under 128 with BF16 rows, long K, a slot an expert at most: the tiles
+// then read the second plane 2 bytes a row and step for one row in 16 (K 2048, gate_up of 44 slots, I 1024 48 / 71; K 4096,
+// I 768, 16 slots 1.21 of the wave's). By the slots' count and the shape alone, so that a per-slot call and a grouped one take
+// the same form (the same bits). Error against 64 bits (2-norm, FP32): 0.9e-7 to 1.1e-7, the tiles 0.6e-7 to 1.3e-7.
+bool lanes_take(int fmt, Act act, int64_t K, int64_t G, int64_t E, int64_t slots, int64_t dots) {
+    if ((act != Act::F32 && fmt != 5) || dots >= 1 << 24) return false;
+    if (act != Act::F32 && G < 128 && K >= 2048 && slots <= E) return true;
     const int64_t span = fmt == 8 ? std::min<int64_t>(G, 64) : G, spans = K / span, ks = split_of(spans);
-    return dots < (1 << 24) && dots * (K + 600) < 400000 * (4 + (spans + ks - 1) / ks * (ks == 8 ? 15 : 9));
+    const double walk = (double)((spans + ks - 1) / ks) * (ks == 8 ? 55 : 25) * (G == 32 ? 0.8 : 1.0);
+    return (double)dots * (double)(K + 1400) * (act == Act::F32 ? 1.0 : 0.55) < 1e5 * (15 + walk);
 }
 template <typename F> void by_lanes(int fmt, Act act, F &&f) {
     using std::integral_constant;
@@ -519,7 +523,7 @@ template <typename F> void by_lanes(int fmt, Act act, F &&f) {
 }  // namespace
 
 void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &a, hipStream_t stream) {
-    if (lanes_take(fmt, x_act, a.K, a.G, a.S * a.ncol * (swiglu && x_act == Act::F32 ? 2 : 1))) {
+    if (lanes_take(fmt, x_act, a.K, a.G, a.E, a.S, a.S * a.ncol * (swiglu ? 2 : 1))) {
         const unsigned blocks = (unsigned)((a.S * a.ncol + kLaneBlock / kWave - 1) / (kLaneBlock / kWave));
         return by_lanes(fmt, x_act, [&](auto fc, auto tx) {
             auto k = swiglu ? lane_rows_kernel<decltype(fc)::value, true, decltype(tx)>
@@ -559,7 +563,7 @@ void project(int fmt, Mode mode, bool swiglu, Act x_act, Act y_act, const Args &
 }
 
 void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStream_t stream) {
-    if (lanes_take(fmt, act, a.K, a.G, a.S * a.A * a.ncol)) {  // as the grouped down of the same slots
+    if (lanes_take(fmt, act, a.K, a.G, a.E, a.S * a.A, a.S * a.A * a.ncol)) {  // as the grouped down of the same slots
         const unsigned blocks = (unsigned)((a.S * a.ncol + kLaneBlock / kWave - 1) / (kLaneBlock / kWave));
         return by_lanes(fmt, act, [&](auto fc, auto tx) {
             lane_perslot_combine_kernel<decltype(fc)::value, decltype(tx)>
