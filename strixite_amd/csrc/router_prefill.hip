@@ -352,6 +352,11 @@ bool prefill_shape_fits(const void *x, const uint16_t *w, int64_t H, int64_t E, 
 bool moe_router_prefill_approx(const void *x, const uint16_t *w, int64_t M, int64_t H, int64_t E, int64_t k,
                                bool shared, float *logits, float *norms, hipStream_t stream) {
     if (!prefill_shape_fits(x, w, H, E, k)) return false;
+    // H 2560 with few logits: the canonical projection and top-k are two launches for these four. Measured on MI355X, layers of I
+    // 128, this way / theirs, us: 64 experts at 400 tokens 73 / 71, 4096 148 / 151; 128 at 700 84 / 82, 1024 107 / 115; 256 at 400
+    // 107 / 102, 700 123 / 126; 512 at 256 152 / 156. (Up to 1024 slots theirs packs in the same one block, much the longer: 64
+    // experts, top-4 at 256 tokens 63 / 88.)
+    if (H == 2560 && M * E < 131072 && M * k > 1024) return false;
     const int64_t ld = E + (shared ? 1 : 0);
     // pass 1: the library GEMM into the logits buffer's second part ([M][E], ld E; parts 1..3 of the [4][M][ld]
     // buffer are scratch) and the row norms. A shape the library declines: false, and the caller routes through the

@@ -345,3 +345,37 @@ def test_small_q5_bf16_experts(M, A):
     z = np.stack([X[s // A] @ g64[e * 2 * I:(e + 1) * 2 * I].T for s, e in enumerate(ids.ravel())])
     assert _rel64(h, z[:, :I] / (1 + np.exp(-z[:, :I])) * z[:, I:]) < 2.0 ** -8  # one BF16 rounding
     assert torch.equal(moe.experts_gather(x, gu, E, tid, moe.zero_err(), swiglu=True), h)
+
+
+# the served widths (H 2560, I 640) with a separate shared expert - its split-K parts ride in the gate_up's and the down's
+# launches - and the prefill router there, on either side of the logits from which it selects from the approximate pass
+@pytest.mark.parametrize("M,E,k,shared", [(1, 24, 6, True), (11, 24, 6, True), (16, 40, 10, True), (300, 512, 10, "stacked"),
+                                          (257, 512, 4, False), (300, 128, 10, True)])
+def test_layer_at_the_served_widths(M, E, k, shared):
+    say("served widths", M, E, k, shared)
+    layer = moe.MoeLayer.synth(2560, E, k, 640, seed=9, shared=shared)
+    x = moe.synth_bf16_normal(9, "x", 0, (M, 2560), 1.0)
+    out = layer.forward(x)
+    rows = np.unique(np.concatenate([np.arange(min(M, 8)), np.arange(max(0, M - 8), M)]))
+    o = orc.moe_layer(oracle_weights(layer), to_np(x)[rows])
+    assert np.array_equal(to_np(out["ids"])[rows], o["ids"])
+    assert rel_err(to_np(out["y"])[rows], o["y"]) < 1e-2  # the layer tests' tolerance
+
+
+# nonzero-mean activations, and codes of a narrow part of their range. The tiles add codes 16 + n times x and take the offset out
+# after: a group's running sum reaches 31 sum |x|, and is rounded at 2^-24 of that some eight times (four products of 32
+# codes, the offset, the scale, the min, the accumulator), whatever the result's own size
+@pytest.mark.parametrize("M,K,low", [(1, 3072, False), (64, 3072, False), (64, 3072, True), (1, 2048, True)])
+def test_fp32_dense_off_centre(M, K, low):
+    say("off centre", M, K, low)
+    N, G = 512, 128
+    rng = np.random.default_rng(M + K)
+    codes = rng.integers(0, 3 if low else 16, size=(N, K)).astype(np.uint8)
+    s = orc.f32_to_bf16(rng.uniform(0.01, 0.03, N * (K // G)).astype(np.float32))
+    m = np.zeros_like(s) if low else orc.f32_to_bf16(orc.bf16_to_f32(s) * np.float32(-7.5))
+    w = moe.QWeight.from_host(4, (codes[:, 0::2] | codes[:, 1::2] << 4).reshape(-1), s, m, N, K, G)
+    x = (rng.standard_normal((M, K)) * 0.5 + 1).astype(np.float32)
+    w64 = _w64(w)
+    got = moe.linear_q4(torch.from_numpy(x).to(DEV), w, out_dtype=torch.float32).double().cpu().numpy()
+    bound = 8 * 2.0 ** -24 * 31 * 0.03 * np.abs(x).sum(axis=1, keepdims=True)
+    assert (np.abs(got - x.astype(np.float64) @ w64.T) < bound).all()
