@@ -151,5 +151,17 @@ __device__ __forceinline__ float4v mfma_bf16(const Frag &a, const Frag &b, float
 
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }  // strixite kernels/swiglu.hip:22
 
+// the current device's CUs, asked for once (256 if the runtime does not say)
+inline int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n = 256;
+        return n > 0 ? n : 256;
+    }();
+    return cus;
+}
+
 }  // namespace dev
 }  // namespace strix

@@ -1096,16 +1096,6 @@ void check_view(const char *fn, const QV &w, int64_t E) {
     STRIX_CHECK(reinterpret_cast<uintptr_t>(w.q) % 16 == 0, fn, ": code array must be 16-byte aligned");
 }
 
-int device_cus() {
-    static int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            n = 256;
-        return n > 0 ? n : 256;
-    }();
-    return cus;
-}
-
 // Persistent grid: as many blocks as fit on the device at once (capped by the items), each looping over items.
 // SwiGLU: K split over ks = 1..4 waves (the block), preferring an even split into whole ring trips of D steps and
 // then the most waves

@@ -51,16 +51,6 @@ namespace {
 using namespace strix::dev;
 constexpr int kWave = 64, kStreams = 4, kChunk = 32;
 constexpr int64_t kMaxR = 1024, kMaxTokens = 65535, kMaxD = 1 << 20;
-int device_cus() {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            n = 256;
-        return n > 0 ? n : 256;
-    }();
-    return cus;
-}
-
 __device__ __forceinline__ float ld_act(const float *p, int64_t i) { return p[i]; }
 __device__ __forceinline__ float ld_act(const uint16_t *p, int64_t i) { return bf16_to_f32(p[i]); }
 __device__ __forceinline__ void st_act(float *p, int64_t i, float v) { p[i] = v; }
@@ -439,9 +429,10 @@ __global__ void __launch_bounds__(dn::kThreads * KH)
 // A block takes TT 16-token tiles against RT tiles of 16 weight rows (BF16 streams), and its NW waves split K: NW / 4 to
 // a stream. A wave also squares its tokens with the matrix cores (x against itself: the diagonal of one more MFMA), so
 // the streams' inverse RMS costs no other pass. The waves' parts meet in LDS once, in wave order: a = sum_s inv_s (P of
-// the stream's waves). The codes enter about the middle of their range, so no sum is larger than the result; single-tile
-// blocks, where lane dots would be the alternative, also keep their running sums in two levels: the error against 64
-// bits stays at the lane dots' (1.3e-7).
+// the stream's waves). The codes enter about the middle of their range, so with weights of mean zero no sum is much larger
+// than the result (where a group's codes lie at one end, s D and the min term cancel: 1.9e-7 against 64 bits with codes 0 .. 2
+// and no min, 1.0e-7 with centred ones); single-tile blocks, where lane dots would be the alternative, also keep their running
+// sums in two levels: the error stays at the lane dots' (1.3e-7).
 // What bounds it: the address path (16 rows a load) and the latency of the wave's K walk. The wave's scales and mins go
 // through LDS: as 2-byte loads a step and row they took a third of the time (16 x 32 blocks: 38 -> 24 us).
 // codes 8 u .. 8 u + 7 of the lane about the middle of their range, exact in bf16, in the paired order: 16 (n - 8) (Q4: the
