@@ -560,13 +560,13 @@ __global__ void __launch_bounds__((W + 1) * kWave) decode_gate_up_lds_kernel(Dec
 // registers. Waves are dealt to tiles, not to a flat unit range: every tile gets floor or ceil(waves / tiles) waves,
 // each a contiguous range of the tile's N / 16 row blocks, so a wave loads its tile's h rows once, before its loop,
 // and streams one contiguous region of the expert's rows. A unit's codes reach LDS by KS direct loads of 1 KB
-// (contiguous), with its rows' scale and min dwords, into the wave's own ring of kDnStages positions; no barrier, no K split. The FP32 partials are stored as each unit ends: the waits count loads only (a
-// store may complete before older loads, so counting it could release a wait early; not counting it only makes a wait
-// stricter).
+// (contiguous), with its rows' scale and min dwords, into the wave's own ring of kDnStages positions; no barrier, no K
+// split. The FP32 partials are stored as each unit ends: the waits count loads only (a store may complete before older
+// loads, so counting it could release a wait early; not counting it only makes a wait stricter).
 // LDS layout of a position (uint4): the rows' 4 KS 16-byte chunks in row order, chunk c of row r at place c ^ swz(r) of
 // its row; then 8 KS dwords of scales (row r's group s: bf16 KS r + s) and as many of mins. swz spreads the 16 rows'
-// reads of one chunk over the 64 LDS banks: rows 16 KS dwords apart share their banks every 4 (KS odd), 8 (KS = 2 mod
-// 4) or 16 / 16 (KS = 4) rows apart, and the aliasing rows take different places of a 4-, 8- or 16-chunk block.
+// reads of one chunk over the 64 LDS banks: rows 16 KS dwords apart share their banks every 4 (KS odd), 2 (KS = 2 mod
+// 4) or 1 (KS = 4, 8) rows apart, and the aliasing rows take different places of a 4-, 8- or 16-chunk block.
 namespace gdn {
 constexpr int kDnStages = 3;                                    // per-wave ring
 template <int KS> constexpr int pos_u4() { return 4 * KS * 17; }  // codes + 16 KS dwords of scales and mins
@@ -575,18 +575,18 @@ template <int KS> constexpr int pos_u4() { return 4 * KS * 17; }  // codes + 16 
 // a block that waits for another to end makes a second round: with five blocks of two, the LDS's worth, the down of 11
 // tokens at H 2560, I 640 took 26.6 us, so 21.1; held to three waves a SIMD it spills, whose scratch loads the ring's
 // waits then count: 66.)
-template <int KS> constexpr int waves() { return 4; }
+constexpr int kDnWaves = 4;
 template <int KS> constexpr int blocks_per_cu() {
-    return std::min(KS <= 4 ? 3 : 2, 163840 / (waves<KS>() * kDnStages * pos_u4<KS>() * 16));
+    return std::min(KS <= 4 ? 3 : 2, 163840 / (kDnWaves * kDnStages * pos_u4<KS>() * 16));
 }
 template <int KS> __device__ __forceinline__ int swz(int r) {
     return KS % 2 ? (r >> 2) & 3 : KS % 4 ? (r >> 1) & 7 : r;
 }
 }  // namespace gdn
 
-template <int SH, int KS, int WB = gdn::waves<KS>(), int NS = gdn::kDnStages>
-__global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs a, SharedJob sh) {
-    static_assert(NS >= 3 && NS <= 8, "ring positions: separate LDS arrays, at most 8");
+template <int SH, int KS>
+__global__ void __launch_bounds__(gdn::kDnWaves * kWave) decode_down_lds_kernel(DecodeArgs a, SharedJob sh) {
+    constexpr int WB = gdn::kDnWaves, NS = gdn::kDnStages;
     static_assert(KS >= 2 && KS <= 8, "K = 128 KS");
     int bid = (int)blockIdx.x, nblk = (int)gridDim.x;
     if constexpr (SH == 2) {
@@ -597,23 +597,17 @@ __global__ void __launch_bounds__(WB * kWave) decode_down_lds_kernel(DecodeArgs 
         }
         bid -= sh.blocks, nblk -= sh.blocks;
     }
-    // one array a ring position (the compiler tracks the direct-to-LDS loads' aliasing per array); unused ones 1 x 1
+    // one array a ring position (the compiler tracks the direct-to-LDS loads' aliasing per array)
+    static_assert(NS == 3, "an array each");
     constexpr int P = gdn::pos_u4<KS>();
-    __shared__ __attribute__((aligned(16))) uint4 rp0[WB][P], rp1[WB][P], rp2[WB][P], rp3[NS > 3 ? WB : 1][NS > 3 ? P : 1],
-        rp4[NS > 4 ? WB : 1][NS > 4 ? P : 1], rp5[NS > 5 ? WB : 1][NS > 5 ? P : 1], rp6[NS > 6 ? WB : 1][NS > 6 ? P : 1],
-        rp7[NS > 7 ? WB : 1][NS > 7 ? P : 1];
+    __shared__ __attribute__((aligned(16))) uint4 rp0[WB][P], rp1[WB][P], rp2[WB][P];
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int g = lane / 16, j = lane % 16;
     auto ring = [&](auto P) -> uint4 * {
         constexpr int p = decltype(P)::value;
         if constexpr (p == 0) return rp0[wave];
         else if constexpr (p == 1) return rp1[wave];
-        else if constexpr (p == 2) return rp2[wave];
-        else if constexpr (p == 3) return rp3[wave];
-        else if constexpr (p == 4) return rp4[wave];
-        else if constexpr (p == 5) return rp5[wave];
-        else if constexpr (p == 6) return rp6[wave];
-        else return rp7[wave];
+        else return rp2[wave];
     };
     const int64_t n_tiles = a.ws[0] < a.tiles_bound ? a.ws[0] : a.tiles_bound;
     if (n_tiles <= 0) return;
@@ -746,17 +740,35 @@ inline bool gate_up_lds_fits(const GemmArgs &ga);
 inline bool scales_dword_aligned(const GemmArgs &ga) {
     return reinterpret_cast<uintptr_t>(ga.scale) % 4 == 0 && reinterpret_cast<uintptr_t>(ga.minv) % 4 == 0;
 }
-// the LDS-ring down kernel's shapes: Q4 g128, K = 512 or 640 (the benchmark's and the served model's I); it deals its
-// waves to tiles, so every tile needs a wave. Measured on MI355X at H 2560, I 640, 513 experts, 11 slots a token, against
-// the register-fed stream kernels (this and the gate_up at W = 10 together, the rest of the layer as it was): a layer of 11
-// tokens 116 -> 86 us, of 1 token 40.0 -> 33.5, of 333 tokens 526 -> 366
+// f(KS) for a row of KS groups, if the LDS-ring down kernel takes it
+template <typename F> bool by_down_groups(int64_t K, F &&f) {
+    using std::integral_constant;
+    if (K % dec::kSpan != 0) return false;
+    switch (K / dec::kSpan) {
+        case 2: f(integral_constant<int, 2>{}); return true;
+        case 3: f(integral_constant<int, 3>{}); return true;
+        case 4: f(integral_constant<int, 4>{}); return true;
+        case 5: f(integral_constant<int, 5>{}); return true;
+        case 6: f(integral_constant<int, 6>{}); return true;
+        case 7: f(integral_constant<int, 7>{}); return true;
+        case 8: f(integral_constant<int, 8>{}); return true;
+        default: return false;
+    }
+}
+// The LDS-ring down kernel's shapes: Q4 g128, rows of 2 to 8 groups (above, a tile's h rows leave no registers); it deals its
+// waves to tiles, so every tile needs a wave. At 8 groups one block of four waves fills a CU's LDS: it is the better one from a
+// few tiles up to some six waves a tile. Measured on MI355X, layers, us, the register-fed stream kernels / this and the
+// gate_up at K = 256 W: H 2560, I 640, 513 experts, 11 slots a token, 11 tokens 116 / 86, 1 token 40.0 / 33.5, 333 tokens 526 /
+// 366; H 2816, I 768, 64 experts top-8 16 tokens 93 / 64, 120 167 / 112; H 2560, I 896, 129 experts 48 tokens 128 / 113; H 2304,
+// I 384 1 token 24 / 19. This alone: H 2048, I 256 16 tokens 48 / 40; H 3072, I 1024, 64 experts top-6 1 token 33.6 / 35.0, 48
+// 125 / 97, 120 157 / 128, 400 167 / 173.
 inline bool down_lds_fits(const GemmArgs &ga) {
     const int64_t tiles = std::min(ga.S, ga.S / 16 + ga.E + 2);
-    auto waves = [](auto ks) { return gdn::blocks_per_cu<decltype(ks)::value>() * gdn::waves<decltype(ks)::value>(); };
     if (ga.G != dec::kSpan || ga.N % 16 != 0 || !scales_dword_aligned(ga)) return false;
-    if (ga.K == 4 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 4>{}) * device_cus();
-    if (ga.K == 5 * dec::kSpan) return tiles <= (int64_t)waves(std::integral_constant<int, 5>{}) * device_cus();
-    return false;
+    int64_t waves = 0;
+    by_down_groups(ga.K, [&](auto ks) { waves = gdn::blocks_per_cu<decltype(ks)::value>() * gdn::kDnWaves; });
+    if (ga.K == 8 * dec::kSpan && (tiles <= 8 || 6 * tiles > waves * device_cus())) return false;
+    return tiles <= waves * device_cus();
 }
 
 // Q4 g128 experts, at most 16 tokens; gate_up: the LDS-ring kernel's shapes or K = 128 * kDecGuWaves * SPW, SPW in 2..4;
@@ -796,12 +808,26 @@ void launch_decode_gate_up_lds(const DecodeArgs &d, SharedJob s, hipStream_t str
     else decode_gate_up_lds_kernel<W, 0><<<blocks, (W + 1) * kWave, 0, stream>>>(d, s);
 }
 
-// the LDS-ring gate_up's shapes: K = 256 W (W 8, 10 or 12: H 2048, 2560, 3072), Q4 g128; a block's unit range (at most ceil(units / CUs)
-// units) must touch at most kGuMaxBlockTiles tiles, and the tile count fit the block's table
+// f(W) for K = 256 W, if the LDS-ring gate_up takes it: 8 to 12 waves (fewer leave a CU's one block too few loads in flight;
+// more do not fit the LDS)
+template <typename F> bool by_gate_up_waves(int64_t K, F &&f) {
+    using std::integral_constant;
+    if (K % 256 != 0) return false;
+    switch (K / 256) {
+        case 8: f(integral_constant<int, 8>{}); return true;
+        case 9: f(integral_constant<int, 9>{}); return true;
+        case 10: f(integral_constant<int, 10>{}); return true;
+        case 11: f(integral_constant<int, 11>{}); return true;
+        case 12: f(integral_constant<int, 12>{}); return true;
+        default: return false;
+    }
+}
+// the LDS-ring gate_up's shapes: Q4 g128, K = 256 W; a block's unit range (at most ceil(units / CUs) units) must touch at most
+// kGuMaxBlockTiles tiles, and the tile count fit the block's table
 inline bool gate_up_lds_fits(const GemmArgs &ga) {
     const int64_t tiles_bound = std::min(ga.S, ga.S / 16 + ga.E + 2);
     const int64_t upt = ga.N / 32, most_units = (tiles_bound * upt + device_cus() - 1) / device_cus();
-    return ga.G == dec::kSpan && scales_dword_aligned(ga) && ga.K % 256 == 0 && (ga.K / 256 == 8 || ga.K / 256 == 10 || ga.K / 256 == 12) && (ga.N / 2) % 16 == 0 &&
+    return ga.G == dec::kSpan && scales_dword_aligned(ga) && by_gate_up_waves(ga.K, [](auto) {}) && (ga.N / 2) % 16 == 0 &&
            (most_units + upt - 1) / upt + 1 <= gul::kGuMaxBlockTiles && tiles_bound <= kDecMaxTilesL;
 }
 
@@ -812,11 +838,7 @@ inline bool gate_up_stream_fits(const GemmArgs &ga, int64_t M) {
 }
 inline void launch_gate_up_stream(const GemmArgs &ga, int64_t M, hipStream_t stream) {
     const DecodeArgs d = decode_args(ga, M, true);
-    switch (ga.K / 256) {
-        case 8: return launch_decode_gate_up_lds<8>(d, SharedJob{}, stream, true);
-        case 10: return launch_decode_gate_up_lds<10>(d, SharedJob{}, stream, true);
-        default: return launch_decode_gate_up_lds<12>(d, SharedJob{}, stream, true);
-    }
+    by_gate_up_waves(ga.K, [&](auto w) { launch_decode_gate_up_lds<decltype(w)::value>(d, SharedJob{}, stream, true); });
 }
 
 template <int SPW>
@@ -840,12 +862,8 @@ inline void launch_decode_gate_up(const GemmArgs &ga, int64_t M, const SharedJob
     if (gate_up_lds_fits(ga)) {
         SharedJob t = s;
         t.units = sh ? s.units : 0;
-        switch (ga.K / 256) {
-            case 8: return launch_decode_gate_up_lds<8>(d, t, stream);
-            case 10: return launch_decode_gate_up_lds<10>(d, t, stream);
-            case 12: return launch_decode_gate_up_lds<12>(d, t, stream);
-            default: break;
-        }
+        by_gate_up_waves(ga.K, [&](auto w) { launch_decode_gate_up_lds<decltype(w)::value>(d, t, stream); });
+        return;
     }
     switch (ga.K / dec::kSpan / kDecGuWaves) {
         case 2: launch_decode_gate_up_spw<2>(d, s, stream); break;
@@ -869,12 +887,11 @@ inline void launch_decode_down(const GemmArgs &ga, int64_t M, const SharedJob *s
     // 2 x 8 109.3, 1 x 8 110.4 - more waves beat more units in flight (the LDS reads and the dequantisation
     // of a unit are hidden by other waves, not by a wave's own ring)
     auto go = [&](auto ksc) {
-        constexpr int KS = decltype(ksc)::value, WB = gdn::waves<KS>();
+        constexpr int KS = decltype(ksc)::value, WB = gdn::kDnWaves;
         s.blocks = sh ? (int)((s.units + WB - 1) / WB) : 0;
         const unsigned nb = (unsigned)(gdn::blocks_per_cu<KS>() * device_cus() + s.blocks);
         if (sh) decode_down_lds_kernel<2, KS><<<nb, WB * kWave, 0, stream>>>(d, s);
         else decode_down_lds_kernel<0, KS><<<nb, WB * kWave, 0, stream>>>(d, s);
     };
-    if (ga.K == 4 * dec::kSpan) go(std::integral_constant<int, 4>{});
-    else go(std::integral_constant<int, 5>{});
+    by_down_groups(ga.K, go);
 }

@@ -26,8 +26,11 @@ def _weight(bits, N, K, G, seed):
 
 # the served model's K (gate_up 2560: ten streaming waves; down 640: five groups a row, the swizzle of odd group counts)
 # at one token, at the most tokens of the decode form, and gathered above it; one slot has an invalid id
+# (and each other count of waves and of groups a row that the two kernels take)
 @pytest.mark.parametrize("M,A,E,H,I", [(1, 3, 8, 2560, 640), (16, 4, 24, 2560, 640), (17, 4, 9, 2560, 640),
-                                       (90, 3, 5, 2560, 640)])
+                                       (90, 3, 5, 2560, 640), (5, 3, 9, 2304, 256), (70, 3, 6, 2304, 384),
+                                       (7, 4, 9, 2816, 768), (60, 2, 7, 2816, 896), (16, 3, 8, 2048, 1024),
+                                       (75, 4, 6, 3072, 1024)])
 def test_streamed_experts_at_the_served_widths(M, A, E, H, I):
     say("streamed experts", M, A, E, H, I)
     gu, dn = _weight(4, E * 2 * I, H, 128, 31), _weight(4, E * H, I, 128, 32)
