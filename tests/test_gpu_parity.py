@@ -923,8 +923,7 @@ def test_grouped_small_groups(bits, G, M, A, E, H, I):
 
 @pytest.mark.parametrize("bits,G,M", [(4, 64, 7), (4, 32, 7), (8, 32, 7), (4, 64, 200), (8, 64, 200), (8, 32, 200)])
 def test_dense_small_groups(bits, G, M):
-    """Decode sizes on the stream kernels, prefill sizes (M >= 128) on the matrix-core GEMM (G 64 / 128) or the stream
-    kernels (G 32)."""
+    """Few outputs, so the exact 16-row tiles at every size (test_gpu_shapes.py: the stream kernel and the GEMM)."""
     say("dense small groups", bits, G, M)
     N, K = 320, 1024
     w = moe.QWeight.synth(bits, 18, "gu_q", "gu_s", 1, N, K, G)
