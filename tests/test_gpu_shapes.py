@@ -352,13 +352,16 @@ def test_small_q5_bf16_experts(M, A):
 
 
 # the served widths (H 2560, I 640) with a separate shared expert - its split-K parts ride in the gate_up's and the down's
-# launches - and the prefill router there, on either side of the logits from which it selects from the approximate pass
-@pytest.mark.parametrize("M,E,k,shared", [(1, 24, 6, True), (11, 24, 6, True), (16, 40, 10, True), (300, 512, 10, "stacked"),
-                                          (257, 512, 4, False), (300, 128, 10, True)])
-def test_layer_at_the_served_widths(M, E, k, shared):
-    say("served widths", M, E, k, shared)
-    layer = moe.MoeLayer.synth(2560, E, k, 640, seed=9, shared=shared)
-    x = moe.synth_bf16_normal(9, "x", 0, (M, 2560), 1.0)
+# launches - and the prefill router there, on either side of the logits from which it selects from the approximate pass; and
+# the shared expert beside other counts of waves and groups
+@pytest.mark.parametrize("H,I,M,E,k,shared", [
+    (2560, 640, 1, 24, 6, True), (2560, 640, 11, 24, 6, True), (2560, 640, 16, 40, 10, True),
+    (2560, 640, 300, 512, 10, "stacked"), (2560, 640, 257, 512, 4, False), (2560, 640, 300, 128, 10, True),
+    (2304, 384, 7, 24, 6, True), (2816, 256, 16, 24, 4, True), (2304, 1024, 3, 24, 6, True), (2816, 896, 1, 24, 6, True)])
+def test_layer_at_the_streamed_widths(H, I, M, E, k, shared):
+    say("streamed widths", H, I, M, E, k, shared)
+    layer = moe.MoeLayer.synth(H, E, k, I, seed=9, shared=shared)
+    x = moe.synth_bf16_normal(9, "x", 0, (M, H), 1.0)
     out = layer.forward(x)
     rows = np.unique(np.concatenate([np.arange(min(M, 8)), np.arange(max(0, M - 8), M)]))
     o = orc.moe_layer(oracle_weights(layer), to_np(x)[rows])
