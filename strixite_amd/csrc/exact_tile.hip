@@ -569,7 +569,11 @@ void perslot_combine(int fmt, Act act, const Args &a, const float *coef, hipStre
                 " slots, ", a.ncol, " columns");
     by_format(fmt, a.G, [&](auto fc, auto sc) {
         constexpr int FMT = decltype(fc)::value, SP = decltype(sc)::value;
-        const int ks = split_of(a.K / SP), sg = (int)std::min<int64_t>(a.A, kCombineWaves / ks);
+        // slots at a time: all that a block's waves hold while the blocks leave CUs idle, then four waves' worth (their rounds
+        // overlap other blocks'; us, all / four waves: 10 slots, H 3072, I 512, Q4 g128 at 1 token 10.9 / 13.3, 3 24 / 21, 10 56
+        // / 41; 4 slots, H 4096, I 512, Q4 g64 at 2 12.4 / 11.7, 6 28 / 22, 40 170 / 110)
+        const int ks = split_of(a.K / SP), waves = a.S * cbs > 2 * device_cus() ? 4 : kCombineWaves;
+        const int sg = (int)std::max<int64_t>(1, std::min<int64_t>(a.A, waves / ks));
         auto go = [&](auto tx) {
             exact_perslot_combine_kernel<FMT, SP, decltype(tx)>
                 <<<(unsigned)(a.S * cbs), ks * sg * kWave, 0, stream>>>(a, coef, act == Act::F32, (int)cbs, ks, sg);

@@ -292,7 +292,9 @@ def test_mix_up_kernels(bits, G, act, T, d, r):
 
 # the per-slot combine: K whole, split over 4 and over 8 waves, slots within one round of waves and past it, a ragged
 # column end; the grouped combine's bits, float64, the first invalid id of a token reported
-@pytest.mark.parametrize("G,K,A,N", [(128, 512, 17, 48), (128, 512, 5, 16), (128, 1024, 9, 32), (32, 1024, 3, 80)])
+# (and four waves a block, past two blocks a CU)
+@pytest.mark.parametrize("G,K,A,N", [(128, 512, 17, 48), (128, 512, 5, 16), (128, 1024, 9, 32), (32, 1024, 3, 80),
+                                     (128, 512, 6, 2816), (32, 1024, 3, 2816)])
 def test_perslot_combine_rounds(G, K, A, N):
     say("per-slot combine", G, K, A, N)
     M, E = 3, 24
