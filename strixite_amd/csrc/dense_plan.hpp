@@ -43,10 +43,9 @@ inline Dense plan(int bits, int64_t G, int64_t M, int64_t N, int64_t K, bool out
     const bool pow2 = (K & (K - 1)) == 0, s = pow2 && K <= kStreamK;
     if (G < 64) {
         // us, stream / tiles: Q4 K 512, N 3072 at 100 tokens 12.0 / 14.4, at 500 23 / 40, at 2000 72 / 141, N 32768 at 1 10.5 /
-        // 15.3; K 1024, N 4096 at 128 29 / 32, at 2000 394 / 457; K 2048, N 131072 at 1
-        // 179 / 194, Q8, N 1088 at 823 115 / 105; K 3072, N 4096 at 700
-        // 440 / 405, K 1408 (Q8), N 10464 at 560 412 / 275; few outputs: K 512, N 512 at 500 12.0 / 11.4, K 1024, N 1024 at
-        // 300 29 / 25
+        // 15.3; K 1024, N 4096 at 128 29 / 32, at 2000 394 / 457; K 2048, N 131072 at 1 179 / 194, Q8, N 1088 at 823 115 / 105; K
+        // 3072, N 4096 at 700 440 / 405; K 1408 (Q8), N 10464 at 560 412 / 275; few outputs: K 512, N 512 at 500 12.0 / 11.4, K
+        // 1024, N 1024 at 300 29 / 25
         return s && K <= (bits == 8 ? 1024 : kStreamK) && padded > (K <= 512 ? 280000 : 400000) ? Dense::Stream : Dense::Tiles;
     }
     const Cost &c = kCosts[bits == 8][G >= 128];

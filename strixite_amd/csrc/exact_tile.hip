@@ -13,9 +13,9 @@
 // product D is rescaled on the FP32 accumulator: w . x = s D' + m' sum(x), with D' and m' for the codes about the middle of
 // their range (D' = D - EXTRA sum(x), m' = m + MID s). The error is relative to what the sums pass through, not to the
 // result: D's running sum carries the offset (up to 31 or 63 times sum |x| a group), and D' and m' sum(x) cancel where a
-// group's codes lie at one end of their range. Measured against 64 bits (2-norm, FP32, Q4 g128, K 3072): 1.3e-7 with activations and weights
-// of mean zero, 1.2e-6 with activations of mean and deviation 1, 2.6e-7 with codes 0 .. 2 and no min. sum(x) comes from one
-// more MFMA, against ones.
+// group's codes lie at one end of their range. Measured against 64 bits (2-norm, FP32, Q4 g128, K 3072): 1.3e-7
+// with activations and weights of mean zero, 1.2e-6 with activations of mean and deviation 1, 2.6e-7 with codes 0 .. 2 and no
+// min. sum(x) comes from one more MFMA, against ones.
 //
 // What bounds it: grouped, the weight stream beside ~80 vector instructions a wave per 32 k x 64 weight rows (the split
 // and the codes' conversion); dense, latency, so K is split over the block's waves (8 from 32 steps, 4 from 8) and their
@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(kMaxWaves *kWave)
 // Block (token, 16 output columns): ks waves split K of a slot, sg slots at a time (kCombineWaves waves at most), each as
 // exact_tile_kernel's one-row tile (MFMA rows 0, 5 and 10 of an FP32 slot, row 0 of a BF16 one), the slots' dots summed with
 // the coefficients in slot order. What bounds it: latency, a round of K's walk for every sg slots. Measured on MI355X, H
-// 3072, I 512, 10 slots a token, Q4 g128, FP32: 12 us at 1 token, 26 at 4 (a slot a round 44 and 47, a wave an output 20 and
+// 3072, I 512, 10 slots a token, Q4 g128, FP32: 11 us at 1 token, 21 at 4 (a slot a round 44 and 47, a wave an output 20 and
 // 67).
 constexpr int kCombineWaves = 16;
 template <int FMT, int SP, typename TX>
@@ -353,8 +353,8 @@ __global__ void __launch_bounds__(kOneTokenSlots *kWave)
 // ---- small calls: a wave an output element ------------------------------------------------------------------------------
 // Lane l takes the row's 32-code chunks l, l + 64, ...: acc = s (x . codes) + m sum(x) a chunk, FP32 with fmaf, the codes
 // about the middle of their range as in the tiles, then a butterfly over the lanes. Every load of a row is in flight at once,
-// so a call whose outputs do not fill the chip costs one round trip, where a tile's waves walk K two steps at a time; a row's codes are converted once an output, so its time grows
-// with the outputs from there (lanes_take).
+// so a call whose outputs do not fill the chip costs one round trip, where a tile's waves walk K two steps at a time; a row's
+// codes are converted once an output, so its time grows with the outputs from there (lanes_take).
 template <int FMT> struct ChunkCodes {
     static constexpr int W = FMT == 5 ? 4 : FMT;
     uint32_t w[W], hi;
